@@ -694,21 +694,43 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
     return z ^ (z >> 31);
 }
 
-// Batch of M rows drawn uniformly (with replacement) from the data set:
-// X[M][128], XT[128][M], T[M][4].
-// Block b draws rows [64 b, 64 b + 64) (M % 64 == 0); XT is written through an
-// LDS transpose, 64 contiguous rows (128 bytes) per feature.
+// The transposing tile of a 64-row block: feature-major in LDS, so that the
+// block's rows leave as 128 rows (one per feature) of 128 contiguous bytes.
 constexpr int BATCH_ROWS = 64, BATCH_THREADS = 256;
-// A training batch: row r takes sample mix64(key + r) mod size.  16 threads
-// per row move its 256 bytes of features as 16-byte pieces (and one the
-// 16-byte target); the block's 64 rows pass through LDS so that XT leaves as
-// 128 rows of 128 contiguous bytes.
+typedef bf16_t BatchTile[KIN][BATCH_ROWS + 8];
+static_assert(KIN == 16 * 8 && BATCH_ROWS * KIN == BATCH_THREADS * 32, "16 pieces of 8 features per row");
+
+// Row q's 8 features of piece `piece` into the tile.  Its 8-row chunk sits at
+// chunk (q / 8) ^ (piece % 8) of the feature's LDS row, so that the 16 pieces
+// a write spans fall on 8 bank groups instead of 2.
+__device__ __forceinline__ void tile_put(BatchTile& tile, int q, int piece, const uint4& v) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    const int col = (((q >> 3) ^ (piece & 7)) << 3) | (q & 7);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        tile[8 * piece + 2 * j][col] = (bf16_t)(w[j] & 0xffffu);
+        tile[8 * piece + 2 * j + 1][col] = (bf16_t)(w[j] >> 16);
+    }
+}
+
+// Feature f of the block's rows: 64 contiguous elements of XT row f.
+__device__ __forceinline__ void tile_out(const BatchTile& tile, int rb, int M, bf16_t* __restrict__ XT) {
+#pragma unroll
+    for (int e = threadIdx.x; e < KIN * BATCH_ROWS / 8; e += BATCH_THREADS) {
+        const int f = e >> 3, part = e & 7;
+        *(uint4*)(XT + (size_t)f * M + rb + 8 * part) = *(const uint4*)&tile[f][8 * (part ^ ((f >> 3) & 7))];
+    }
+}
+
+// Batch of M rows drawn uniformly (with replacement) from the data set:
+// X[M][128], XT[128][M], T[M][4].  Row r takes sample mix64(key + r) mod size;
+// block b draws rows [64 b, 64 b + 64) (M % 64 == 0).  16 threads per row move
+// its 256 bytes of features as 16-byte pieces (and one the 16-byte target).
 __global__ __launch_bounds__(BATCH_THREADS) void batch_kernel(const bf16_t* __restrict__ DX,
                                                               const float* __restrict__ DT, long size, uint64_t key,
                                                               int M, bf16_t* __restrict__ X, bf16_t* __restrict__ XT,
                                                               float* __restrict__ T) {
-    static_assert(KIN == 16 * 8 && BATCH_ROWS * KIN == BATCH_THREADS * 32, "16 pieces of 8 features per row");
-    __shared__ __align__(16) bf16_t tile[KIN][BATCH_ROWS + 8];
+    __shared__ __align__(16) BatchTile tile;
     const int piece = threadIdx.x & 15, rb = blockIdx.x * BATCH_ROWS;
 #pragma unroll
     for (int pass = 0; pass < BATCH_ROWS / 16; ++pass) {
@@ -716,25 +738,48 @@ __global__ __launch_bounds__(BATCH_THREADS) void batch_kernel(const bf16_t* __re
         const long p = (long)(mix64(key + (uint64_t)r) % (uint64_t)size);
         const uint4 v = *(const uint4*)(DX + (size_t)p * KIN + 8 * piece);
         *(uint4*)(X + (size_t)r * KIN + 8 * piece) = v;
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-        // row q's 8-row chunk sits at chunk (q / 8) ^ (piece % 8) of the
-        // feature's LDS row, so that the 16 pieces a write spans fall on 8 bank
-        // groups instead of 2
-        const int col = (((q >> 3) ^ (piece & 7)) << 3) | (q & 7);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            tile[8 * piece + 2 * j][col] = (bf16_t)(w[j] & 0xffffu);
-            tile[8 * piece + 2 * j + 1][col] = (bf16_t)(w[j] >> 16);
-        }
+        tile_put(tile, q, piece, v);
         if (piece == 0) *(float4*)(T + 4 * (size_t)r) = *(const float4*)(DT + 4 * (size_t)p);
     }
     __syncthreads();
-    // feature f of the block's rows: 64 contiguous elements of XT row f
+    tile_out(tile, rb, M, XT);
+}
+
+// Caller's FP32 feature rows (already in device memory) as the GEMMs read
+// them: X[M][128] in bf16 (rows m .. M-1 zero) and, with XT, its transpose
+// (M % 64 == 0).  Bound by HBM: 4 B in, 2 or 4 B out per feature.  With the
+// rounding and transposition done one element at a time on the host, a gradient
+// over 16,384 rows took 23-46 ms (two boxes), of which the GPU worked 0.12; here
+// the call takes 0.46 ms, bound by the copies of the rows and the gradient.
+template <bool TRANSPOSE>
+__global__ __launch_bounds__(BATCH_THREADS) void rows_kernel(const float* __restrict__ in, int m, int M,
+                                                             bf16_t* __restrict__ X, bf16_t* __restrict__ XT) {
+    __shared__ __align__(16) BatchTile tile;
+    const int piece = threadIdx.x & 15, rb = blockIdx.x * BATCH_ROWS;
 #pragma unroll
-    for (int e = threadIdx.x; e < KIN * BATCH_ROWS / 8; e += BATCH_THREADS) {
-        const int f = e >> 3, part = e & 7;
-        *(uint4*)(XT + (size_t)f * M + rb + 8 * part) = *(const uint4*)&tile[f][8 * (part ^ ((f >> 3) & 7))];
+    for (int pass = 0; pass < BATCH_ROWS / 16; ++pass) {
+        const int q = pass * 16 + (threadIdx.x >> 4), r = rb + q;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (r < m) {
+            const float4* src = (const float4*)(in + (size_t)r * KIN + 8 * piece);
+            const float4 a = src[0], b = src[1];
+            v.x = (uint32_t)f2bf(a.x) | ((uint32_t)f2bf(a.y) << 16);
+            v.y = (uint32_t)f2bf(a.z) | ((uint32_t)f2bf(a.w) << 16);
+            v.z = (uint32_t)f2bf(b.x) | ((uint32_t)f2bf(b.y) << 16);
+            v.w = (uint32_t)f2bf(b.z) | ((uint32_t)f2bf(b.w) << 16);
+        }
+        *(uint4*)(X + (size_t)r * KIN + 8 * piece) = v;
+        if (TRANSPOSE) tile_put(tile, q, piece, v);
     }
+    if (!TRANSPOSE) return;
+    __syncthreads();
+    tile_out(tile, rb, M, XT);
+}
+
+// The three outputs of each row, without the padding columns.
+__global__ __launch_bounds__(256) void outputs_kernel(const float* __restrict__ Yo, int m, float* __restrict__ y) {
+    const long e = (long)blockIdx.x * 256 + threadIdx.x;
+    if (e < (long)m * NOUT) y[e] = Yo[e / NOUT * KOUT + e % NOUT];
 }
 
 // dY = 2 w (Y - T) / M on the first 3 outputs (w = T[r][3]), 0 elsewhere,
@@ -1367,15 +1412,17 @@ extern "C" int ct2_mlp_forward(const float* x, size_t m, float* y) {
     CT2_TRY(ensure_work((int)m, false));
     Context& c = ctx();
     const int M = ((int)m + 127) / 128 * 128;
-    std::vector<bf16_t> hx((size_t)M * KIN, 0);
-    for (size_t i = 0; i < m * KIN; ++i) hx[i] = f2bf(x[i]);
-    CT2_HIP(hipMemcpyAsync(g_mlp.X, hx.data(), hx.size() * 2, hipMemcpyHostToDevice, c.stream));
+    float* rows = (float*)g_mlp.H1;  // as many bytes as the FP32 rows, written by layer 1 only
+    static_assert(HID * sizeof(bf16_t) == KIN * sizeof(float), "H1 holds the FP32 feature rows");
+    CT2_HIP(hipMemcpyAsync(rows, x, m * KIN * 4, hipMemcpyHostToDevice, c.stream));
+    rows_kernel<false><<<M / BATCH_ROWS, BATCH_THREADS, 0, c.stream>>>(rows, (int)m, M, g_mlp.X, nullptr);
+    CT2_LAUNCH_CHECK();
     CT2_TRY(forward(c.stream, M, false));
-    std::vector<float> hy((size_t)M * KOUT);
-    CT2_HIP(hipMemcpyAsync(hy.data(), g_mlp.Yo, hy.size() * 4, hipMemcpyDeviceToHost, c.stream));
+    float* out = (float*)g_mlp.H2;  // free once layer 3 is done
+    outputs_kernel<<<(unsigned)((m * NOUT + 255) / 256), 256, 0, c.stream>>>(g_mlp.Yo, (int)m, out);
+    CT2_LAUNCH_CHECK();
+    CT2_HIP(hipMemcpyAsync(y, out, m * NOUT * 4, hipMemcpyDeviceToHost, c.stream));
     CT2_HIP(hipStreamSynchronize(c.stream));
-    for (size_t r = 0; r < m; ++r)
-        for (int o = 0; o < NOUT; ++o) y[r * NOUT + o] = hy[r * KOUT + o];
     return CT2_OK;
 }
 
@@ -1388,17 +1435,11 @@ extern "C" int ct2_mlp_grad(const float* x, const float* t, size_t m, float* gra
     CT2_TRY(ensure_work((int)m, true));
     Context& c = ctx();
     const int M = (int)m;
-    std::vector<bf16_t> hx((size_t)M * KIN), hxt((size_t)M * KIN);
-    for (int r = 0; r < M; ++r)
-        for (int k = 0; k < KIN; ++k) {
-            const bf16_t v = f2bf(x[(size_t)r * KIN + k]);
-            hx[(size_t)r * KIN + k] = v;
-            hxt[(size_t)k * M + r] = v;
-        }
-    std::vector<float> ht(t, t + (size_t)M * 4);
-    CT2_HIP(hipMemcpyAsync(g_mlp.X, hx.data(), hx.size() * 2, hipMemcpyHostToDevice, c.stream));
-    CT2_HIP(hipMemcpyAsync(g_mlp.XT, hxt.data(), hxt.size() * 2, hipMemcpyHostToDevice, c.stream));
-    CT2_HIP(hipMemcpyAsync(g_mlp.T, ht.data(), ht.size() * 4, hipMemcpyHostToDevice, c.stream));
+    float* rows = (float*)g_mlp.H1;  // written by layer 1 only
+    CT2_HIP(hipMemcpyAsync(rows, x, m * KIN * 4, hipMemcpyHostToDevice, c.stream));
+    CT2_HIP(hipMemcpyAsync(g_mlp.T, t, m * 16, hipMemcpyHostToDevice, c.stream));
+    rows_kernel<true><<<M / BATCH_ROWS, BATCH_THREADS, 0, c.stream>>>(rows, M, M, g_mlp.X, g_mlp.XT);
+    CT2_LAUNCH_CHECK();
     CT2_TRY(forward(c.stream, M, true));
     CT2_TRY(backward(c.stream, M, nullptr));
     std::vector<float> lp(M / LOSS_ROWS);

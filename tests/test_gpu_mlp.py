@@ -249,3 +249,40 @@ def test_kick_pm_mlp_falls_back_to_the_direct_sum(ct2):
         assert ct2.last_force_path() == ct2.PATH_PM
     finally:
         ct2.pm_assignment(1)
+
+
+def bf16(a):
+    """Round to nearest even bf16, as float32."""
+    u = np.ascontiguousarray(a, np.float32).view(np.uint32).astype(np.uint64)
+    return ((u + 0x7fff + ((u >> 16) & 1)) & 0xffff0000).astype(np.uint32).view(np.float32)
+
+
+@pytest.mark.parametrize("m", [1, 63, 129, 384])
+def test_mlp_forward_rows_are_rounded_and_padded_on_the_device(ct2, m):
+    """Ragged row counts: a row's outputs do not depend on the rows beside it
+    or on the padding, and rows already rounded to bf16 give the same bits."""
+    ct2.mlp_init(7)
+    X = features(np.random.default_rng(m), 512)
+    full = ct2.mlp_forward(X)
+    assert np.array_equal(ct2.mlp_forward(X[:m]), full[:m])
+    assert np.array_equal(ct2.mlp_forward(bf16(X[:m])), full[:m])
+
+
+@pytest.mark.parametrize("m", [128, 2176])
+def test_mlp_grad_rows_are_rounded_and_transposed_on_the_device(ct2, m):
+    """The layer-1 weight gradient reads the transposed rows: rows already
+    rounded to bf16 give the same bits, and a feature that is zero everywhere
+    leaves exactly its own row of the gradient zero."""
+    ct2.mlp_init(11)
+    rng = np.random.default_rng(m)
+    X = features(rng, m)
+    T = np.concatenate([rng.standard_normal((m, 3)), rng.uniform(0.5, 2.0, (m, 1))], axis=1).astype(np.float32)
+    loss, g = ct2.mlp_grad(X, T)
+    loss2, g2 = ct2.mlp_grad(bf16(X), T)
+    assert loss == loss2 and np.array_equal(g, g2)
+    # a feature that is zero in every row has no gradient, its neighbours keep theirs
+    Z = X.copy()
+    Z[:, 37] = 0.0
+    gz = ct2.mlp_grad(Z, T)[1][:128 * 256].reshape(128, 256)
+    assert not gz[37].any() and not gz[111:].any()
+    assert (np.abs(gz[:111]).max(axis=1) > 0)[np.arange(111) != 37].all()
