@@ -15,20 +15,22 @@
 //       reference; here the planar layout out[(N/2+1)(N i + j) + k] = Re,
 //       + N^2 (N/2+1) for Im, that transpose.cpp:36-56 prepares).
 //
-// Each 1-D transform is one workgroup: the whole sequence sits in LDS as FP64
-// complex (N <= 4096: 64 KiB), log2 N radix-2 butterfly stages in place (the
-// input already is in bit-reversed order, so the classic iterative DIT
-// produces natural order), twiddles from an FP64 libm table, e^{-2 pi i m/N}.
+// The 1-D transforms sit in LDS as FP64 complex, several to a workgroup, and
+// take radix-8 decimation-in-time steps in place (the input already is in
+// bit-reversed order, so the output comes out in natural order), twiddles from
+// an FP64 libm table, e^{-2 pi i m/N}; a real transform is a complex one of
+// half the length.
 // The 3-D transforms run the FP64 3-D transform of fft.hip on a complex copy.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
+#include "fft_radix.h"
 #include "internal.h"
 
 namespace ct2 {
 namespace {
 
-constexpr int F1_THREADS = 256;
 constexpr int F1_MAXN = 4096;
 
 struct Twiddles {
@@ -39,15 +41,15 @@ std::vector<Twiddles> g_tw;
 double2* g_cplx = nullptr;  // 3-D scratch
 size_t g_cplx_bytes = 0;
 
-// Table W[m] = e^{-2 pi i m / N}, m < N/2, FP64 from libm.
+// Table W[m] = e^{-2 pi i m / N}, m < N, FP64 from libm.
 int twiddles(int N, const double2** out) {
     for (const Twiddles& t : g_tw)
         if (t.n == N) {
             *out = t.d;
             return CT2_OK;
         }
-    std::vector<double2> h(std::max(1, N / 2));
-    for (int m = 0; m < N / 2; ++m) h[m] = make_double2(std::cos(2.0 * M_PI * m / N), -std::sin(2.0 * M_PI * m / N));
+    std::vector<double2> h(N);
+    for (int m = 0; m < N; ++m) h[m] = make_double2(std::cos(2.0 * M_PI * m / N), -std::sin(2.0 * M_PI * m / N));
     Twiddles t;
     t.n = N;
     CT2_TRY(dev_alloc((void**)&t.d, h.size() * sizeof(double2), "1-D FFT twiddles"));
@@ -57,53 +59,100 @@ int twiddles(int N, const double2** out) {
     return CT2_OK;
 }
 
-__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-    return make_double2(fma(a.x, b.x, -a.y * b.y), fma(a.x, b.y, a.y * b.x));
-}
-
-// One workgroup per (batch, lane) transform.
-template <bool REAL>
-__global__ __launch_bounds__(F1_THREADS) void fft1d_ct2(double* __restrict__ X, int N, int lanes, int dir,
-                                                        const double2* __restrict__ W) {
-    extern __shared__ double2 s[];
-    const int t = blockIdx.x;
-    const long b = t / lanes;
-    const int l = t % lanes;
-    const int tid = threadIdx.x;
-    if (REAL) {
-        const double* src = X + b * lanes * N;
-        for (int n = tid; n < N; n += F1_THREADS) s[n] = make_double2(src[(long)lanes * n + l], 0.0);
-    } else {
-        const double* src = X + b * 2 * lanes * N;
-        for (int n = tid; n < N; n += F1_THREADS)
-            s[n] = make_double2(src[2L * lanes * n + l], src[2L * lanes * n + lanes + l]);
+// One radix-R step (log2 R stages) of the transforms in LDS, T of M = 2^lm
+// complex elements each, sub-transforms of 2^lh already done: outputs
+// k + q h (q < R) of a group from its R sub-transforms' element k, which sit
+// in bit-reversed order of the sub-transform.  W is the table of 2^(lm + 1)
+// or 2^lm roots (ws = 1 or 0).
+template <int R>
+__device__ __forceinline__ void f1_step(double2* s, int threads, int T, int lm, int lh, int pitch,
+                                        const double2* __restrict__ W, int ws) {
+    constexpr int LR = R == 8 ? 3 : R == 4 ? 2 : 1;
+    const int lq = lm - LR, nb = T << lq;
+    for (int b = threadIdx.x; b < nb; b += threads) {
+        const int q = b & ((1 << lq) - 1), k = q & ((1 << lh) - 1);
+        const int base = ((q - k) << LR) + k;
+        double2* row = s + (b >> lq) * pitch;
+        double2 v[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const int rev = R == 8 ? ((j & 1) << 2 | (j & 2) | j >> 2) : R == 4 ? ((j & 1) << 1 | j >> 1) : j;
+            const int i = base + (rev << lh);
+            v[j] = row[i + (i >> 3)];
+            if (lh > 0 && j > 0) v[j] = cmul(v[j], W[(j * k) << (lm - lh - LR + ws)]);
+        }
+        dft<R, 1>(v);
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const int i = base + (j << lh);
+            row[i + (i >> 3)] = v[j];
+        }
     }
     __syncthreads();
-    for (int half = 1; half < N; half <<= 1) {
-        const int stride = N / (2 * half);
-        for (int q = tid; q < N / 2; q += F1_THREADS) {
-            const int k = q & (half - 1);
-            const int i0 = ((q - k) << 1) + k, i1 = i0 + half;
-            double2 w = W[k * stride];
-            if (dir < 0) w.y = -w.y;
-            const double2 a = s[i0], c = cmul(s[i1], w);
-            s[i0] = make_double2(a.x + c.x, a.y + c.y);
-            s[i1] = make_double2(a.x - c.x, a.y - c.y);
-        }
-        __syncthreads();
+}
+
+// T = E / M transforms per workgroup of E / 8 threads, in LDS: transform t,
+// element e at t pitch + e + e/8 (the padding keeps the radix-8 steps' strided
+// accesses, and the lanes of a group, off one bank group).  A transform holds 2 M doubles in memory, M = 2^lm:
+//   complex (N = M): row r of a group's 2 M x L array is part r % 2 of element
+//     r / 2;
+//   real (N = 2 M): bit-reversed input holds the even samples in its first
+//     half and the odd ones in its second, each again bit-reversed, so row r
+//     is part r / M of element r % M of z = x_even + i x_odd, and
+//     F_k = (Z_k + conj Z_{M-k}) / 2 - i W_N^k (Z_k - conj Z_{M-k}) / 2.
+// dir = -1: the conjugate transform, as swapped parts in and out (complex) or
+// the conjugate output (real).
+// Bound by HBM (32 B per complex element, 16 B per real one) and the LDS
+// passes: log8 M steps, one barrier each.  A group's L lanes stay in one
+// workgroup wherever they fit (E up to 8192 elements, 148 KB), so that its
+// interleaved lines are read once: 2,048 x 4 real transforms of 1,024 (67 MB
+// each way) take 47 us.  One transform per workgroup with a radix-2
+// stage per barrier, and every lane of a group read by another workgroup, took
+// 121 us.
+template <bool REAL, int L, int E>
+__global__ __launch_bounds__(E / 8) void fft1d_ct2(double* __restrict__ X, int lm, long nt, int T, int dir,
+                                                   const double2* __restrict__ W) {
+    constexpr int TH = E / 8;
+    __shared__ double2 s[E + E / 8 + E / 32];
+    const int M = 1 << lm, pitch = M + (M >> 3) + (lm >= 5);
+    const long t0 = (long)blockIdx.x * T;
+    const int Lw = min(T, L);                     // lanes of a group in this workgroup
+    const int ll = 31 - __clz(Lw);                // Lw is 1, 2 or 4
+    const int have = (int)min((long)T, nt - t0);  // a multiple of Lw: nt and t0 are
+    const int swap = !REAL && dir < 0;
+    const int nd = have << (lm + 1);
+    const long g0 = t0 / L, l0 = t0 % L;
+    auto address = [&](int d) -> long {  // double d of the workgroup, in memory order
+        const int l = d & (Lw - 1), r = (d >> ll) & (2 * M - 1), g = d >> (ll + lm + 1);
+        return (((g0 + g) << (lm + 1)) + r) * L + l0 + l;
+    };
+    for (int d = threadIdx.x; d < nd; d += TH) {
+        const int l = d & (Lw - 1), r = (d >> ll) & (2 * M - 1), g = d >> (ll + lm + 1);
+        const int e = REAL ? r & (M - 1) : r >> 1;
+        const int part = REAL ? r >> lm : (r & 1) ^ swap;
+        ((double*)&s[((g << ll) + l) * pitch + e + (e >> 3)])[part] = X[address(d)];
     }
-    if (REAL) {
-        double* dst = X + b * lanes * N;
-        for (int k = tid; k <= N / 2; k += F1_THREADS) {
-            const double2 v = s[k];
-            dst[(long)lanes * k + l] = v.x;
-            if (k > 0 && k < N / 2) dst[(long)lanes * (N - k) + l] = v.y;
-        }
-    } else {
-        double* dst = X + b * 2 * lanes * N;
-        for (int n = tid; n < N; n += F1_THREADS) {
-            dst[2L * lanes * n + l] = s[n].x;
-            dst[2L * lanes * n + lanes + l] = s[n].y;
+    __syncthreads();
+    const int ws = REAL ? 1 : 0;
+    int lh = lm % 3;
+    if (lh == 1) f1_step<2>(s, TH, have, lm, 0, pitch, W, ws);
+    if (lh == 2) f1_step<4>(s, TH, have, lm, 0, pitch, W, ws);
+    for (; lh < lm; lh += 3) f1_step<8>(s, TH, have, lm, lh, pitch, W, ws);
+    for (int d = threadIdx.x; d < nd; d += TH) {
+        const int l = d & (Lw - 1), r = (d >> ll) & (2 * M - 1), g = d >> (ll + lm + 1);
+        const double2* row = s + ((g << ll) + l) * pitch;
+        if constexpr (REAL) {  // row r of the half-complex output: Re F_r, or Im F_{N-r} above N/2
+            const bool im = r > M;
+            const int k = im ? 2 * M - r : r;
+            const int a = k & (M - 1), b = (M - k) & (M - 1);
+            const double2 z1 = row[a + (a >> 3)], z2 = row[b + (b >> 3)], w = W[k];
+            const double ox = 0.5 * (z1.x - z2.x), oy = 0.5 * (z1.y + z2.y);
+            const double re = 0.5 * (z1.x + z2.x) + (w.x * oy + w.y * ox);
+            const double mi = 0.5 * (z1.y - z2.y) - (w.x * ox - w.y * oy);
+            X[address(d)] = im ? (dir < 0 ? -mi : mi) : re;
+        } else {
+            const int e = r >> 1;
+            X[address(d)] = ((const double*)&row[e + (e >> 3)])[(r & 1) ^ swap];
         }
     }
 }
@@ -221,6 +270,28 @@ int check_1d(const void* X, int N, int dir, int lanes, size_t batch) {
     return CT2_OK;
 }
 
+template <bool REAL, int L, int E>
+int fft1d_launch(double* X, int N, int dir, size_t batch) {
+    const double2* W;
+    CT2_TRY(twiddles(N, &W));
+    const int lm = ilog2(N) - (REAL ? 1 : 0);
+    const int T = E >> lm;
+    const long nt = (long)batch * L;
+    fft1d_ct2<REAL, L, E><<<(unsigned)((nt + T - 1) / T), E / 8, 0, ctx().stream>>>(X, lm, nt, T, dir, W);
+    CT2_LAUNCH_CHECK();
+    return CT2_OK;
+}
+
+// 2048 elements per workgroup (256 threads, four workgroups per CU), more
+// where a group's lanes or a single transform need it.
+template <bool REAL, int L>
+int fft1d_elements(double* X, int N, int dir, size_t batch) {
+    const int need = (REAL ? N / 2 : N) * L;
+    if (need <= 2048) return fft1d_launch<REAL, L, 2048>(X, N, dir, batch);
+    if (need <= 4096) return fft1d_launch<REAL, L, 4096>(X, N, dir, batch);
+    return fft1d_launch<REAL, L, 8192>(X, N, dir, batch);
+}
+
 int grid_1d(long total) { return (int)((total + 255) / 256); }
 
 int check_3d(const void* a, const void* b, int N) {
@@ -246,22 +317,12 @@ using namespace ct2;
 
 extern "C" int ct2_fft_complex_1d(double* X, int N, int dir, int lanes, size_t batch) {
     CT2_TRY(check_1d(X, N, dir, lanes, batch));
-    const double2* W;
-    CT2_TRY(twiddles(N, &W));
-    Context& c = ctx();
-    fft1d_ct2<false><<<(unsigned)(batch * lanes), F1_THREADS, N * sizeof(double2), c.stream>>>(X, N, lanes, dir, W);
-    CT2_LAUNCH_CHECK();
-    return CT2_OK;
+    return lanes == 1 ? fft1d_elements<false, 1>(X, N, dir, batch) : fft1d_elements<false, 4>(X, N, dir, batch);
 }
 
 extern "C" int ct2_fft_real_1d(double* X, int N, int dir, int lanes, size_t batch) {
     CT2_TRY(check_1d(X, N, dir, lanes, batch));
-    const double2* W;
-    CT2_TRY(twiddles(N, &W));
-    Context& c = ctx();
-    fft1d_ct2<true><<<(unsigned)(batch * lanes), F1_THREADS, N * sizeof(double2), c.stream>>>(X, N, lanes, dir, W);
-    CT2_LAUNCH_CHECK();
-    return CT2_OK;
+    return lanes == 1 ? fft1d_elements<true, 1>(X, N, dir, batch) : fft1d_elements<true, 4>(X, N, dir, batch);
 }
 
 extern "C" int ct2_scramble(double* X, int N1, int N2, int N3) {

@@ -34,6 +34,26 @@ def test_fft_real_1d(ct2, orc, N, lanes, dir):
     assert relerr(got, want) < 1e-14
 
 
+@pytest.mark.parametrize("N,lanes,batch", [(2, 1, 700), (4, 4, 130), (16, 1, 129), (64, 4, 33), (128, 1, 17), (512, 1, 5),
+                                           (1024, 4, 2), (2048, 1, 3), (2048, 4, 3), (4096, 1, 2), (4096, 4, 2)])
+@pytest.mark.parametrize("dir", [1, -1])
+def test_fft_1d_ragged_batches(ct2, orc, N, lanes, batch, dir):
+    """Batches that end inside a workgroup's set of transforms, every radix
+    remainder (2, 4, none) and the sizes where a group's lanes share a
+    workgroup or split over two.  A transform rounds to a few FP64 ulps per
+    step, so 1e-14 bounds log2 N of them."""
+    rng = np.random.default_rng(N * lanes + batch)
+    scale = np.repeat(10.0 ** rng.integers(-6, 7, batch), lanes * N)  # transforms of unequal size stay apart
+    X = rng.standard_normal(batch * lanes * N) * scale
+    got, want = ct2.fft_real(X, N, dir, lanes), [orc.fft_real(g, N, dir, lanes) for g in np.split(X, batch)]
+    for g, w in zip(np.split(got, batch), want):
+        assert relerr(g, w) < 1e-14
+    X = rng.standard_normal(2 * batch * lanes * N)
+    got, want = ct2.fft_complex(X, N, dir, lanes), [orc.fft_complex(g, N, dir, lanes) for g in np.split(X, batch)]
+    for g, w in zip(np.split(got, batch), want):
+        assert relerr(g, w) < 1e-14
+
+
 def test_fft_real_matches_numpy_after_scramble(ct2, orc):
     """End to end in ct2's order of calls (fft_test.cpp:108-127): scramble on
     the device, then fft_real; the half-complex result equals numpy's rfft."""
