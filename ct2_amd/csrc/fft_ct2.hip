@@ -20,7 +20,7 @@
 // bit-reversed order, so the output comes out in natural order), twiddles from
 // an FP64 libm table, e^{-2 pi i m/N}; a real transform is a complex one of
 // half the length.
-// The 3-D transforms run the FP64 3-D transform of fft.hip on a complex copy.
+// The 3-D transforms are fft.hip's real ones.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -38,8 +38,8 @@ struct Twiddles {
     double2* d = nullptr;
 };
 std::vector<Twiddles> g_tw;
-double2* g_cplx = nullptr;  // 3-D scratch
-size_t g_cplx_bytes = 0;
+double2* g_half = nullptr;  // 3-D scratch: a half spectrum
+size_t g_half_bytes = 0;
 
 // Table W[m] = e^{-2 pi i m / N}, m < N, FP64 from libm.
 int twiddles(int N, const double2** out) {
@@ -219,47 +219,6 @@ __global__ __launch_bounds__(256) void transpose_c2r_kernel(const double* __rest
     if (iy != 0 && iy != N / 2) out[(ix * N + (N - iy)) * N + iz] = in[jr + dimag];
 }
 
-__global__ __launch_bounds__(256) void real_to_cplx(const double* __restrict__ in, double2* __restrict__ c, long n3) {
-    const long q = (long)blockIdx.x * 256 + threadIdx.x;
-    if (q < n3) c[q] = make_double2(in[q], 0.0);
-}
-
-// Planar half spectrum from the full complex spectrum.
-__global__ __launch_bounds__(256) void cplx_to_planar(const double2* __restrict__ c, double* __restrict__ out, int N) {
-    const int h = N / 2 + 1;
-    const long e = (long)blockIdx.x * 256 + threadIdx.x;
-    const long tot = (long)N * N * h;
-    if (e >= tot) return;
-    const int k = (int)(e % h);
-    const long ij = e / h;
-    const double2 v = c[ij * N + k];
-    out[e] = v.x;
-    out[tot + e] = v.y;
-}
-
-// Full Hermitian spectrum from the planar half spectrum.
-__global__ __launch_bounds__(256) void planar_to_cplx(const double* __restrict__ in, double2* __restrict__ c, int N) {
-    const int h = N / 2 + 1;
-    const long e = (long)blockIdx.x * 256 + threadIdx.x;
-    const long n3 = (long)N * N * N;
-    if (e >= n3) return;
-    const long dimag = (long)N * N * h;
-    const int k = (int)(e % N), j = (int)((e / N) % N), i = (int)(e / ((long)N * N));
-    if (k < h) {
-        const long q = ((long)i * N + j) * h + k;
-        c[e] = make_double2(in[q], in[dimag + q]);
-    } else {
-        const int i2 = (N - i) % N, j2 = (N - j) % N, k2 = N - k;
-        const long q = ((long)i2 * N + j2) * h + k2;
-        c[e] = make_double2(in[q], -in[dimag + q]);
-    }
-}
-
-__global__ __launch_bounds__(256) void cplx_to_real(const double2* __restrict__ c, double* __restrict__ out, long n3) {
-    const long q = (long)blockIdx.x * 256 + threadIdx.x;
-    if (q < n3) out[q] = c[q].x;
-}
-
 int check_1d(const void* X, int N, int dir, int lanes, size_t batch) {
     CT2_TRY(require_init());
     if (!X) return set_error(CT2_ERR_INVALID, "null data");
@@ -306,9 +265,9 @@ int check_3d(const void* a, const void* b, int N) {
 void release_fft_ct2() {
     for (Twiddles& t : g_tw) dev_free(t.d);
     g_tw.clear();
-    dev_free(g_cplx);
-    g_cplx = nullptr;
-    g_cplx_bytes = 0;
+    dev_free(g_half);
+    g_half = nullptr;
+    g_half_bytes = 0;
 }
 
 }  // namespace ct2
@@ -359,30 +318,18 @@ extern "C" int ct2_transpose_c2r(const double* in, double* out, int N) {
     return CT2_OK;
 }
 
+// Both directions read all of `in` into the scratch before the first write of
+// `out`, which may overlap it.
 extern "C" int ct2_fft_r2c_3d(const double* in, double* out, int N) {
     CT2_TRY(check_3d(in, out, N));
-    Context& c = ctx();
-    const long n3 = (long)N * N * N;
-    CT2_TRY(ensure_scratch((void**)&g_cplx, &g_cplx_bytes, n3 * sizeof(double2), "3-D r2c scratch"));
-    real_to_cplx<<<grid_1d(n3), 256, 0, c.stream>>>(in, g_cplx, n3);
-    CT2_LAUNCH_CHECK();
-    CT2_TRY(fft3d(g_cplx, N, 1, true));
-    cplx_to_planar<<<grid_1d((long)N * N * (N / 2 + 1)), 256, 0, c.stream>>>(g_cplx, out, N);
-    CT2_LAUNCH_CHECK();
-    return CT2_OK;
+    CT2_TRY(ensure_scratch((void**)&g_half, &g_half_bytes, fft_half_elems(N) * sizeof(double2), "3-D r2c scratch"));
+    return rfft3d_f64(in, out, g_half, N);
 }
 
 extern "C" int ct2_fft_c2r_3d(const double* in, double* out, int N) {
     CT2_TRY(check_3d(in, out, N));
-    Context& c = ctx();
-    const long n3 = (long)N * N * N;
-    CT2_TRY(ensure_scratch((void**)&g_cplx, &g_cplx_bytes, n3 * sizeof(double2), "3-D c2r scratch"));
-    planar_to_cplx<<<grid_1d(n3), 256, 0, c.stream>>>(in, g_cplx, N);
-    CT2_LAUNCH_CHECK();
-    CT2_TRY(fft3d(g_cplx, N, -1, true));
-    cplx_to_real<<<grid_1d(n3), 256, 0, c.stream>>>(g_cplx, out, n3);
-    CT2_LAUNCH_CHECK();
-    return CT2_OK;
+    CT2_TRY(ensure_scratch((void**)&g_half, &g_half_bytes, fft_half_elems(N) * sizeof(double2), "3-D c2r scratch"));
+    return irfft3d_f64(in, out, g_half, N);
 }
 
 extern "C" int ct2_twiddles(int N, double* cosw, double* sinw, double* invsinw) {

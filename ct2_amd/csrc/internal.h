@@ -64,6 +64,11 @@ int fft3d(void* data, int n, int dir, bool f64);
 // `batch` such cubes stored one after the other, in one set of launches.
 int fft3d_batch(void* data, int n, int dir, bool f64, int batch);
 int fft3d_density(const unsigned long long* W, void* out, int n);
+// Complex elements of the half spectrum of an n^3 real field: the columns
+// kz < n/2, then kz = n/2.
+constexpr size_t fft_half_elems(size_t n) { return n * n * (n / 2 + 1); }
+int rfft3d_f64(const double* in, double* planar, double2* half, int n);
+int irfft3d_f64(const double* planar, double* out, double2* half, int n);
 
 // PM force of the container into the context force arrays (pm.hip).
 int pm_forces();

@@ -96,6 +96,59 @@ def test_fft_r2c_c2r_3d(ct2, orc, N):
     assert relerr(Z / N ** 3, X) < 1e-14
 
 
+@pytest.mark.parametrize("N", [8, 16, 128, 256, 512])
+def test_fft_r2c_c2r_3d_half_spectrum(ct2, N):
+    """Every size class of the half-spectrum passes (one-stage and multi-stage
+    rows, 4 to 16 columns per workgroup, the kz = N/2 plane on its own) against
+    numpy, with a mean much larger than the fluctuations.  The FP64 transforms
+    round to a few ulps per stage: 1e-14."""
+    X = np.random.default_rng(N).standard_normal(N ** 3) + 50.0
+    Y = ct2.fft_r2c_3d(X)
+    R = np.fft.rfftn(X.reshape(N, N, N))
+    h = N * N * (N // 2 + 1)
+    assert relerr(Y[:h], R.real.ravel()) < 1e-14
+    Y[0], R[0, 0, 0] = 0.0, 0.0  # the fluctuations on their own, against the error of the mean
+    e = np.hypot(Y[:h] - R.real.ravel(), Y[h:] - R.imag.ravel())
+    assert np.linalg.norm(e) < 50.0 * 1e-14 * np.linalg.norm(R) and e[N // 2::N // 2 + 1].max() < 50.0 * 1e-14 * N ** 1.5 * 10
+    Z = ct2.fft_c2r_3d(Y, N)
+    assert relerr(Z / N ** 3, X - X.mean()) < 50.0 * 1e-14
+
+
+@pytest.mark.parametrize("N", [8, 32])
+def test_fft_c2r_3d_of_any_half_spectrum(ct2, N):
+    """A planar spectrum whose kz = 0 and N/2 planes have no Hermitian symmetry:
+    the result is the real part of the complex transform, those planes taken as
+    they are and the columns above N/2 as the partners' conjugates."""
+    h = N // 2 + 1
+    Y = np.random.default_rng(N).standard_normal(2 * N * N * h)
+    C = (Y[:N * N * h] + 1j * Y[N * N * h:]).reshape(N, N, h)
+    full = np.zeros((N, N, N), complex)
+    full[:, :, :h] = C
+    neg = (-np.arange(N)) % N
+    full[:, :, h:] = np.conj(C[neg][:, neg][:, :, h - 2:0:-1])
+    want = (np.fft.ifftn(full) * N ** 3).real
+    assert relerr(ct2.fft_c2r_3d(Y, N), want.ravel()) < 1e-14
+
+
+def test_fft_r2c_c2r_3d_in_place(ct2):
+    """Input and output in one device buffer (the library reads all of the
+    input before it writes)."""
+    from ct2_amd import _lib
+
+    N = 32
+    h = N * N * (N // 2 + 1)
+    X = np.random.default_rng(1).standard_normal(N ** 3)
+    buf = ct2.DeviceBuffer(2 * h * 8)
+    buf.upload(X)
+    _lib.check(_lib.load().ct2_fft_r2c_3d(buf.ptr, buf.ptr, N))
+    ct2.synchronize()
+    assert np.array_equal(buf.download(np.empty(2 * h)), ct2.fft_r2c_3d(X))
+    _lib.check(_lib.load().ct2_fft_c2r_3d(buf.ptr, buf.ptr, N))
+    ct2.synchronize()
+    assert relerr(buf.download(np.empty(N ** 3)) / N ** 3, X) < 1e-14
+    buf.close()
+
+
 def test_twiddles(ct2, orc):
     for N in (8, 1000, 4096):
         for a, b in zip(ct2.twiddles(N), orc.twiddles(N)):
