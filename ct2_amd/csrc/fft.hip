@@ -10,7 +10,8 @@
 //   y and x passes (stride n and n^2): `fft_cols`, C adjacent columns per
 //     workgroup so that every HBM access is a C*sizeof(complex) segment
 //     (128 bytes for FP32 at C=16).
-// Real fields go through half spectra
+// Cubes whose planes fit in LDS take the z and y passes, and the smallest all
+// three, in one kernel (`fft_block`).  Real fields go through half spectra
 // (`rfft_rows`, `half_cols`, `irfft_rows`): half the bytes of a complex
 // transform per pass.
 // Twiddles W_N^m are tabulated once per size on the host in FP64 libm
@@ -86,6 +87,62 @@ __global__ __launch_bounds__((col_lanes<T, N>())) void fft_cols(typename V2<T>::
     run_stages<T, N, DIR, false, false>([&](int i, int) { return data[(long)i * stride_i]; },
                                         [&](int i, int, T2 v) { data[(long)i * stride_i] = v; },
                                         [&](int i) { return i * CF::COLS + c; }, sm, tw, p);
+}
+
+// The z and y passes of one x plane, or all three of a cube (N <= 16), in LDS:
+// one read and one write of HBM for the axes it covers, and a launch fewer
+// (small cubes are bound by launches of ~3 us).  A phase gives each line P
+// lanes; the lanes of a column phase run over z.  Taken wherever a plane fits
+// (FP32 N <= 128, FP64 N <= 64).  us per transform, one pass per axis -> this:
+// FP32 8^3 8.0 -> 2.9, 16^3 8.1 -> 4.5, 32^3 8.0 -> 5.6, 64^3 10.3 -> 8.3, 128^3
+// 34 -> 28 (128 workgroups, one per CU); FP64 8^3 7.7 -> 2.8, 64^3 14.1 -> 11.3;
+// 83 FP32 cubes of 64^3 as the multipole mesh transforms them: 158 -> 107.
+template <typename T, int N, bool CUBE>
+struct Block {
+    using CF = Cfg<T, N>;
+    static constexpr int LINES = CUBE ? N * N : N;  // per phase
+    static constexpr int ELEMS = LINES * CF::ROWLEN;
+    static constexpr int TH = LINES * CF::P < 1024 ? LINES * CF::P : 1024;
+    static constexpr int LPI = TH / CF::P;  // lines at a time
+    static constexpr bool ok = (ELEMS + N) * (int)sizeof(typename V2<T>::t) <= 160 * 1024;
+};
+
+template <typename T, int N, int DIR, bool CUBE>
+__global__ __launch_bounds__((Block<T, N, CUBE>::TH)) void fft_block(typename V2<T>::t* __restrict__ data,
+                                                                    const typename V2<T>::t* __restrict__ twg) {
+    using T2 = typename V2<T>::t;
+    using CF = Cfg<T, N>;
+    using BK = Block<T, N, CUBE>;
+    __shared__ T2 sm[BK::ELEMS];
+    __shared__ T2 tw[N];
+    load_twiddles<N>(tw, twg, BK::TH);
+    data += (size_t)blockIdx.x * BK::LINES * N;  // plane (or cube) blockIdx.x of the batch
+    for (int l0 = 0; l0 < BK::LINES; l0 += BK::LPI) {  // z lines: line l holds (x, y)
+        const int p = threadIdx.x % CF::P, l = l0 + threadIdx.x / CF::P;
+        auto ix = [&](int i) { return l * CF::ROWLEN + i + (i >> 3); };
+        run_stages<T, N, DIR, false, true>([&](int i, int) { return data[l * N + i]; },
+                                           [&](int i, int, T2 v) { sm[ix(i)] = v; }, ix, sm, tw, p);
+    }
+    __syncthreads();
+    const int p = threadIdx.x / BK::LPI;
+    for (int l0 = 0; l0 < BK::LINES; l0 += BK::LPI) {  // y lines: line l holds (x, z)
+        const int l = l0 + threadIdx.x % BK::LPI, z = l % N, x = l / N;
+        auto ix = [&](int i) { return (x * N + i) * CF::ROWLEN + z + (z >> 3); };
+        auto ld = [&](int i, int) { return sm[ix(i)]; };
+        if constexpr (CUBE)
+            run_stages<T, N, DIR, true, true>(ld, [&](int i, int, T2 v) { sm[ix(i)] = v; }, ix, sm, tw, p);
+        else
+            run_stages<T, N, DIR, true, false>(ld, [&](int i, int, T2 v) { data[i * N + z] = v; }, ix, sm, tw, p);
+    }
+    if constexpr (CUBE) {
+        __syncthreads();
+        for (int l0 = 0; l0 < BK::LINES; l0 += BK::LPI) {  // x lines: line l holds (y, z)
+            const int l = l0 + threadIdx.x % BK::LPI, z = l % N, y = l / N;
+            auto ix = [&](int i) { return (i * N + y) * CF::ROWLEN + z + (z >> 3); };
+            run_stages<T, N, DIR, true, false>([&](int i, int) { return sm[ix(i)]; },
+                                               [&](int i, int, T2 v) { data[(i * N + y) * N + z] = v; }, ix, sm, tw, p);
+        }
+    }
 }
 
 // ------------------------------------------------------------ real fields
@@ -242,27 +299,48 @@ int twiddle_table(int N, const typename V2<T>::t** out) {
     return CT2_OK;
 }
 
-// batch cubes of N^3 one after the other; the uint64 source (wsrc) only with
-// batch 1
+// z and y passes of batch cubes of N^3, one after the other; the uint64 source
+// (wsrc) only with batch 1
 template <typename T, int N, int DIR>
-int fft3d_launch(typename V2<T>::t* d, hipStream_t st, int batch, const unsigned long long* wsrc = nullptr) {
+int fft_zy(typename V2<T>::t* d, const typename V2<T>::t* tw, hipStream_t st, int batch, const unsigned long long* wsrc) {
+    if constexpr (Block<T, N, false>::ok) {
+        if (!wsrc) {
+            fft_block<T, N, DIR, false><<<(unsigned)(N * batch), Block<T, N, false>::TH, 0, st>>>(d, tw);
+            CT2_LAUNCH_CHECK();
+            return CT2_OK;
+        }
+    }
     using CF = Cfg<T, N>;
-    const typename V2<T>::t* tw = nullptr;
-    CT2_TRY(twiddle_table<T>(N, &tw));
-    // z
+    constexpr int inner = N / CF::COLS;
     const dim3 rows((unsigned)(N * N / CF::ROWS), batch);
     if (wsrc)
         fft_rows<T, N, DIR, true><<<rows, row_lanes<T, N>(), 0, st>>>(d, tw, wsrc);
     else
         fft_rows<T, N, DIR><<<rows, row_lanes<T, N>(), 0, st>>>(d, tw);
     CT2_LAUNCH_CHECK();
-    constexpr int inner = N / CF::COLS;
-    const dim3 cols((unsigned)(N * inner), batch);
     // y: columns z, slabs x
-    fft_cols<T, N, DIR><<<cols, col_lanes<T, N>(), 0, st>>>(d, tw, N, (long)N * N, inner, false);
+    fft_cols<T, N, DIR><<<dim3((unsigned)(N * inner), batch), col_lanes<T, N>(), 0, st>>>(d, tw, N, (long)N * N, inner,
+                                                                                          false);
     CT2_LAUNCH_CHECK();
+    return CT2_OK;
+}
+
+template <typename T, int N, int DIR>
+int fft3d_launch(typename V2<T>::t* d, hipStream_t st, int batch, const unsigned long long* wsrc = nullptr) {
+    const typename V2<T>::t* tw = nullptr;
+    CT2_TRY(twiddle_table<T>(N, &tw));
+    if constexpr (N <= 16) {
+        if (!wsrc) {
+            fft_block<T, N, DIR, true><<<(unsigned)batch, Block<T, N, true>::TH, 0, st>>>(d, tw);
+            CT2_LAUNCH_CHECK();
+            return CT2_OK;
+        }
+    }
+    CT2_TRY((fft_zy<T, N, DIR>(d, tw, st, batch, wsrc)));
     // x: columns z, slabs y
-    fft_cols<T, N, DIR><<<cols, col_lanes<T, N>(), 0, st>>>(d, tw, (long)N * N, N, inner, true);
+    constexpr int inner = N / Cfg<T, N>::COLS;
+    fft_cols<T, N, DIR><<<dim3((unsigned)(N * inner), batch), col_lanes<T, N>(), 0, st>>>(d, tw, (long)N * N, N, inner,
+                                                                                          true);
     CT2_LAUNCH_CHECK();
     return CT2_OK;
 }
