@@ -39,12 +39,9 @@ constexpr int row_lanes() {
 
 // z pass: lines of N contiguous elements; workgroup = ROWS lines; cube
 // blockIdx.y of a batch.
-// With U64 the lines are read from the uint64 field wsrc (real, scaled by
-// 2^-32) and the transform is written to data.
-template <typename T, int N, int DIR, bool U64 = false>
+template <typename T, int N, int DIR>
 __global__ __launch_bounds__((row_lanes<T, N>())) void fft_rows(typename V2<T>::t* __restrict__ data,
-                                                               const typename V2<T>::t* __restrict__ twg,
-                                                               const unsigned long long* __restrict__ wsrc = nullptr) {
+                                                               const typename V2<T>::t* __restrict__ twg) {
     using T2 = typename V2<T>::t;
     using CF = Cfg<T, N>;
     __shared__ T2 sm[CF::ROWS * CF::ROWLEN];
@@ -52,13 +49,8 @@ __global__ __launch_bounds__((row_lanes<T, N>())) void fft_rows(typename V2<T>::
     load_twiddles<N>(tw, twg, row_lanes<T, N>());
     const int p = threadIdx.x % CF::P;
     const int c = threadIdx.x / CF::P;
-    const size_t at = (size_t)blockIdx.y * ((size_t)N * N * N) + ((size_t)blockIdx.x * CF::ROWS + c) * N;
-    data += at;
-    auto ld = [&](int i, int) {
-        if constexpr (U64) return T2{(T)((double)wsrc[at + i] * 0x1p-32), (T)0};
-        return data[i];
-    };
-    run_stages<T, N, DIR, false, false>(ld, [&](int i, int, T2 v) { data[i] = v; },
+    data += (size_t)blockIdx.y * ((size_t)N * N * N) + ((size_t)blockIdx.x * CF::ROWS + c) * N;
+    run_stages<T, N, DIR, false, false>([&](int i, int) { return data[i]; }, [&](int i, int, T2 v) { data[i] = v; },
                                         [&](int i) { return c * CF::ROWLEN + i + (i >> 3); }, sm, tw, p);
 }
 
@@ -157,6 +149,16 @@ struct RealField {
     template <typename T2>
     __device__ __forceinline__ T2 pair(long at) const {
         return T2{f[at], f[at + 1]};
+    }
+};
+
+struct DensityField {  // uint64 fixed point, 2^-32 units
+    const unsigned long long* w;
+    template <typename T2>
+    __device__ __forceinline__ T2 pair(long at) const {
+        using T = decltype(T2{}.x);
+        const ulonglong2 v = *(const ulonglong2*)(w + at);
+        return T2{(T)((double)v.x * 0x1p-32), (T)((double)v.y * 0x1p-32)};
     }
 };
 
@@ -299,49 +301,42 @@ int twiddle_table(int N, const typename V2<T>::t** out) {
     return CT2_OK;
 }
 
-// z and y passes of batch cubes of N^3, one after the other; the uint64 source
-// (wsrc) only with batch 1
+// z and y passes of batch cubes of N^3, one after the other (each axis is
+// independent, so they may also follow the x pass)
 template <typename T, int N, int DIR>
-int fft_zy(typename V2<T>::t* d, const typename V2<T>::t* tw, hipStream_t st, int batch, const unsigned long long* wsrc) {
+int fft_zy(typename V2<T>::t* d, const typename V2<T>::t* tw, hipStream_t st, int batch) {
     if constexpr (Block<T, N, false>::ok) {
-        if (!wsrc) {
-            fft_block<T, N, DIR, false><<<(unsigned)(N * batch), Block<T, N, false>::TH, 0, st>>>(d, tw);
-            CT2_LAUNCH_CHECK();
-            return CT2_OK;
-        }
+        fft_block<T, N, DIR, false><<<(unsigned)(N * batch), Block<T, N, false>::TH, 0, st>>>(d, tw);
+        CT2_LAUNCH_CHECK();
+    } else {
+        using CF = Cfg<T, N>;
+        constexpr int inner = N / CF::COLS;
+        fft_rows<T, N, DIR><<<dim3((unsigned)(N * N / CF::ROWS), batch), row_lanes<T, N>(), 0, st>>>(d, tw);
+        CT2_LAUNCH_CHECK();
+        // y: columns z, slabs x
+        fft_cols<T, N, DIR><<<dim3((unsigned)(N * inner), batch), col_lanes<T, N>(), 0, st>>>(d, tw, N, (long)N * N,
+                                                                                              inner, false);
+        CT2_LAUNCH_CHECK();
     }
-    using CF = Cfg<T, N>;
-    constexpr int inner = N / CF::COLS;
-    const dim3 rows((unsigned)(N * N / CF::ROWS), batch);
-    if (wsrc)
-        fft_rows<T, N, DIR, true><<<rows, row_lanes<T, N>(), 0, st>>>(d, tw, wsrc);
-    else
-        fft_rows<T, N, DIR><<<rows, row_lanes<T, N>(), 0, st>>>(d, tw);
-    CT2_LAUNCH_CHECK();
-    // y: columns z, slabs x
-    fft_cols<T, N, DIR><<<dim3((unsigned)(N * inner), batch), col_lanes<T, N>(), 0, st>>>(d, tw, N, (long)N * N, inner,
-                                                                                          false);
-    CT2_LAUNCH_CHECK();
     return CT2_OK;
 }
 
+// batch cubes of N^3 one after the other
 template <typename T, int N, int DIR>
-int fft3d_launch(typename V2<T>::t* d, hipStream_t st, int batch, const unsigned long long* wsrc = nullptr) {
+int fft3d_launch(typename V2<T>::t* d, hipStream_t st, int batch) {
     const typename V2<T>::t* tw = nullptr;
     CT2_TRY(twiddle_table<T>(N, &tw));
     if constexpr (N <= 16) {
-        if (!wsrc) {
-            fft_block<T, N, DIR, true><<<(unsigned)batch, Block<T, N, true>::TH, 0, st>>>(d, tw);
-            CT2_LAUNCH_CHECK();
-            return CT2_OK;
-        }
+        fft_block<T, N, DIR, true><<<(unsigned)batch, Block<T, N, true>::TH, 0, st>>>(d, tw);
+        CT2_LAUNCH_CHECK();
+    } else {
+        CT2_TRY((fft_zy<T, N, DIR>(d, tw, st, batch)));
+        // x: columns z, slabs y
+        constexpr int inner = N / Cfg<T, N>::COLS;
+        fft_cols<T, N, DIR><<<dim3((unsigned)(N * inner), batch), col_lanes<T, N>(), 0, st>>>(d, tw, (long)N * N, N,
+                                                                                              inner, true);
+        CT2_LAUNCH_CHECK();
     }
-    CT2_TRY((fft_zy<T, N, DIR>(d, tw, st, batch, wsrc)));
-    // x: columns z, slabs y
-    constexpr int inner = N / Cfg<T, N>::COLS;
-    fft_cols<T, N, DIR><<<dim3((unsigned)(N * inner), batch), col_lanes<T, N>(), 0, st>>>(d, tw, (long)N * N, N, inner,
-                                                                                          true);
-    CT2_LAUNCH_CHECK();
     return CT2_OK;
 }
 
@@ -405,16 +400,36 @@ int irfft3d_launch(const double* planar, double* out, double2* half, hipStream_t
 
 }  // namespace
 
-// Forward FP32 transform of the real field W * 2^-32 (uint64 fixed point, n^3)
-// into the complex grid out: the density transform of the PM force.
-int fft3d_density(const unsigned long long* W, void* out, int n) {
+int fft_table_f32(int n, const float2** tw) { return twiddle_table<float>(n, tw); }
+
+// The density W * 2^-32 (uint64 fixed point, n^3) through the z and y passes
+// into its half spectrum (fft_half_elems(n) elements); the x pass is the
+// caller's.
+int rfft_zy_density(const unsigned long long* W, float2* half, int n) {
     CT2_TRY(require_init());
-    if (!W || !out) return set_error(CT2_ERR_INVALID, "null FFT buffer");
+    if (!W || !half) return set_error(CT2_ERR_INVALID, "null FFT buffer");
     hipStream_t st = ctx().stream;
-    float2* d = (float2*)out;
+    const float2* tw = nullptr;
     switch (n) {
 #define CT2_CASE(N) \
-    case N: return fft3d_launch<float, N, 1>(d, st, 1, W);
+    case N: return rfft_zy_launch<float, N>(DensityField{W}, half, st, &tw);
+        CT2_FFT_SIZES(CT2_CASE)
+        CT2_CASE(1024)
+#undef CT2_CASE
+        default: return set_error(CT2_ERR_INVALID, "unsupported FFT size %d", n);
+    }
+}
+
+// Inverse y and z passes of `batch` FP32 cubes.
+int fft_inverse_yz(float2* data, int n, int batch) {
+    CT2_TRY(require_init());
+    if (!data) return set_error(CT2_ERR_INVALID, "null FFT buffer");
+    hipStream_t st = ctx().stream;
+    const float2* tw = nullptr;
+    CT2_TRY(twiddle_table<float>(n, &tw));
+    switch (n) {
+#define CT2_CASE(N) \
+    case N: return fft_zy<float, N, -1>(data, tw, st, batch);
         CT2_FFT_SIZES(CT2_CASE)
         CT2_CASE(1024)
 #undef CT2_CASE

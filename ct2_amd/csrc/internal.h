@@ -63,10 +63,13 @@ int ensure_scratch(void** p, size_t* have, size_t bytes, const char* what);
 int fft3d(void* data, int n, int dir, bool f64);
 // `batch` such cubes stored one after the other, in one set of launches.
 int fft3d_batch(void* data, int n, int dir, bool f64, int batch);
-int fft3d_density(const unsigned long long* W, void* out, int n);
 // Complex elements of the half spectrum of an n^3 real field: the columns
 // kz < n/2, then kz = n/2.
 constexpr size_t fft_half_elems(size_t n) { return n * n * (n / 2 + 1); }
+int rfft_zy_density(const unsigned long long* W, float2* half, int n);
+int fft_inverse_yz(float2* data, int n, int batch);
+// The FP32 table of n roots of unity, e^{-2 pi i m / n}.
+int fft_table_f32(int n, const float2** tw);
 int rfft3d_f64(const double* in, double* planar, double2* half, int n);
 int irfft3d_f64(const double* planar, double* out, double2* half, int n);
 

@@ -9,12 +9,14 @@
 //                 tile, each tile summed in LDS, then one global atomic per
 //                 touched node (dep_*); smaller grids: one global atomic per
 //                 particle and stencil node (mesh_deposit)
-//   fft3d_density forward FP32 transform of the density (fft.hip; its first
-//                 pass reads the uint64 grid directly)
-//   green_mul     rho_hat * G (FP64 Green's table, octant-symmetric), then
-//                 the spectral gradient; two real fields share one complex
-//                 grid: A = Fx + i Fy, B = Fz + i pot
-//   fft3d x2      inverse transforms (two instead of four)
+//   rfft_zy_density  z and y passes of the density's FP32 transform to its
+//                 half spectrum (fft.hip; the first reads the uint64 grid
+//                 directly)
+//   pm_xpass      the x pass, rho_hat * G (FP64 Green's table, octant-
+//                 symmetric), the spectral gradient, and the inverse x passes;
+//                 two real fields share one complex grid: A = Fx + i Fy,
+//                 B = Fz + i pot
+//   fft_inverse_yz  the inverse y and z passes of A and B
 //   interp        force and potential at the particles (same weights): in
 //                 deposit-tile order from LDS-staged half tiles (interp_tile)
 //                 when tiles hold enough particles, else per particle
@@ -24,6 +26,7 @@
 #include <vector>
 
 #include "epilogue.h"
+#include "fft_stages.h"
 #include "internal.h"
 #include "wave.h"
 
@@ -39,7 +42,8 @@ struct PmState {
     int order_table = 0;              // assignment order the table was built for
     float gm_table = 0.0f;  // GM the table was built for
     unsigned long long* W = nullptr;  // density, 2^-32 particle units
-    float2* A = nullptr;              // rho_hat -> Fx + i Fy
+    float2* half = nullptr;           // the density's half spectrum
+    float2* A = nullptr;              // Fx + i Fy, and right after it
     float2* B = nullptr;              // Fz + i pot
     double* G = nullptr;              // Green's table on the octant, (ng/2+1)^3
     // tiled deposit: particles binned by tile of 16 x 16 x 32 nodes
@@ -236,25 +240,119 @@ __global__ __launch_bounds__(DEP_THREADS) void dep_tile(const uint32_t* __restri
     }
 }
 
-// One thread per k-cell.  phi_hat = G rho_hat (FP64); F_hat = -i k phi_hat
-// with the Nyquist component of k zeroed; pot_hat = -phi_hat.
-__global__ __launch_bounds__(PM_BLOCK) void green_mul(float2* __restrict__ A, float2* __restrict__ B,
-                                                      const double* __restrict__ G, int g) {
-    const long c = (long)blockIdx.x * PM_BLOCK + threadIdx.x;
-    const int ng = 1 << g, h = ng / 2 + 1;
-    if (c >= (long)ng * ng * ng) return;
-    const int l = (int)(c & (ng - 1)), j = (int)((c >> g) & (ng - 1)), i = (int)(c >> (2 * g));
-    const int mi = i < ng / 2 ? i : i - ng, mj = j < ng / 2 ? j : j - ng, ml = l < ng / 2 ? l : l - ng;
-    const double gv = G[((size_t)abs(mi) * h + abs(mj)) * h + abs(ml)];
-    const float2 r = A[c];
-    const double pr = gv * (double)r.x, pi = gv * (double)r.y;
-    const double twopi = 6.283185307179586476925;
-    const double kx = i == ng / 2 ? 0.0 : twopi * mi;
-    const double ky = j == ng / 2 ? 0.0 : twopi * mj;
-    const double kz = l == ng / 2 ? 0.0 : twopi * ml;
-    // A = F_hat_x + i F_hat_y ; B = F_hat_z + i pot_hat
-    A[c] = make_float2((float)(kx * pi + ky * pr), (float)(-kx * pr + ky * pi));
-    B[c] = make_float2((float)((kz + 1.0) * pi), (float)(-(kz + 1.0) * pr));
+// The x pass of the force transforms, forward and inverse in one kernel.  A
+// workgroup takes COLS columns (ky, kz <= N/2) of the half spectrum (after its
+// z and y passes), transforms them along x, keeps phi_hat = G rho_hat (FP64) in
+// registers (a lane's outputs of a transform are its inputs of the next), and
+// from it transforms back the columns of
+//   A = F_hat_x + i F_hat_y,  B = F_hat_z + i pot_hat,
+// F_hat = -i k phi_hat with the Nyquist components of k zeroed, pot_hat =
+// -phi_hat, at (ky, kz) and, for 0 < kz < N/2, at (-ky, -kz), where rho_hat is
+// the conjugate; there element i holds -kx, so the forward sign inverts it.
+// Bound by HBM: 4 B of half spectrum and 4 of table in, 16 out per cell: 109 us
+// on a 256^3 grid, 3.7 TB/s.  The forward x pass of the whole spectrum, the
+// product and the two inverse x passes as kernels of their own moved 72 B per
+// cell in 205 us; with the half-spectrum z and y passes before it the
+// transforms of one force on 256^3 went from 453 to 327 us, on 64^3 from 36 to
+// 22 us (ten launches to four).
+template <int N>
+__global__ __launch_bounds__((Cfg<float, N, N / 2>::P * Cfg<float, N, N / 2>::COLS)) void pm_xpass(
+    const float2* __restrict__ half, float2* __restrict__ A, const double* __restrict__ G,
+    const float2* __restrict__ twg) {
+    constexpr int H = N / 2;
+    using CF = Cfg<float, N, H>;
+    constexpr int COLS = CF::COLS;
+    constexpr unsigned MAIN = (unsigned)N * (H / COLS);
+    constexpr double twopi = 6.283185307179586476925;
+    __shared__ float2 sm[N * COLS];
+    __shared__ float2 tw[N];
+    load_twiddles<N>(tw, twg, CF::P * COLS);
+    const int c = threadIdx.x % COLS, p = threadIdx.x / COLS;
+    int ky, kz;
+    const float2* d;
+    long stride;
+    if (blockIdx.x < MAIN) {
+        const unsigned b = xcd_contiguous(blockIdx.x, MAIN);
+        ky = b / (H / COLS);
+        kz = b % (H / COLS) * COLS + c;
+        d = half + (long)ky * H + kz;
+        stride = (long)N * H;
+    } else {  // kz = N/2: nyq[ky][x]
+        ky = (blockIdx.x - MAIN) * COLS + c;
+        kz = H;
+        d = half + (long)N * N * H + (long)ky * N;
+        stride = 1;
+    }
+    const int my = ky < H ? ky : ky - N;
+    auto ix = [&](int i) { return i * COLS + c; };
+    auto wave_x = [](int i) { return i == H ? 0.0 : twopi * (i < H ? i : i - N); };
+    const double wy = ky == H ? 0.0 : twopi * my, wz = kz == H ? 0.0 : twopi * kz;
+    double2 phi[CF::RM];
+    const double* Gc = G + (long)abs(my) * (H + 1) + kz;
+    run_stages<float, N, 1, false, false>(
+        [&](int i, int) { return d[(long)i * stride]; },
+        [&](int i, int m, float2 v) {
+            const double g = Gc[(long)(i < H ? i : N - i) * (H + 1) * (H + 1)];
+            phi[m] = double2{g * (double)v.x, g * (double)v.y};
+        },
+        ix, sm, tw, p);
+    constexpr long N2 = (long)N * N, N3 = N2 * N;
+    float2* out = A + (long)ky * N + kz;
+    __syncthreads();
+    run_stages<float, N, -1, false, false>(
+        [&](int i, int m) {
+            const double kx = wave_x(i);
+            return float2{(float)(kx * phi[m].y + wy * phi[m].x), (float)(-kx * phi[m].x + wy * phi[m].y)};
+        },
+        [&](int i, int, float2 v) { out[i * N2] = v; }, ix, sm, tw, p);
+    __syncthreads();
+    run_stages<float, N, -1, false, false>(
+        [&](int, int m) { return float2{(float)((wz + 1.0) * phi[m].y), (float)(-(wz + 1.0) * phi[m].x)}; },
+        [&](int i, int, float2 v) { out[N3 + i * N2] = v; }, ix, sm, tw, p);
+    if (blockIdx.x >= MAIN) return;  // uniform: the kz = N/2 plane is its own mirror
+    const bool mirror = kz > 0;      // and so is kz = 0
+    out = A + (long)((N - ky) % N) * N + (N - kz);
+    __syncthreads();
+    run_stages<float, N, 1, false, false>(
+        [&](int i, int m) {
+            const double kx = wave_x(i);
+            return float2{(float)(kx * phi[m].y - wy * phi[m].x), (float)(kx * phi[m].x + wy * phi[m].y)};
+        },
+        [&](int i, int, float2 v) {
+            if (mirror) out[i * N2] = v;
+        },
+        ix, sm, tw, p);
+    __syncthreads();
+    run_stages<float, N, 1, false, false>(
+        [&](int, int m) { return float2{(float)((wz - 1.0) * phi[m].y), (float)((wz - 1.0) * phi[m].x)}; },
+        [&](int i, int, float2 v) {
+            if (mirror) out[N3 + i * N2] = v;
+        },
+        ix, sm, tw, p);
+}
+
+template <int N>
+int xpass_launch(const float2* half, float2* A, const double* G, hipStream_t st) {
+    using CF = Cfg<float, N, N / 2>;
+    const float2* tw = nullptr;
+    CT2_TRY(fft_table_f32(N, &tw));
+    pm_xpass<N><<<N * (N / 2) / CF::COLS + N / CF::COLS, CF::P * CF::COLS, 0, st>>>(half, A, G, tw);
+    CT2_LAUNCH_CHECK();
+    return CT2_OK;
+}
+
+int xpass(int n, const float2* half, float2* A, const double* G, hipStream_t st) {
+    switch (n) {
+        case 8: return xpass_launch<8>(half, A, G, st);
+        case 16: return xpass_launch<16>(half, A, G, st);
+        case 32: return xpass_launch<32>(half, A, G, st);
+        case 64: return xpass_launch<64>(half, A, G, st);
+        case 128: return xpass_launch<128>(half, A, G, st);
+        case 256: return xpass_launch<256>(half, A, G, st);
+        case 512: return xpass_launch<512>(half, A, G, st);
+        case 1024: return xpass_launch<1024>(half, A, G, st);
+        default: return set_error(CT2_ERR_INVALID, "unsupported PM grid %d", n);
+    }
 }
 
 template <int ORDER>
@@ -378,8 +476,8 @@ __global__ __launch_bounds__(DEP_THREADS) void interp_tile(const uint32_t* __res
 
 void free_pm() {
     dev_free(g_pm.W);
+    dev_free(g_pm.half);
     dev_free(g_pm.A);
-    dev_free(g_pm.B);
     dev_free(g_pm.G);
     dev_free(g_pm.tcount);
     dev_free(g_pm.tstart);
@@ -482,14 +580,11 @@ int pm_forces() {
     CT2_TRY(ensure_table());
     Context& c = ctx();
     const int n = (int)c.n, g = g_pm.g;
-    const long n3 = 1L << (3 * g);
-    const unsigned gb = (unsigned)((n3 + PM_BLOCK - 1) / PM_BLOCK), pb = (unsigned)((n + PM_BLOCK - 1) / PM_BLOCK);
+    const unsigned pb = (unsigned)((n + PM_BLOCK - 1) / PM_BLOCK);
     CT2_TRY(g_assign == 1 ? deposit<1>(c) : deposit<2>(c));
-    CT2_TRY(fft3d_density(g_pm.W, g_pm.A, g_pm.ng));  // density (real) -> rho_hat
-    green_mul<<<gb, PM_BLOCK, 0, c.stream>>>(g_pm.A, g_pm.B, g_pm.G, g);
-    CT2_LAUNCH_CHECK();
-    CT2_TRY(fft3d(g_pm.A, g_pm.ng, -1, false));
-    CT2_TRY(fft3d(g_pm.B, g_pm.ng, -1, false));
+    CT2_TRY(rfft_zy_density(g_pm.W, g_pm.half, g_pm.ng));
+    CT2_TRY(xpass(g_pm.ng, g_pm.half, g_pm.A, g_pm.G, c.stream));
+    CT2_TRY(fft_inverse_yz(g_pm.A, g_pm.ng, 2));
     // tiles hold n / ntile particles on average: stage a tile's nodes once when
     // that beats one L2 read per particle and stencil node.  Measured: faster
     // on 256^3 grids (0.19 -> 0.16 ms, TSC, 2^21 particles), slower on 512^3
@@ -545,12 +640,13 @@ extern "C" int ct2_pm_init(int ng, double rs_cells) {
     const size_t n3 = (size_t)ng * ng * ng, h = ng / 2 + 1;
     int rc;
     if ((rc = dev_alloc((void**)&g_pm.W, n3 * sizeof(unsigned long long), "PM density")) ||
-        (rc = dev_alloc((void**)&g_pm.A, n3 * sizeof(float2), "PM grid A")) ||
-        (rc = dev_alloc((void**)&g_pm.B, n3 * sizeof(float2), "PM grid B")) ||
+        (rc = dev_alloc((void**)&g_pm.half, fft_half_elems(ng) * sizeof(float2), "PM half spectrum")) ||
+        (rc = dev_alloc((void**)&g_pm.A, 2 * n3 * sizeof(float2), "PM grids")) ||
         (rc = dev_alloc((void**)&g_pm.G, h * h * h * sizeof(double), "PM Green's table"))) {
         free_pm();
         return rc;
     }
+    g_pm.B = g_pm.A + n3;
     g_pm.ng = ng;
     g_pm.g = ilog2(ng);
     if (g_pm.g >= TILE_MIN_G) {

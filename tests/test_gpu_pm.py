@@ -49,6 +49,38 @@ def test_pm_forces_vs_fp64_oracle(ct2, orc, ng, rs):
     assert np.max(np.abs(pot - op)) < 1e-5 * np.abs(op).max()
 
 
+@pytest.mark.parametrize("ng", [8, 16, 32, 64, 128, 256, 512])
+def test_pm_fields_of_the_density_at_every_grid_size(ct2, ng):
+    """The force and potential grids against FP64 transforms of the same
+    density: every size of the half-spectrum passes and of the fused x pass
+    (its kz = 0 and N/2 columns and its mirrored half).  An FP32 transform
+    stays within 1e-6 of the complex grid it transforms (relative L2), forward
+    and inverse within 2e-6: Fx + i Fy and Fz + i pot are one grid each."""
+    rng = np.random.default_rng(ng)
+    n, rs = 4000, 1.0
+    x, y, z = (rng.integers(0, TWO32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
+    load(ct2, x, y, z)
+    gm = f32(1.0 / n)
+    ct2.set_force_options(1e-3, gm, 0)
+    ct2.pm_init(ng, rs)
+    ct2.pm_forces()
+    hat = np.fft.rfftn(ct2.pm_density_download().astype(np.float64) * 2.0 ** -32)
+    m = np.fft.fftfreq(ng, 1.0 / ng)
+    k = [2 * np.pi * v for v in np.meshgrid(m, m, np.abs(m[:ng // 2 + 1]), indexing="ij", sparse=True)]
+    k2 = sum(v * v for v in k)
+    k2[0, 0, 0] = 1.0
+    w = 1.0
+    for v in k:
+        w = w * np.sinc(v / (2 * np.pi * ng)) ** 4
+    phi = -4 * np.pi * gm * np.exp(-k2 * (rs / ng) ** 2) / (k2 * w) * hat
+    phi[0, 0, 0] = 0.0
+    k = [np.where(np.abs(v) > np.pi * ng - 1.0, 0.0, v) for v in k]  # no force from the Nyquist components
+    for which, pair in ((0, (-1j * k[0] * phi, -1j * k[1] * phi)), (1, (-1j * k[2] * phi, -phi))):
+        re, im = (np.fft.irfftn(f, s=(ng,) * 3, axes=(0, 1, 2)) * float(ng) ** 3 for f in pair)
+        want = (re + 1j * im).ravel()
+        assert np.linalg.norm(ct2.pm_grid_download(which).ravel() - want) < 2e-6 * np.linalg.norm(want)
+
+
 def test_pm_matches_periodic_judge_on_a_single_mode(ct2):
     """Linear single-mode lattice: PM long-range force 4 pi psi exp(-k^2 rs^2),
     the periodic FP64 judge the full 4 pi psi."""
