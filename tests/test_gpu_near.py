@@ -88,6 +88,30 @@ def test_near_field_vs_fp64_oracle(ct2, orc, name, kind, ng, rs_cells, rcut_rs, 
     assert np.median(ep) < 1e-5 and ep.max() < 1e-3, (np.median(ep), ep.max())
 
 
+@pytest.mark.parametrize("kernel", [0, 1])
+@pytest.mark.parametrize("n", [2, 15, 17, 65, 2000, 2001])
+def test_near_field_work_items(ct2, orc, n, kernel):
+    """Work items of fewer than 16 sinks, rows of one sink more than whole
+    items, and both sides of the density (16 per cell, 5^3 cells) above which
+    cells are split in x and y; the tolerance of the cases above."""
+    rng = np.random.default_rng(n)
+    x, y, z = (rng.integers(0, TWO32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
+    x[: n // 2] = (x[: n // 2] >> 6) + np.uint32(2 ** 31)  # half of them within a few columns
+    y[: n // 2] = (y[: n // 2] >> 6) + np.uint32(2 ** 31)
+    load(ct2, x, y, z)
+    gm, soft, ng, rs, rcut_rs = f32(1.0 / n), f32(2e-3), 64, 2.0, 6.0
+    ct2.set_force_options(soft, gm, kernel)
+    ct2.pm_init(ng, rs)
+    tot, near = near_only(ct2, rcut_rs)
+    assert ct2.pm_near_cells() == 5
+    want = np.stack(orc.pm_near(x, y, z, gm, soft, rs / ng, rcut_rs * rs / ng, kernel))
+    scale = np.linalg.norm(tot[:3], axis=0) + np.linalg.norm(want[:3], axis=0)
+    e = np.linalg.norm(near[:3] - want[:3], axis=0) / scale
+    assert np.median(e) < 1e-5 and e.max() < 2e-3, (np.median(e), e.max())
+    ep = np.abs(near[3] - want[3]) / (np.abs(tot[3]) + np.abs(want[3]))  # the total passes through zero
+    assert np.median(ep) < 1e-5 and ep.max() < 1e-3, (np.median(ep), ep.max())
+
+
 def test_near_field_is_deterministic(ct2):
     x, y, z = ct2.ic_plummer_mix(30000, 20000, 3, 0.01, 0.1, 9)
     load(ct2, x, y, z)
