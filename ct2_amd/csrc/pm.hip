@@ -5,10 +5,10 @@
 // kick.cpp:29) with cloud-in-cell mass assignment, keeping its pipeline:
 //   deposit       fixed-point CIC (default) or TSC weights, uint64 atomics:
 //                 deterministic, bit-identical to the CPU oracle.  Grids of 32
-//                 nodes a side or more: particles binned by 16 x 16 x 32-node
-//                 tile, each tile summed in LDS, then one global atomic per
-//                 touched node (dep_*); smaller grids: one global atomic per
-//                 particle and stencil node (mesh_deposit)
+//                 nodes a side or more: particles binned by 16^3-node tile
+//                 (bin_*), each tile summed in LDS and stored (dep_tile);
+//                 smaller grids: one global atomic per particle and stencil
+//                 node (mesh_deposit)
 //   rfft_zy_density  z and y passes of the density's FP32 transform to its
 //                 half spectrum (fft.hip; the first reads the uint64 grid
 //                 directly)
@@ -18,10 +18,11 @@
 //                 B = Fz + i pot
 //   fft_inverse_yz  the inverse y and z passes of A and B
 //   interp        force and potential at the particles (same weights): in
-//                 deposit-tile order from LDS-staged half tiles (interp_tile)
+//                 deposit-tile order from LDS-staged tiles (interp_tile)
 //                 when tiles hold enough particles, else per particle
 //                 (mesh_interp)
 // Grid layout: (i*ng + j)*ng + k with i along x; node c at position c/ng.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -46,13 +47,13 @@ struct PmState {
     float2* A = nullptr;              // Fx + i Fy, and right after it
     float2* B = nullptr;              // Fz + i pot
     double* G = nullptr;              // Green's table on the octant, (ng/2+1)^3
-    // tiled deposit: particles binned by tile of 16 x 16 x 32 nodes
+    // tiled deposit: particles binned by tile of 16^3 nodes
     int ntile = 0;
     int* tcount = nullptr;  // [ntile]
     int* tstart = nullptr;  // [ntile + 1]
-    size_t cap = 0;         // particles slot / order hold
-    int* slot = nullptr;    // [cap] position within the tile
-    int* order = nullptr;   // [cap] particle indices grouped by tile
+    int* bins = nullptr;    // [BIN_WGS][ntile] counts per binning workgroup
+    size_t cap = 0;         // particles order has room for
+    int* order = nullptr;   // [cap MAX_COPIES] particle indices grouped by tile
 } g_pm;
 int g_assign = 1;  // mass assignment: 1 CIC, 2 TSC (kept across ct2_pm_init)
 
@@ -61,22 +62,23 @@ int g_assign = 1;  // mass assignment: 1 CIC, 2 TSC (kept across ct2_pm_init)
 //   ORDER 2 (TSC): nearest node c = (x + 2^(s-1)) >> s, signed offset D in
 //     [-2^20, 2^20) (2^-21 cells); nodes c-1, c, c+1 get round((2^20-D)^2/2^22),
 //     the rest, round((2^20+D)^2/2^22): the quadratic spline (1/2)(1/2 -+ d)^2.
+// Everything but the squares fits in 32 bits.
 template <int ORDER>
-__device__ __forceinline__ void assign_axis(uint32_t x, int s, uint32_t& lo, uint64_t (&w)[ORDER + 1]) {
+__device__ __forceinline__ void assign_axis(uint32_t x, int s, uint32_t& lo, uint32_t (&w)[ORDER + 1]) {
     if constexpr (ORDER == 1) {
         lo = x >> s;
         const uint32_t t = x & ((1u << s) - 1u);
-        w[1] = (uint64_t)(t >> (s - CIC_BITS));
-        w[0] = (1ull << CIC_BITS) - w[1];
+        w[1] = t >> (s - CIC_BITS);
+        w[0] = (1u << CIC_BITS) - w[1];
     } else {
         const uint32_t half = 1u << (s - 1);
         const uint32_t xs = x + half;
         const int32_t d = (int32_t)(xs & ((1u << s) - 1u)) - (int32_t)half;
-        const int64_t D = (int64_t)(d >> (s - CIC_BITS));
-        const uint64_t a = (uint64_t)((1 << 20) - D), b = (uint64_t)((1 << 20) + D);
-        w[0] = (a * a + (1ull << 21)) >> 22;
-        w[2] = (b * b + (1ull << 21)) >> 22;
-        w[1] = (1ull << CIC_BITS) - w[0] - w[2];
+        const int32_t D = d >> (s - CIC_BITS);
+        const uint32_t a = (uint32_t)((1 << 20) - D), b = (uint32_t)((1 << 20) + D);
+        w[0] = (uint32_t)(((uint64_t)a * a + (1ull << 21)) >> 22);
+        w[2] = (uint32_t)(((uint64_t)b * b + (1ull << 21)) >> 22);
+        w[1] = (1u << CIC_BITS) - w[0] - w[2];
         lo = (xs >> s) - 1u;
     }
 }
@@ -95,7 +97,7 @@ __global__ __launch_bounds__(PM_BLOCK) void mesh_deposit(const uint32_t* __restr
     const int s = 32 - g;
     const uint32_t ng = 1u << g, mask = ng - 1;
     uint32_t i0, j0, k0;
-    uint64_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
+    uint32_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
     assign_axis<ORDER>(X[p], s, i0, ax);
     assign_axis<ORDER>(Y[p], s, j0, ay);
     assign_axis<ORDER>(Z[p], s, k0, az);
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(PM_BLOCK) void mesh_deposit(const uint32_t* __restr
     for (int dx = 0; dx <= ORDER; ++dx)
 #pragma unroll
         for (int dy = 0; dy <= ORDER; ++dy) {
-            const uint64_t axy = ax[dx] * ay[dy];
+            const uint64_t axy = (uint64_t)ax[dx] * ay[dy];
             const size_t row = ((size_t)((i0 + dx) & mask) * ng + ((j0 + dy) & mask)) * ng;
 #pragma unroll
             for (int dz = 0; dz <= ORDER; ++dz)
@@ -112,131 +114,234 @@ __global__ __launch_bounds__(PM_BLOCK) void mesh_deposit(const uint32_t* __restr
 }
 
 // Tiled deposit for grids of 32 nodes and more a side.  The grid is cut into
-// tiles of 16 x 16 x 32 nodes; a particle belongs to the tile of its anchor
-// node (CIC: its first node; TSC: its nearest node), so its stencil lies in the
-// tile grown by one node on every side.  Particles are binned by tile
-// (dep_count, tile_scan, dep_scatter); one workgroup per tile then adds its
-// particles' weights into an LDS copy of the grown tile (uint64 LDS atomics)
-// and adds each nonzero LDS node into the grid with one global atomic.  The
-// weights are those of mesh_deposit and integer sums do not depend on order,
-// so the grid is bit-identical to mesh_deposit's.
-constexpr int TILE_BX = 4, TILE_BY = 4, TILE_BZ = 5;  // log2 tile size per axis
-constexpr int TLX = (1 << TILE_BX) + 2, TLY = (1 << TILE_BY) + 2, TLZ = (1 << TILE_BZ) + 2;
-constexpr int TL_NODES = TLX * TLY * TLZ;  // 11,016 nodes: 88,128 B of LDS
-constexpr int DEP_THREADS = 1024;
-constexpr int TILE_MIN_G = TILE_BZ;  // grids of at least 2^5 nodes a side
+// tiles of 16^3 nodes; a particle's home is the tile of its anchor node (CIC:
+// its first node; TSC: its nearest node), and where its stencil reaches over a
+// face of that tile it is listed in the neighbours there too (1.4 entries per
+// particle with TSC, 1.2 with CIC).  One workgroup per tile (dep_tile) adds the
+// weights that fall on the tile's own nodes in LDS (uint64 LDS atomics) and
+// stores them, each node once.  No global atomics: on this chip they leave the
+// XCD's L2.  Adding the LDS copies of grown tiles into a cleared grid with them
+// took 186 us for 2^21 particles on 256^3 (TSC), and a binning that counted with
+// them 54; tiles and binning take 43 and 48 this way.  Setting the nodes around
+// each tile aside for a second pass over the faces, instead of listing particles
+// twice: 127 and 46 (the z faces touch every line of the grid again).  The
+// weights are those of mesh_deposit and integer sums do not depend on order, so
+// the grid is bit-identical to mesh_deposit's.
+constexpr int TILE_B = 4;  // log2 of the tile's side
+constexpr int TS = 1 << TILE_B;
+constexpr int TROW = TS + 1;                 // padded LDS row
+constexpr int TL = TS + 2;                   // side of the grown tile
+constexpr int TL_NODES = TL * TL * TL;
+constexpr int TILE_THREADS = 512;
+constexpr int TILE_MIN_G = TILE_B + 1;  // grids of at least 2^5 nodes a side
+constexpr int BIN_THREADS = 1024;
+constexpr int BIN_WGS = 128;            // binning workgroups at most
+constexpr int BIN_TILES = 32768;        // tiles whose counters fit in LDS (512^3 grids)
+constexpr int MAX_COPIES = 8;           // tiles a stencil can touch
 
 template <int ORDER>
 __device__ __forceinline__ uint32_t anchor_node(uint32_t x, int s) {
     return ORDER == 1 ? x >> s : (uint32_t)(x + (1u << (s - 1))) >> s;
 }
 
-template <int ORDER>
-__device__ __forceinline__ int tile_of(uint32_t x, uint32_t y, uint32_t z, int g) {
-    const int s = 32 - g;
-    const int tx = (int)(anchor_node<ORDER>(x, s) >> TILE_BX);
-    const int ty = (int)(anchor_node<ORDER>(y, s) >> TILE_BY);
-    const int tz = (int)(anchor_node<ORDER>(z, s) >> TILE_BZ);
-    return (tx << (2 * g - TILE_BY - TILE_BZ)) + (ty << (g - TILE_BZ)) + tz;
+// f(tile, home) for every tile the particle's stencil touches, its home first.
+template <int ORDER, typename F>
+__device__ __forceinline__ void for_tiles(uint32_t x, uint32_t y, uint32_t z, int g, const F& f) {
+    const int s = 32 - g, gt = g - TILE_B, m = (1 << gt) - 1;
+    int t[3][2];
+    bool two[3];
+    const uint32_t v[3] = {x, y, z};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int n = (int)anchor_node<ORDER>(v[a], s), o = n & (TS - 1);
+        const bool up = o == TS - 1, down = ORDER == 2 && o == 0;
+        t[a][0] = n >> TILE_B;
+        t[a][1] = (t[a][0] + (up ? 1 : m)) & m;
+        two[a] = up || down;
+    }
+    f((((t[0][0] << gt) + t[1][0]) << gt) + t[2][0], true);
+    if (!(two[0] || two[1] || two[2])) return;
+#pragma unroll
+    for (int d = 1; d < 8; ++d) {
+        const bool ux = d & 1, uy = d & 2, uz = d & 4;
+        if ((ux && !two[0]) || (uy && !two[1]) || (uz && !two[2])) continue;
+        f((((t[0][ux] << gt) + t[1][uy]) << gt) + t[2][uz], false);
+    }
 }
 
+// The first node of a tile along each axis.
+__device__ __forceinline__ void tile_origin(int tile, int g, uint32_t& ox, uint32_t& oy, uint32_t& oz) {
+    const int gt = g - TILE_B, m = (1 << gt) - 1;
+    ox = (uint32_t)(tile >> (2 * gt)) << TILE_B;
+    oy = (uint32_t)((tile >> gt) & m) << TILE_B;
+    oz = (uint32_t)(tile & m) << TILE_B;
+}
+
+// Binning, first half: the entries of workgroup w's particles [w per,
+// (w + 1) per) counted by tile in LDS, cnt[w][tile].
+template <int ORDER, int TILES>
+__global__ __launch_bounds__(BIN_THREADS) void bin_count(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
+                                                        const uint32_t* __restrict__ Z, int n, int per, int g, int nt,
+                                                        int* __restrict__ cnt) {
+    __shared__ int h[TILES];
+    for (int t = threadIdx.x; t < nt; t += BIN_THREADS) h[t] = 0;
+    __syncthreads();
+    const int p1 = (int)min((long)n, (long)(blockIdx.x + 1) * per);
+    for (int p = blockIdx.x * per + threadIdx.x; p < p1; p += BIN_THREADS)
+        for_tiles<ORDER>(X[p], Y[p], Z[p], g, [&](int t, bool) { atomicAdd(&h[t], 1); });
+    __syncthreads();
+    for (int t = threadIdx.x; t < nt; t += BIN_THREADS) cnt[(size_t)blockIdx.x * nt + t] = h[t];
+}
+
+// cnt[w][tile] -> the tile's entries from the workgroups before w, and the
+// tile's total.
+__global__ __launch_bounds__(PM_BLOCK) void bin_prefix(int* __restrict__ cnt, int nw, int nt, int* __restrict__ total) {
+    const int t = blockIdx.x * PM_BLOCK + threadIdx.x;
+    if (t >= nt) return;
+    int run = 0;
+    constexpr int AHEAD = 16;  // counts read together: the stores would otherwise hold back the next loads
+    for (int w0 = 0; w0 < nw; w0 += AHEAD) {
+        int v[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) v[u] = w0 + u < nw ? cnt[(size_t)(w0 + u) * nt + t] : 0;
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            if (w0 + u < nw) cnt[(size_t)(w0 + u) * nt + t] = run;
+            run += v[u];
+        }
+    }
+    total[t] = run;
+}
+
+// Exclusive scan of nt values by one workgroup of BIN_THREADS: out(t, prefix)
+// for every t, in thread-contiguous pieces; returns the total.
+template <typename IN, typename OUT>
+__device__ __forceinline__ int block_scan(int nt, const IN& in, const OUT& out) {
+    __shared__ int part[BIN_THREADS / 64];
+    const int t = threadIdx.x, lane = t & 63;
+    const int per = (nt + BIN_THREADS - 1) / BIN_THREADS;
+    const int b = min(nt, t * per), e = min(nt, b + per);
+    int sum = 0;
+    for (int i = b; i < e; ++i) sum += in(i);
+    int s = sum;  // inclusive over the wave
+    for (int off = 1; off < 64; off <<= 1) {
+        const int u = __shfl_up(s, off);
+        if (lane >= off) s += u;
+    }
+    if (lane == 63) part[t >> 6] = s;
+    __syncthreads();
+    int run = s - sum, total = 0;
+    for (int k = 0; k < BIN_THREADS / 64; ++k) {
+        if (k < t >> 6) run += part[k];
+        total += part[k];
+    }
+    for (int i = b; i < e; ++i) {
+        const int v = in(i);
+        out(i, run);
+        run += v;
+    }
+    return total;
+}
+
+// Binning, second half: every workgroup scans the tile totals (workgroup 0
+// writes them out as tstart) and places its particles' entries, grouped by
+// tile, in order.  Which of a tile's slots an entry gets depends on scheduling;
+// the set does not.
+template <int ORDER, int TILES>
+__global__ __launch_bounds__(BIN_THREADS) void bin_scatter(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
+                                                          const uint32_t* __restrict__ Z, int n, int per, int g, int nt,
+                                                          const int* __restrict__ cnt, const int* __restrict__ total,
+                                                          int* __restrict__ tstart, int* __restrict__ order) {
+    __shared__ int h[TILES];
+    const int* mine = cnt + (size_t)blockIdx.x * nt;
+    const bool first = blockIdx.x == 0;
+    const int sum = block_scan(nt, [&](int t) { return total[t]; },
+                               [&](int t, int s) {
+                                   h[t] = s + mine[t];
+                                   if (first) tstart[t] = s;
+                               });
+    if (first && threadIdx.x == 0) tstart[nt] = sum;
+    __syncthreads();
+    const int p1 = (int)min((long)n, (long)(blockIdx.x + 1) * per);
+    for (int p = blockIdx.x * per + threadIdx.x; p < p1; p += BIN_THREADS)
+        for_tiles<ORDER>(X[p], Y[p], Z[p], g, [&](int t, bool) { order[atomicAdd(&h[t], 1)] = p; });
+}
+
+// The same for grids of more tiles than LDS holds counters for, with global
+// atomics: one per run of particles of one home tile, one per further entry.
 __global__ __launch_bounds__(PM_BLOCK) void fill_i32(int* __restrict__ p, int n) {
     const int i = blockIdx.x * PM_BLOCK + threadIdx.x;
     if (i < n) p[i] = 0;
 }
 
-template <int ORDER>
-__global__ __launch_bounds__(PM_BLOCK) void dep_count(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
-                                                      const uint32_t* __restrict__ Z, int n, int g,
-                                                      int* __restrict__ tcount, int* __restrict__ slot) {
+template <int ORDER, bool PLACE>
+__global__ __launch_bounds__(PM_BLOCK) void bin_global(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
+                                                       const uint32_t* __restrict__ Z, int n, int g,
+                                                       int* __restrict__ counter, int* __restrict__ order) {
     const int p = blockIdx.x * PM_BLOCK + threadIdx.x;
-    const int t = p < n ? tile_of<ORDER>(X[p], Y[p], Z[p], g) : -1;
-    const int k = run_increment(tcount, t);  // every lane of the wave takes part
-    if (p < n) slot[p] = k;
+    int home = -1;
+    if (p < n)
+        for_tiles<ORDER>(X[p], Y[p], Z[p], g, [&](int t, bool h) {
+            if (h) {
+                home = t;
+            } else {
+                const int k = atomicAdd(counter + t, 1);
+                if (PLACE) order[k] = p;
+            }
+        });
+    const int k = run_increment(counter, home);  // every lane of the wave takes part
+    if (PLACE && p < n) order[k] = p;
 }
 
-// Exclusive scan of len counts (one workgroup): out[0..len], out[len] = total.
-__global__ __launch_bounds__(DEP_THREADS) void tile_scan(const int* __restrict__ in, int len, int* __restrict__ out) {
-    __shared__ int part[DEP_THREADS];
-    const int t = threadIdx.x;
-    const int per = (len + DEP_THREADS - 1) / DEP_THREADS;
-    const int b = min(len, t * per), e = min(len, b + per);
-    int s = 0;
-    for (int i = b; i < e; ++i) s += in[i];
-    part[t] = s;
-    __syncthreads();
-    for (int off = 1; off < DEP_THREADS; off <<= 1) {
-        const int v = t >= off ? part[t - off] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
-    }
-    int run = part[t] - s;
-    for (int i = b; i < e; ++i) {
-        out[i] = run;
-        run += in[i];
-    }
-    if (t == DEP_THREADS - 1) out[len] = part[t];
+// Exclusive scan into out[0 .. len] and, as cursors for the placement, over in.
+__global__ __launch_bounds__(BIN_THREADS) void tile_scan(int* __restrict__ in, int len, int* __restrict__ out) {
+    const int sum = block_scan(len, [&](int t) { return in[t]; }, [&](int t, int s) { out[t] = in[t] = s; });
+    if (threadIdx.x == 0) out[len] = sum;
 }
 
 template <int ORDER>
-__global__ __launch_bounds__(PM_BLOCK) void dep_scatter(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
-                                                        const uint32_t* __restrict__ Z, int n, int g,
-                                                        const int* __restrict__ tstart, const int* __restrict__ slot,
-                                                        int* __restrict__ order) {
-    const int p = blockIdx.x * PM_BLOCK + threadIdx.x;
-    if (p >= n) return;
-    order[tstart[tile_of<ORDER>(X[p], Y[p], Z[p], g)] + slot[p]] = p;
-}
-
-template <int ORDER>
-__global__ __launch_bounds__(DEP_THREADS) void dep_tile(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
+__global__ __launch_bounds__(TILE_THREADS) void dep_tile(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
                                                         const uint32_t* __restrict__ Z, const int* __restrict__ order,
                                                         const int* __restrict__ tstart, int g,
                                                         unsigned long long* __restrict__ W) {
-    __shared__ unsigned long long acc[TL_NODES];
-    const int tile = blockIdx.x;
+    __shared__ unsigned long long acc[TS * TS * TROW];
+    const int tile = (int)xcd_contiguous(blockIdx.x, gridDim.x), tid = threadIdx.x;
     const int b = tstart[tile], e = tstart[tile + 1];
-    if (b == e) return;  // uniform across the workgroup
-    const int tid = threadIdx.x;
     const int s = 32 - g;
     const uint32_t mask = (1u << g) - 1u;
-    const uint32_t ox = (uint32_t)(tile >> (2 * g - TILE_BY - TILE_BZ)) << TILE_BX;
-    const uint32_t oy = (uint32_t)((tile >> (g - TILE_BZ)) & ((1 << (g - TILE_BY)) - 1)) << TILE_BY;
-    const uint32_t oz = (uint32_t)(tile & ((1 << (g - TILE_BZ)) - 1)) << TILE_BZ;
-    for (int i = tid; i < TL_NODES; i += DEP_THREADS) acc[i] = 0ull;
+    uint32_t ox, oy, oz;
+    tile_origin(tile, g, ox, oy, oz);
+    for (int i = tid; i < TS * TS * TROW; i += TILE_THREADS) acc[i] = 0ull;
     __syncthreads();
-    // local index of the stencil's first node: anchor - origin + (CIC: 1, TSC: 0)
-    constexpr uint32_t SHIFT = ORDER == 1 ? 1u : 0u;
-    for (int k = b + tid; k < e; k += DEP_THREADS) {
+    for (int k = b + tid; k < e; k += TILE_THREADS) {
         const int p = order[k];
         const uint32_t x = X[p], y = Y[p], z = Z[p];
         uint32_t lo;
-        uint64_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
+        uint32_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
         assign_axis<ORDER>(x, s, lo, ax);
         assign_axis<ORDER>(y, s, lo, ay);
         assign_axis<ORDER>(z, s, lo, az);
-        const int lx = (int)(anchor_node<ORDER>(x, s) - ox + SHIFT);
-        const int ly = (int)(anchor_node<ORDER>(y, s) - oy + SHIFT);
-        const int lz = (int)(anchor_node<ORDER>(z, s) - oz + SHIFT);
+        // the stencil's first node from the tile's first, -2 .. TS
+        constexpr int SHIFT = ORDER == 1 ? 1 : 2;
+        const int lx = (int)((anchor_node<ORDER>(x, s) - ox + 1u) & mask) - SHIFT;
+        const int ly = (int)((anchor_node<ORDER>(y, s) - oy + 1u) & mask) - SHIFT;
+        const int lz = (int)((anchor_node<ORDER>(z, s) - oz + 1u) & mask) - SHIFT;
 #pragma unroll
         for (int dx = 0; dx <= ORDER; ++dx)
 #pragma unroll
             for (int dy = 0; dy <= ORDER; ++dy) {
-                const uint64_t axy = ax[dx] * ay[dy];
-                unsigned long long* row = acc + ((lx + dx) * TLY + (ly + dy)) * TLZ + lz;
+                if ((unsigned)(lx + dx) >= TS || (unsigned)(ly + dy) >= TS) continue;
+                const uint64_t axy = (uint64_t)ax[dx] * ay[dy];
+                unsigned long long* row = acc + ((lx + dx) * TS + (ly + dy)) * TROW + lz;
 #pragma unroll
                 for (int dz = 0; dz <= ORDER; ++dz)
-                    atomicAdd(row + dz, (unsigned long long)((axy * az[dz]) >> 31));
+                    if ((unsigned)(lz + dz) < TS) atomicAdd(row + dz, (unsigned long long)((axy * az[dz]) >> 31));
             }
     }
     __syncthreads();
-    for (int i = tid; i < TL_NODES; i += DEP_THREADS) {
-        const unsigned long long v = acc[i];
-        if (!v) continue;
-        const int lx = i / (TLY * TLZ), ly = (i / TLZ) % TLY, lz = i % TLZ;
-        const size_t gx = (ox + lx - 1u) & mask, gy = (oy + ly - 1u) & mask, gz = (oz + lz - 1u) & mask;
-        atomicAdd(W + ((((gx << g) + gy) << g) + gz), v);
+    for (int i = tid; i < TS * TS * TS; i += TILE_THREADS) {
+        const int lz = i % TS, ly = i / TS % TS, lx = i / (TS * TS);
+        W[((((size_t)(ox + lx) << g) + (oy + ly)) << g) + (oz + lz)] = acc[(lx * TS + ly) * TROW + lz];
     }
 }
 
@@ -366,7 +471,7 @@ __global__ __launch_bounds__(PM_BLOCK) void mesh_interp(const uint32_t* __restri
     const int s = 32 - g;
     const uint32_t ng = 1u << g, mask = ng - 1;
     uint32_t i0, j0, k0;
-    uint64_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
+    uint32_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
     assign_axis<ORDER>(X[p], s, i0, ax);
     assign_axis<ORDER>(Y[p], s, j0, ay);
     assign_axis<ORDER>(Z[p], s, k0, az);
@@ -395,82 +500,77 @@ __global__ __launch_bounds__(PM_BLOCK) void mesh_interp(const uint32_t* __restri
     pot[p] = acc3;
 }
 
-// Interpolation in tile order, for grids with enough particles per tile: one
-// workgroup per deposit tile (16 x 16 x 32 nodes) stages the force and
-// potential of one 16-node half of the tile along z, grown by one node on
-// every side (18^3 nodes of (Fx, Fy, Fz, pot), 93 KB), in LDS and
-// interpolates the particles whose anchor node lies in that half; then the
-// other half.  The same weights and summation order as mesh_interp, so the
-// results are identical; each node is read from L2 once per tile half instead
-// of once per particle and stencil node.
-constexpr int IH = 1 << (TILE_BZ - 1);  // z nodes per half tile
-constexpr int ILX = (1 << TILE_BX) + 2, ILY = (1 << TILE_BY) + 2, ILZ = IH + 2;
+// Interpolation in tile order, for grids with enough particles per tile: a
+// workgroup per deposit tile and grid (blockIdx.y: A = (Fx, Fy), B = (Fz, pot))
+// stages the grown tile's 18^3 nodes in LDS (47 KB, three workgroups per CU) and
+// interpolates the particles at home in it.  The same weights and summation
+// order as mesh_interp, so the results are identical.  Bound by the reads of the
+// grown tiles (rows of 144 bytes, 2.1 lines each): 130 us for 2^21 particles on
+// 256^3 with neighbouring tiles on one XCD, 165 with the tiles dealt to the XCDs
+// in turn.
 template <int ORDER>
-__global__ __launch_bounds__(DEP_THREADS) void interp_tile(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
+__global__ __launch_bounds__(TILE_THREADS) void interp_tile(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
                                                            const uint32_t* __restrict__ Z, const int* __restrict__ order,
                                                            const int* __restrict__ tstart, int g,
-                                                           const float2* __restrict__ A, const float2* __restrict__ B,
-                                                           float* __restrict__ fx, float* __restrict__ fy,
-                                                           float* __restrict__ fz, float* __restrict__ pot) {
-    __shared__ float4 nd[ILX * ILY * ILZ];
-    const int tile = blockIdx.x;
+                                                           const float2* __restrict__ A, float* __restrict__ fx,
+                                                           float* __restrict__ fy, float* __restrict__ fz,
+                                                           float* __restrict__ pot) {
+    __shared__ float2 nd[TL_NODES];
+    const int tile = (int)xcd_contiguous(blockIdx.x, gridDim.x);
     const int b = tstart[tile], e = tstart[tile + 1];
     if (b == e) return;  // uniform across the workgroup
     const int tid = threadIdx.x;
     const int s = 32 - g;
     const uint32_t mask = (1u << g) - 1u;
-    const uint32_t ox = (uint32_t)(tile >> (2 * g - TILE_BY - TILE_BZ)) << TILE_BX;
-    const uint32_t oy = (uint32_t)((tile >> (g - TILE_BZ)) & ((1 << (g - TILE_BY)) - 1)) << TILE_BY;
-    const uint32_t oz = (uint32_t)(tile & ((1 << (g - TILE_BZ)) - 1)) << TILE_BZ;
+    uint32_t ox, oy, oz;
+    tile_origin(tile, g, ox, oy, oz);
+    A += (size_t)blockIdx.y << (3 * g);
+    float* out0 = blockIdx.y ? fz : fx;
+    float* out1 = blockIdx.y ? pot : fy;
+    constexpr int LOADS = (TL_NODES + TILE_THREADS - 1) / TILE_THREADS;
+    float2 v[LOADS];  // all in flight before the first is stored
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u) {
+        const int i = min(tid + u * TILE_THREADS, TL_NODES - 1);
+        const int lx = i / (TL * TL), ly = i / TL % TL, lz = i % TL;
+        const size_t gx = (ox + lx - 1u) & mask, gy = (oy + ly - 1u) & mask, gz = (oz + lz - 1u) & mask;
+        v[u] = A[(((gx << g) + gy) << g) + gz];
+    }
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u)
+        if (tid + u * TILE_THREADS < TL_NODES) nd[tid + u * TILE_THREADS] = v[u];
+    __syncthreads();
     constexpr uint32_t SHIFT = ORDER == 1 ? 1u : 0u;
     const float q = 0x1p-21f;
-    for (int h = 0; h < 2; ++h) {
-        const uint32_t hz = oz + (uint32_t)(h * IH);
-        __syncthreads();  // the previous half's reads are done
-        for (int i = tid; i < ILX * ILY * ILZ; i += DEP_THREADS) {
-            const int lx = i / (ILY * ILZ), ly = (i / ILZ) % ILY, lz = i % ILZ;
-            const size_t gx = (ox + lx - 1u) & mask, gy = (oy + ly - 1u) & mask, gz = (hz + lz - 1u) & mask;
-            const size_t cc = (((gx << g) + gy) << g) + gz;
-            const float2 a = A[cc], bb = B[cc];
-            nd[i] = make_float4(a.x, a.y, bb.x, bb.y);
-        }
-        __syncthreads();
-        for (int k = b + tid; k < e; k += DEP_THREADS) {
-            const int p = order[k];
-            const uint32_t z = Z[p];
-            const uint32_t lzs = anchor_node<ORDER>(z, s) - hz;  // anchor z within this half: [0, IH)
-            if (lzs >= (uint32_t)IH) continue;
-            const uint32_t x = X[p], y = Y[p];
-            uint32_t lo;
-            uint64_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
-            assign_axis<ORDER>(x, s, lo, ax);
-            assign_axis<ORDER>(y, s, lo, ay);
-            assign_axis<ORDER>(z, s, lo, az);
-            const int lx = (int)(anchor_node<ORDER>(x, s) - ox + SHIFT);
-            const int ly = (int)(anchor_node<ORDER>(y, s) - oy + SHIFT);
-            const int lz = (int)(lzs + SHIFT);
-            float acc0 = 0.f, acc1 = 0.f, acc2 = 0.f, acc3 = 0.f;
+    for (int k = b + tid; k < e; k += TILE_THREADS) {
+        const int p = order[k];
+        const uint32_t x = X[p], y = Y[p], z = Z[p];
+        uint32_t lo;
+        uint32_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
+        assign_axis<ORDER>(x, s, lo, ax);
+        assign_axis<ORDER>(y, s, lo, ay);
+        assign_axis<ORDER>(z, s, lo, az);
+        const uint32_t hx = anchor_node<ORDER>(x, s) - ox, hy = anchor_node<ORDER>(y, s) - oy,
+                       hz = anchor_node<ORDER>(z, s) - oz;
+        if ((hx | hy | hz) >= (uint32_t)TS) continue;  // at home in a neighbour
+        const int lx = (int)(hx + SHIFT), ly = (int)(hy + SHIFT), lz = (int)(hz + SHIFT);
+        float acc0 = 0.f, acc1 = 0.f;
 #pragma unroll
-            for (int dx = 0; dx <= ORDER; ++dx)
+        for (int dx = 0; dx <= ORDER; ++dx)
 #pragma unroll
-                for (int dy = 0; dy <= ORDER; ++dy) {
-                    const float wxy = ((float)ax[dx] * q) * ((float)ay[dy] * q);
-                    const float4* row = nd + ((lx + dx) * ILY + (ly + dy)) * ILZ + lz;
+            for (int dy = 0; dy <= ORDER; ++dy) {
+                const float wxy = ((float)ax[dx] * q) * ((float)ay[dy] * q);
+                const float2* row = nd + ((lx + dx) * TL + (ly + dy)) * TL + lz;
 #pragma unroll
-                    for (int dz = 0; dz <= ORDER; ++dz) {
-                        const float w = wxy * ((float)az[dz] * q);
-                        const float4 v = row[dz];
-                        acc0 = fmaf(w, v.x, acc0);
-                        acc1 = fmaf(w, v.y, acc1);
-                        acc2 = fmaf(w, v.z, acc2);
-                        acc3 = fmaf(w, v.w, acc3);
-                    }
+                for (int dz = 0; dz <= ORDER; ++dz) {
+                    const float w = wxy * ((float)az[dz] * q);
+                    const float2 v = row[dz];
+                    acc0 = fmaf(w, v.x, acc0);
+                    acc1 = fmaf(w, v.y, acc1);
                 }
-            fx[p] = acc0;
-            fy[p] = acc1;
-            fz[p] = acc2;
-            pot[p] = acc3;
-        }
+            }
+        out0[p] = acc0;
+        out1[p] = acc1;
     }
 }
 
@@ -481,48 +581,73 @@ void free_pm() {
     dev_free(g_pm.G);
     dev_free(g_pm.tcount);
     dev_free(g_pm.tstart);
-    dev_free(g_pm.slot);
+    dev_free(g_pm.bins);
     dev_free(g_pm.order);
     g_pm = PmState{};
 }
 
-// Per-particle buffers of the tiled deposit, grown to the container size.
+// The tile lists' entries, grown to what the container can need.
 int ensure_deposit(size_t n) {
     if (n <= g_pm.cap) return CT2_OK;
-    dev_free(g_pm.slot);
     dev_free(g_pm.order);
-    g_pm.slot = g_pm.order = nullptr;
+    g_pm.order = nullptr;
     g_pm.cap = 0;
-    CT2_TRY(dev_alloc((void**)&g_pm.slot, n * sizeof(int), "PM deposit slots"));
-    CT2_TRY(dev_alloc((void**)&g_pm.order, n * sizeof(int), "PM deposit order"));
+    CT2_TRY(dev_alloc((void**)&g_pm.order, n * MAX_COPIES * sizeof(int), "PM deposit order"));
     g_pm.cap = n;
     return CT2_OK;
 }
 
-// Density of the container's particles into g_pm.W (zeroed here).
+// The container's particles grouped by tile: g_pm.tstart, g_pm.order.
+template <int ORDER, int TILES>
+int bin_in_lds(const Context& c) {
+    const int n = (int)c.n, g = g_pm.g, nt = g_pm.ntile;
+    // at least 4 particles per thread, at most BIN_WGS workgroups: the counts of
+    // each are a row that bin_prefix walks
+    const int nw = std::max(1, std::min(BIN_WGS, n / (4 * BIN_THREADS)));
+    const int per = (n + nw - 1) / nw;
+    bin_count<ORDER, TILES><<<nw, BIN_THREADS, 0, c.stream>>>(c.x, c.y, c.z, n, per, g, nt, g_pm.bins);
+    CT2_LAUNCH_CHECK();
+    bin_prefix<<<(nt + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, c.stream>>>(g_pm.bins, nw, nt, g_pm.tcount);
+    CT2_LAUNCH_CHECK();
+    bin_scatter<ORDER, TILES><<<nw, BIN_THREADS, 0, c.stream>>>(c.x, c.y, c.z, n, per, g, nt, g_pm.bins, g_pm.tcount,
+                                                                g_pm.tstart, g_pm.order);
+    CT2_LAUNCH_CHECK();
+    return CT2_OK;
+}
+
+template <int ORDER>
+int bin_particles(const Context& c) {
+    CT2_TRY(ensure_deposit(c.n));
+    const int n = (int)c.n, g = g_pm.g, nt = g_pm.ntile;
+    if (nt <= BIN_TILES / 8) return bin_in_lds<ORDER, BIN_TILES / 8>(c);
+    if (nt <= BIN_TILES) return bin_in_lds<ORDER, BIN_TILES>(c);
+    const unsigned pb = (unsigned)((n + PM_BLOCK - 1) / PM_BLOCK);
+    fill_i32<<<(nt + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, c.stream>>>(g_pm.tcount, nt);
+    CT2_LAUNCH_CHECK();
+    bin_global<ORDER, false><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.tcount, nullptr);
+    CT2_LAUNCH_CHECK();
+    tile_scan<<<1, BIN_THREADS, 0, c.stream>>>(g_pm.tcount, nt, g_pm.tstart);
+    CT2_LAUNCH_CHECK();
+    bin_global<ORDER, true><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.tcount, g_pm.order);
+    CT2_LAUNCH_CHECK();
+    return CT2_OK;
+}
+
+// Density of the container's particles into g_pm.W.
 template <int ORDER>
 int deposit(const Context& c) {
     const int n = (int)c.n, g = g_pm.g;
-    const long n3 = 1L << (3 * g);
-    const unsigned gb = (unsigned)((n3 + PM_BLOCK - 1) / PM_BLOCK), pb = (unsigned)((n + PM_BLOCK - 1) / PM_BLOCK);
-    fill_u64<<<gb, PM_BLOCK, 0, c.stream>>>(g_pm.W, n3);
-    CT2_LAUNCH_CHECK();
     if (g < TILE_MIN_G) {
-        mesh_deposit<ORDER><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.W);
+        const long n3 = 1L << (3 * g);
+        fill_u64<<<(unsigned)((n3 + PM_BLOCK - 1) / PM_BLOCK), PM_BLOCK, 0, c.stream>>>(g_pm.W, n3);
+        CT2_LAUNCH_CHECK();
+        mesh_deposit<ORDER><<<(n + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.W);
         CT2_LAUNCH_CHECK();
         return CT2_OK;
     }
-    CT2_TRY(ensure_deposit(c.n));
+    CT2_TRY(bin_particles<ORDER>(c));
     const int nt = g_pm.ntile;
-    fill_i32<<<(nt + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, c.stream>>>(g_pm.tcount, nt);
-    CT2_LAUNCH_CHECK();
-    dep_count<ORDER><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.tcount, g_pm.slot);
-    CT2_LAUNCH_CHECK();
-    tile_scan<<<1, DEP_THREADS, 0, c.stream>>>(g_pm.tcount, nt, g_pm.tstart);
-    CT2_LAUNCH_CHECK();
-    dep_scatter<ORDER><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.tstart, g_pm.slot, g_pm.order);
-    CT2_LAUNCH_CHECK();
-    dep_tile<ORDER><<<nt, DEP_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.W);
+    dep_tile<ORDER><<<nt, TILE_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.W);
     CT2_LAUNCH_CHECK();
     return CT2_OK;
 }
@@ -586,19 +711,18 @@ int pm_forces() {
     CT2_TRY(xpass(g_pm.ng, g_pm.half, g_pm.A, g_pm.G, c.stream));
     CT2_TRY(fft_inverse_yz(g_pm.A, g_pm.ng, 2));
     // tiles hold n / ntile particles on average: stage a tile's nodes once when
-    // that beats one L2 read per particle and stencil node.  Measured: faster
-    // on 256^3 grids (0.19 -> 0.16 ms, TSC, 2^21 particles), slower on 512^3
-    // (1.0 -> 1.4 ms, 2^24 particles), where the per-particle gathers of
-    // particles in lattice order already hit L2 and the staged workgroup (one
-    // per CU) cannot overlap its loads with its arithmetic.
-    const bool tiled = g >= TILE_MIN_G && g <= 8 &&
-                       (long)n * (g_assign == 1 ? 8 : 27) > 2L * 2 * ILX * ILY * ILZ * g_pm.ntile;
+    // that beats one L2 read per particle and stencil node.  Measured, PM force
+    // per particle / tiled (TSC): 2^24 particles on 512^3, lattice 6.06 / 5.12 ms,
+    // half in Plummer spheres 12.7 / 10.7, random field 4.98 / 5.06.
+    const bool tiled = g >= TILE_MIN_G && g <= 9 &&
+                       (long)n * (g_assign == 1 ? 8 : 27) > 2L * TL_NODES * g_pm.ntile;
+    const dim3 tiles(g_pm.ntile, 2);
     if (tiled && g_assign == 1)
-        interp_tile<1><<<g_pm.ntile, DEP_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.A,
-                                                                 g_pm.B, c.fx, c.fy, c.fz, c.pot);
+        interp_tile<1><<<tiles, TILE_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.A, c.fx,
+                                                             c.fy, c.fz, c.pot);
     else if (tiled)
-        interp_tile<2><<<g_pm.ntile, DEP_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.A,
-                                                                 g_pm.B, c.fx, c.fy, c.fz, c.pot);
+        interp_tile<2><<<tiles, TILE_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.A, c.fx,
+                                                             c.fy, c.fz, c.pot);
     else if (g_assign == 1)
         mesh_interp<1><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.A, g_pm.B, c.fx, c.fy, c.fz, c.pot);
     else
@@ -650,8 +774,10 @@ extern "C" int ct2_pm_init(int ng, double rs_cells) {
     g_pm.ng = ng;
     g_pm.g = ilog2(ng);
     if (g_pm.g >= TILE_MIN_G) {
-        g_pm.ntile = 1 << (3 * g_pm.g - TILE_BX - TILE_BY - TILE_BZ);
-        if ((rc = dev_alloc((void**)&g_pm.tcount, (size_t)g_pm.ntile * sizeof(int), "PM tile counts")) ||
+        g_pm.ntile = 1 << (3 * (g_pm.g - TILE_B));
+        const size_t nt = (size_t)g_pm.ntile;
+        if ((rc = dev_alloc((void**)&g_pm.tcount, nt * sizeof(int), "PM tile counts")) ||
+            (nt <= BIN_TILES && (rc = dev_alloc((void**)&g_pm.bins, nt * BIN_WGS * sizeof(int), "PM bins"))) ||
             (rc = dev_alloc((void**)&g_pm.tstart, (size_t)(g_pm.ntile + 1) * sizeof(int), "PM tile starts"))) {
             free_pm();
             return rc;

@@ -185,6 +185,29 @@ def test_tsc_deposit_bit_exact(ct2, orc, tsc, ng):
     assert np.array_equal(ct2.pm_density_download(), orc.mesh_deposit(x, y, z, ng.bit_length() - 1, 2))
 
 
+@pytest.mark.parametrize("ng,order", [(128, 1), (512, 2), (1024, 2)])
+def test_deposit_binning_by_grid_size_bit_exact(ct2, orc, ng, order):
+    """The three ways tiles are counted (512 and 32,768 tiles in LDS, 262,144 by
+    global atomics), with several binning workgroups, and particles on every
+    face, edge and corner of tiles."""
+    rng = np.random.default_rng(ng)
+    n, s = 9001, 32 - (ng.bit_length() - 1)
+    node = rng.integers(0, ng, (3, n), dtype=np.uint64) // 16 * 16  # the first node of a tile, or next to it
+    x, y, z = ((node.astype(np.int64) + rng.integers(-2, 2, (3, n))) % ng * (1 << s) +
+               rng.integers(0, 1 << s, (3, n))).astype(np.uint64).astype(np.uint32)
+    load(ct2, x, y, z)
+    ct2.set_force_options(1e-3, 1.0 / n, 0)
+    ct2.pm_assignment(order)
+    try:
+        ct2.pm_init(ng, 1.25)
+        ct2.pm_forces()
+        got = ct2.pm_density_download()
+    finally:
+        ct2.pm_assignment(1)
+        ct2.pm_init(8, 1.25)  # the large grids are released
+    assert np.array_equal(got.ravel(), orc.mesh_deposit(x, y, z, ng.bit_length() - 1, order).ravel())
+
+
 @pytest.mark.parametrize("order", [1, 2])
 @pytest.mark.parametrize("ng", [8, 32, 64])
 @pytest.mark.parametrize("n", [1, 63, 1037, 4096])
