@@ -883,6 +883,27 @@ KickConst kick_const(double h) {
     return kc;
 }
 
+// Only a descending kick assigns rungs (kick.cpp:84-99); any other returns 0,
+// whatever the counter holds, and neither clears nor copies it (a launch and a
+// copy of ~2 us each between the kernels of a small kick).
+int clear_max_rung(Context& c, const ct2_kick_params* p, int* maxrung) {
+    if (!p->descending) return CT2_OK;
+    zero_int<<<1, 1, 0, c.stream>>>(maxrung);
+    CT2_LAUNCH_CHECK();
+    return CT2_OK;
+}
+
+// kick()'s return value, synchronously; null: neither copied nor waited for.
+int return_max_rung(Context& c, const ct2_kick_params* p, const int* maxrung, int* max_rung) {
+    if (!max_rung) return CT2_OK;
+    if (p->descending)
+        CT2_HIP(hipMemcpyAsync(max_rung, maxrung, sizeof(int), hipMemcpyDeviceToHost, c.stream));
+    else
+        *max_rung = 0;
+    CT2_HIP(hipStreamSynchronize(c.stream));
+    return CT2_OK;
+}
+
 // Sums the partial-sum sets, stores the force and runs the epilogue, then
 // hands back kick()'s return value from the device counter maxrung.
 int finish_kick(Context& c, const ct2_kick_params* p, const PartialSums* sets, int n, int i0, int* maxrung,
@@ -898,11 +919,7 @@ int finish_kick(Context& c, const ct2_kick_params* p, const PartialSums* sets, i
     CT2_LAUNCH_CHECK();
     c.forces_valid = true;
     c.last_path = CT2_PATH_DIRECT;
-    if (max_rung) {
-        CT2_HIP(hipMemcpyAsync(max_rung, maxrung, sizeof(int), hipMemcpyDeviceToHost, c.stream));
-        CT2_HIP(hipStreamSynchronize(c.stream));
-    }
-    return CT2_OK;
+    return return_max_rung(c, p, maxrung, max_rung);
 }
 
 }  // namespace
@@ -961,8 +978,7 @@ int check_kick_params(const ct2_kick_params* p) {
 int run_epilogue(const ct2_kick_params* p, int* max_rung) {
     Context& c = ctx();
     if (!c.maxrung) CT2_TRY(dev_alloc((void**)&c.maxrung, sizeof(int), "max rung"));
-    zero_int<<<1, 1, 0, c.stream>>>(c.maxrung);
-    CT2_LAUNCH_CHECK();
+    CT2_TRY(clear_max_rung(c, p, c.maxrung));
     if (epilogue_active(p)) {
         const EpiConst e = make_epilogue(p, c.opts.hsoft);
         const int n = (int)c.n, i0 = (int)c.rung_begin;
@@ -972,11 +988,7 @@ int run_epilogue(const ct2_kick_params* p, int* max_rung) {
             CT2_LAUNCH_CHECK();
         }
     }
-    if (max_rung) {
-        CT2_HIP(hipMemcpyAsync(max_rung, c.maxrung, sizeof(int), hipMemcpyDeviceToHost, c.stream));
-        CT2_HIP(hipStreamSynchronize(c.stream));
-    }
-    return CT2_OK;
+    return return_max_rung(c, p, c.maxrung, max_rung);
 }
 
 }  // namespace ct2
@@ -1003,8 +1015,7 @@ extern "C" int ct2_kick(const ct2_kick_params* p, unsigned flags, int* max_rung)
     const KickConst kc = kick_const(c.opts.hsoft);
     const bool naive = flags & CT2_KICK_NAIVE;
     const bool plummer = c.opts.kernel == CT2_KERNEL_PLUMMER;
-    zero_int<<<1, 1, 0, c.stream>>>(c.maxrung);
-    CT2_LAUNCH_CHECK();
+    CT2_TRY(clear_max_rung(c, p, c.maxrung));
     // Each unordered pair once where possible: the symmetric kernels take the
     // last m = floor(ns / 1024) * 1024 active sinks (the core [c0, n)); the
     // ordered kernel adds the core's pairs with the particles before it and
@@ -1051,8 +1062,7 @@ extern "C" int ct2_kick_noalloc(const ct2_kick_params* p, unsigned flags, int* m
         return CT2_OK;
     }
     int* maxrung = (int*)((char*)base + NOALLOC_PART_BYTES);
-    zero_int<<<1, 1, 0, c.stream>>>(maxrung);
-    CT2_LAUNCH_CHECK();
+    CT2_TRY(clear_max_rung(c, p, maxrung));
     PartialSums sets[3] = {{nullptr, 0, 0, 0}, {nullptr, 0, 0, 0}, {nullptr, 0, 0, 0}};
     CT2_TRY(ordered_pass(c, i0, n, n, flags & CT2_KICK_NAIVE, c.opts.kernel == CT2_KERNEL_PLUMMER,
                          kick_const(c.opts.hsoft), nullptr, nullptr, &sets[0], (double*)base, NOALLOC_PART_BYTES));
