@@ -1,7 +1,7 @@
 // kick.hip -- the direct-sum kick of kick.cpp:3-125 on gfx950.
 //
-// kick_direct: one sink per lane; sources stream through LDS in tiles of
-// KICK_TILE (coalesced SoA loads, double-buffered, one barrier per tile) and
+// kick_direct: one sink per lane; sources stream through LDS in tiles
+// (coalesced SoA loads, double-buffered, one barrier per tile) and
 // are read back as 16-byte LDS broadcasts.  Separations are formed in the
 // fixed32 integer domain (exact minimum image) and converted to FP32 in
 // units of 2^-32, so no per-pair scale multiply is needed.  Each tile is
@@ -26,8 +26,7 @@
 namespace ct2 {
 namespace {
 
-constexpr int KICK_BLOCK = 256;  // sinks per workgroup
-constexpr int KICK_TILE = 256;   // sources per LDS tile (== KICK_BLOCK: one load per lane)
+constexpr int KICK_BLOCK = 256;  // threads per workgroup of kick_direct
 
 struct KickConst {
     float eps2u;   // Plummer: (h 2^32)^2
@@ -73,37 +72,61 @@ __device__ __forceinline__ void interact(const uint4 src, uint32_t xi, uint32_t 
     }
 }
 
-// grid: (ceil(nsink/KICK_BLOCK), nsplit), sinks i0 .. i1-1; block y sums
-// sources [y*jchunk, min(nsrc, (y+1)*jchunk)) of sources 0 .. nsrc-1.
+// grid: (ceil(nsink / sinks per workgroup), nsplit), sinks i0 .. i1-1; block y
+// sums sources [y*jchunk, min(nsrc, (y+1)*jchunk)) of sources 0 .. nsrc-1.
 // Output: partial[(a*nsplit + y)*nsink + i] for a in {x,y,z,pot}, in units
 // of 2^-64 (force) and 2^-32 (potential); see the scaling in kick_finalize.
+// A workgroup takes 64 sinks; its four waves share every tile of 512 sources, a
+// quarter each, and their sums are added in FP64 in LDS: a quarter of the
+// partial sums that one sink per thread leaves for the same number of waves in
+// flight, and no more than 63 idle lanes in the last workgroup.  (NAIVE: 256
+// sinks and one sum over the chunk each, as its plain FP32 accumulation means.)
+// Bound by VALU issue, 16 instructions a pair.
+template <bool NAIVE>
+struct Kick {
+    static constexpr int PARTS = NAIVE ? 1 : KICK_BLOCK / 64;  // waves that share a sink's sources
+    static constexpr int SINKS = KICK_BLOCK / PARTS;
+    static constexpr int TILE = NAIVE ? KICK_BLOCK : 2 * KICK_BLOCK;
+    static constexpr int LOADS = TILE / KICK_BLOCK;
+};
+
 template <int KERNEL, bool NAIVE>
 __global__ __launch_bounds__(KICK_BLOCK) void kick_direct(const uint32_t* __restrict__ X,
                                                           const uint32_t* __restrict__ Y,
                                                           const uint32_t* __restrict__ Z, int i0, int i1, int nsrc,
                                                           int jchunk, KickConst kc,
                                                           double* __restrict__ partial) {
-    __shared__ uint4 tile[2][KICK_TILE];
+    using K = Kick<NAIVE>;
+    constexpr int PART = K::TILE / K::PARTS;  // sources of a tile per wave
+    __shared__ uint4 tile[2][K::TILE];
     const int tid = threadIdx.x;
     const int ns = i1 - i0;  // sinks i0 .. i1-1
-    const int i = blockIdx.x * KICK_BLOCK + tid;
+    const int i = blockIdx.x * K::SINKS + tid % K::SINKS;
     const int ic = i < ns ? i0 + i : i1 - 1;
     const uint32_t xi = X[ic], yi = Y[ic], zi = Z[ic];
+    const int part = __builtin_amdgcn_readfirstlane(tid / K::SINKS);
 
     const int j0 = blockIdx.y * jchunk;
     const int j1 = min(nsrc, j0 + jchunk);
     float sx = 0.f, sy = 0.f, sz = 0.f, sp = 0.f;
     float cx = 0.f, cy = 0.f, cz = 0.f, cp = 0.f;
 
-    uint4 pre = make_uint4(0u, 0u, 0u, 0u);
-    if (j0 + tid < j1) pre = make_uint4(X[j0 + tid], Y[j0 + tid], Z[j0 + tid], 0u);
+    uint4 pre[K::LOADS];
+    auto fetch = [&](int jt) {
+#pragma unroll
+        for (int u = 0; u < K::LOADS; ++u) {
+            const int j = jt + u * KICK_BLOCK + tid;
+            if (j < j1) pre[u] = make_uint4(X[j], Y[j], Z[j], 0u);
+        }
+    };
+    fetch(j0);
     int buf = 0;
-    for (int jt = j0; jt < j1; jt += KICK_TILE) {
-        tile[buf][tid] = pre;
+    for (int jt = j0; jt < j1; jt += K::TILE) {
+#pragma unroll
+        for (int u = 0; u < K::LOADS; ++u) tile[buf][u * KICK_BLOCK + tid] = pre[u];
         __syncthreads();
-        const int jn = jt + KICK_TILE + tid;
-        if (jn < j1) pre = make_uint4(X[jn], Y[jn], Z[jn], 0u);
-        const int cnt = min(KICK_TILE, j1 - jt);
+        fetch(jt + K::TILE);
+        const int cnt = min(PART, j1 - jt - part * PART);
         float tx = 0.f, ty = 0.f, tz = 0.f, tp = 0.f;
         if (NAIVE) {
             tx = sx;
@@ -111,10 +134,10 @@ __global__ __launch_bounds__(KICK_BLOCK) void kick_direct(const uint32_t* __rest
             tz = sz;
             tp = sp;
         }
-        const uint4* T = tile[buf];
-        if (cnt == KICK_TILE) {
+        const uint4* T = tile[buf] + part * PART;
+        if (cnt == PART) {
 #pragma unroll 16
-            for (int j = 0; j < KICK_TILE; ++j) interact<KERNEL>(T[j], xi, yi, zi, kc, tx, ty, tz, tp);
+            for (int j = 0; j < PART; ++j) interact<KERNEL>(T[j], xi, yi, zi, kc, tx, ty, tz, tp);
         } else {
             for (int j = 0; j < cnt; ++j) interact<KERNEL>(T[j], xi, yi, zi, kc, tx, ty, tz, tp);
         }
@@ -131,12 +154,25 @@ __global__ __launch_bounds__(KICK_BLOCK) void kick_direct(const uint32_t* __rest
         }
         buf ^= 1;
     }
-    if (i < ns) {
-        const long nsp = gridDim.y, y = blockIdx.y;
-        partial[(0 * nsp + y) * ns + i] = (double)sx + (double)cx;
-        partial[(1 * nsp + y) * ns + i] = (double)sy + (double)cy;
-        partial[(2 * nsp + y) * ns + i] = (double)sz + (double)cz;
-        partial[(3 * nsp + y) * ns + i] = (double)sp + (double)cp;
+    const long nsp = gridDim.y, y = blockIdx.y;
+    const double own[4] = {(double)sx + (double)cx, (double)sy + (double)cy, (double)sz + (double)cz,
+                           (double)sp + (double)cp};
+    if constexpr (K::PARTS == 1) {
+        if (i < ns)
+#pragma unroll
+            for (int a = 0; a < 4; ++a) partial[(a * nsp + y) * ns + i] = own[a];
+    } else {
+        double(*red)[4][K::SINKS] = (double(*)[4][K::SINKS]) & tile[0][0];  // [part][component][sink]
+        static_assert(sizeof(double) * K::PARTS * 4 * K::SINKS <= sizeof(tile), "the sums fit in the tiles");
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < 4; ++a) red[part][a][tid % K::SINKS] = own[a];
+        __syncthreads();
+        // thread t: component t / 64 of sink t % 64
+        double v = 0.0;
+#pragma unroll
+        for (int q = 0; q < K::PARTS; ++q) v += red[q][part][tid % K::SINKS];
+        if (i < ns) partial[(part * nsp + y) * ns + i] = v;
     }
 }
 
@@ -147,7 +183,12 @@ struct PartialSums {
 };
 
 // Sums, for every sink i in [i0, n), the planes of each of the (up to three)
-// partial-sum sets that cover i, in the set order given.
+// partial-sum sets that cover i, in the set order given.  A workgroup takes SW
+// sinks: 4 threads a sink for the components, times 64 / SW that walk the planes
+// in turn; the fewer the sinks (and the more the planes), the smaller SW (one
+// thread a sink took 29 us for 32,768 sinks of 32 planes, and 800 us of the 870
+// for 100 sinks of 977).
+template <int SW>
 __global__ __launch_bounds__(256) void kick_finalize(PartialSums s0, PartialSums s1, PartialSums s2,
                                                      int n, int i0, double fscale, double pscale, EpiConst e,
                                                      float* __restrict__ vx, float* __restrict__ vy,
@@ -155,27 +196,38 @@ __global__ __launch_bounds__(256) void kick_finalize(PartialSums s0, PartialSums
                                                      float* __restrict__ fx, float* __restrict__ fy,
                                                      float* __restrict__ fz, float* __restrict__ pot,
                                                      int* __restrict__ maxrung) {
+    constexpr int G = 64 / SW;
+    __shared__ double red[4][G][SW];
     const int ns = n - i0;
-    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int k = threadIdx.x % SW, grp = threadIdx.x / SW % G, c = threadIdx.x / 64;
+    const int t = blockIdx.x * SW + k;
     const int i = i0 + t;
+    double a = 0.0;
+    for (const PartialSums& ps : {s0, s1, s2}) {
+        const int r = i - ps.first;
+        if (t >= ns || !ps.part || r < 0 || r >= ps.count) continue;
+        const double* p = ps.part + (long)c * ps.nsplit * ps.count + r;
+        double s = 0.0;
+#pragma unroll 8
+        for (int y = grp; y < ps.nsplit; y += G) s += p[(long)y * ps.count];
+        a += s;
+    }
+    red[c][grp][k] = a;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;  // the first wave carries on, one sink a lane
     int rmax = 0;
-    if (t < ns) {
-        double a[4] = {0.0, 0.0, 0.0, 0.0};
-        for (const PartialSums& ps : {s0, s1, s2}) {
-            const int k = i - ps.first;
-            if (!ps.part || k < 0 || k >= ps.count) continue;
+    if (threadIdx.x < SW && t < ns) {
+        double f[4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                double s = 0.0;
-                for (int y = 0; y < ps.nsplit; ++y) s += ps.part[((long)c * ps.nsplit + y) * ps.count + k];
-                a[c] += s;
-            }
+        for (int q = 0; q < 4; ++q) {
+            f[q] = 0.0;
+            for (int g = 0; g < G; ++g) f[q] += red[q][g][k];
         }
-        const float f0 = (float)(a[0] * fscale), f1 = (float)(a[1] * fscale), f2 = (float)(a[2] * fscale);
+        const float f0 = (float)(f[0] * fscale), f1 = (float)(f[1] * fscale), f2 = (float)(f[2] * fscale);
         fx[i] = f0;
         fy[i] = f1;
         fz[i] = f2;
-        pot[i] = (float)(a[3] * pscale);
+        pot[i] = (float)(f[3] * pscale);
         if (e.kick_ascending || e.descending) {
             float u = vx[i], v = vy[i], w = vz[i];
             int8_t r = rung[i];
@@ -186,9 +238,9 @@ __global__ __launch_bounds__(256) void kick_finalize(PartialSums s0, PartialSums
             rung[i] = r;
         }
     }
-    // wave-level max, then one atomic per wave
+    // the wave's max, then one atomic
     for (int off = 32; off > 0; off >>= 1) rmax = max(rmax, __shfl_xor(rmax, off));
-    if ((threadIdx.x & 63) == 0 && rmax > 0) atomicMax(maxrung, rmax);
+    if (threadIdx.x == 0 && rmax > 0) atomicMax(maxrung, rmax);
 }
 
 // Epilogue over stored forces (mesh-based kicks).
@@ -772,13 +824,20 @@ size_t g_part_b_bytes = 0;
 int ordered_pass(Context& c, int i0, int i1, int nsrc, bool naive, bool plummer, const KickConst& kc, double** buf,
                  size_t* bytes, PartialSums* out, double* fixed = nullptr, size_t fixed_bytes = 0) {
     const int ns = i1 - i0;
-    const int nb = (ns + KICK_BLOCK - 1) / KICK_BLOCK;
-    const int max_split = std::max(1, nsrc / (4 * KICK_TILE));
-    int nsplit = std::min(max_split, std::max(1, (4096 + nb - 1) / nb));
+    const int sinks = naive ? Kick<true>::SINKS : Kick<false>::SINKS, tile = naive ? Kick<true>::TILE : Kick<false>::TILE;
+    const int nb = (ns + sinks - 1) / sinks;
+    // 16,384 workgroups even out the last ones to finish (8 waves of them are in
+    // flight at a time): 15,625 sinks x 1,000,003 sources 4.87 ms, with 8,192
+    // 4.94, with 4,096 5.39; 32,768 x 32,768 0.355 / 0.358 / 0.381.  Below 5e8
+    // pairs there is little to even out, and 4,096 workgroups leave at most 8 MiB
+    // of partial sums, what ct2_kick_noalloc has room for.
+    const int want = (double)ns * nsrc > 5e8 ? 16384 : 4096;
+    const int max_split = std::max(1, nsrc / (naive ? 4 * tile : tile));
+    int nsplit = std::min(max_split, std::max(1, naive ? (4096 + nb - 1) / nb : want / nb));
     const size_t per_split = sizeof(double) * 4 * (size_t)ns;
     if (fixed) nsplit = (int)std::max<size_t>(1, std::min<size_t>(nsplit, fixed_bytes / per_split));
     int jchunk = (nsrc + nsplit - 1) / nsplit;
-    jchunk = (jchunk + KICK_TILE - 1) / KICK_TILE * KICK_TILE;
+    jchunk = (jchunk + tile - 1) / tile * tile;
     const int nsplit_eff = (nsrc + jchunk - 1) / jchunk;
     double* part = fixed;
     if (fixed) {
@@ -913,9 +972,17 @@ int finish_kick(Context& c, const ct2_kick_params* p, const PartialSums* sets, i
     // force in box units: sum(dxu * w3u) * 2^64 * GM; potential: sum(wu) * 2^32 * GM
     const double fscale = (double)c.opts.GM * two32 * two32;
     const double pscale = (double)c.opts.GM * two32;
-    kick_finalize<<<(n - i0 + 255) / 256, 256, 0, c.stream>>>(sets[0], sets[1], sets[2], n, i0, fscale, pscale, e,
-                                                              c.vx, c.vy, c.vz, c.rung, c.fx, c.fy, c.fz, c.pot,
-                                                              maxrung);
+    const int planes = std::max({sets[0].nsplit, sets[1].nsplit, sets[2].nsplit});
+    auto launch = [&](auto kernel, int sw) {
+        kernel<<<(n - i0 + sw - 1) / sw, 256, 0, c.stream>>>(sets[0], sets[1], sets[2], n, i0, fscale, pscale, e, c.vx,
+                                                             c.vy, c.vz, c.rung, c.fx, c.fy, c.fz, c.pot, maxrung);
+    };
+    if (planes >= 128)
+        launch(kick_finalize<4>, 4);
+    else if (planes >= 32)
+        launch(kick_finalize<16>, 16);
+    else
+        launch(kick_finalize<64>, 64);
     CT2_LAUNCH_CHECK();
     c.forces_valid = true;
     c.last_path = CT2_PATH_DIRECT;
