@@ -351,23 +351,29 @@ __global__ __launch_bounds__(256) void mm_row_items(const int* __restrict__ star
 
 // ------------------------------------------------------------ P2M
 
-// MM_P2M_CELLS consecutive cells per workgroup, MM_P2M_CELLS / 4 of them per
-// wave in turn: the powers of -b (offset from the cell centre, in cells) of up
-// to 64 particles in the wave's LDS slot, lane c (and c + 64, c + 128) sums
-// component c over them in FP64; the moments of the block's cells collect in
-// LDS and leave as rows of MM_P2M_CELLS consecutive cells per grid.  Component
-// c goes to grid c/2, real part for even c, imaginary for odd (an odd K leaves
-// the last imaginary part 0).
-constexpr int MM_P2M_CELLS = 32;
+// MM_P2M_CELLS consecutive cells per workgroup, a wave taking every fourth: the
+// powers of -b (offset from the cell centre, in cells) of up to MM_P2M_PART
+// particles in the wave's LDS slot (one lane per particle and axis), lane c (and
+// c + 64, c + 128) sums component c over them in FP64, four particles' reads in
+// flight together; the moments of the block's cells collect in LDS and leave as
+// rows of MM_P2M_CELLS consecutive cells (128 bytes) per grid.  Component c goes
+// to grid c/2, real part for even c, imaginary for odd (an odd K leaves the last
+// imaginary part 0).  Bound by the latency of its LDS reads: 19 KB of LDS per
+// workgroup, so that eight share a CU (with room for 64 particles per wave and
+// 32 cells, three did), took order 8 on 64^3 cells of 8 particles from 299 to
+// 125 us.
+constexpr int MM_P2M_CELLS = 16, MM_P2M_PART = 16;
 __global__ __launch_bounds__(256) void mm_p2m(const uint4* __restrict__ P, const int* __restrict__ start, int lg, int Pord,
                                               int K, size_t n3, float2* __restrict__ Zm) {
-    __shared__ float pw[4][64][3][MM_PMAX + 1];
+    __shared__ float pw[4][MM_P2M_PART][3][MM_PMAX + 1];
     __shared__ float Mo[MM_KMAX + 1][MM_P2M_CELLS + 1];  // + 1: a cell's column spreads over the banks
+    static_assert(3 * MM_P2M_PART <= 64 && MM_P2M_PART % 4 == 0, "a lane per particle and axis, four particles at a time");
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const size_t cell0 = (size_t)blockIdx.x * MM_P2M_CELLS;
     const int sh = 32 - lg;
     const uint32_t mask = (1u << sh) - 1u, half = 1u << (sh - 1);
     const float inv = ldexpf(1.0f, -sh);
+    const int q = lane / MM_P2M_PART, j = lane % MM_P2M_PART;
     int ex[3][3];
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
@@ -380,30 +386,34 @@ __global__ __launch_bounds__(256) void mm_p2m(const uint4* __restrict__ P, const
         const size_t cell = cell0 + lc;
         const int s0 = start[cell], s1 = start[cell + 1];
         double acc[3] = {0.0, 0.0, 0.0};
-        for (int base = s0; base < s1; base += 64) {
-            if (base + lane < s1) {
-                const uint4 p = P[base + lane];
-                const uint32_t v[3] = {p.x, p.y, p.z};
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    const float mb = -(float)(int32_t)((v[q] & mask) - half) * inv;  // -b in cells
-                    float pv = 1.0f;
-                    pw[w][lane][q][0] = 1.0f;
-                    for (int e = 1; e <= Pord; ++e) {
-                        pv *= mb;
-                        pw[w][lane][q][e] = pv;
-                    }
+        for (int base = s0; base < s1; base += MM_P2M_PART) {
+            if (q < 3) {
+                // past the cell's last particle: all powers 0, so that it adds nothing
+                const bool have = base + j < s1;
+                const uint32_t v = have ? ((const uint32_t*)(P + base + j))[q] : 0u;
+                const float mb = have ? -(float)(int32_t)((v & mask) - half) * inv : 0.0f;  // -b in cells
+                float pv = have ? 1.0f : 0.0f;
+                for (int e = 0; e <= Pord; ++e) {
+                    pw[w][j][q][e] = pv;
+                    pv *= mb;
                 }
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            const int cnt = min(64, s1 - base);
+            const int cnt = min(MM_P2M_PART, s1 - base);
+            for (int j0 = 0; j0 < cnt; j0 += 4) {
 #pragma unroll
-            for (int r = 0; r < 3; ++r)
-                if (lane + 64 * r < K)
-                    for (int j = 0; j < cnt; ++j)
-                        acc[r] += (double)(pw[w][j][0][ex[r][0]] * pw[w][j][1][ex[r][1]] * pw[w][j][2][ex[r][2]]);
+                for (int r = 0; r < 3; ++r) {
+                    if (lane + 64 * r >= K) continue;
+                    float m[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        m[u] = pw[w][j0 + u][0][ex[r][0]] * pw[w][j0 + u][1][ex[r][1]] * pw[w][j0 + u][2][ex[r][2]];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) acc[r] += (double)m[u];
+                }
+            }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
