@@ -47,29 +47,24 @@ constexpr int MM_PMAX = 8;
 constexpr int MM_KMAX = 165;       // components at P = 8
 constexpr int MM_NEAR2 = 10;       // |cell offset|^2 of the direct set (particle.cpp:136)
 constexpr double MM_BETA = 0.5;    // Ewald split per cell
-constexpr int MM_QB = 16;          // wave vectors per MG2L workgroup
-constexpr int MM_SLOTS = 16;       // MG2L work lists per wave vector (256 threads)
-constexpr int MM_SCHED_MAX = 384;  // entries per list
-// list stride in words: rows of whole 16-byte groups, the lists of a wave 16 bytes apart modulo 128
-constexpr int mg2l_stride(int slen) { return (slen + 31) / 32 * 32 + 4; }
+constexpr int MM_QB = 64;          // wave vectors per MG2L workgroup, one per lane
 constexpr int MM_COLS_MAX = 48;    // (dx, dy) columns of the near set (37 at |d|^2 <= 10)
 constexpr int MM_WAVES = 4;        // waves per near-field workgroup
 
-// MG2L list entry: flags | l << 7 | j << 15 | n << 22, so that l * 128 (the
-// byte offset of row l of the LDS multipoles) is a mask of the word and n * 64
-// (row n of the LDS table) a shift.  Entries come in groups of four products
-// M^_l D^_n of one output component and one parity of |n| (D^_n is real for
-// even |n|, i times real for odd); the group's last entry carries its flags.
-// The components 2j and 2j+1 share a list: at the last group of 2j (save) the
-// sum is set aside, at the last of 2j+1 (flush) L^_2j + i L^_2j+1 goes out.
-// Pads: l = 0 and n = K, a zero row.
-constexpr uint32_t G_ODD = 1u, G_SAVE = 2u, G_FLUSH = 4u;
-__host__ __device__ constexpr uint32_t mg2l_entry(int l, int n, int j, uint32_t flags) {
-    return flags | (uint32_t)l << 7 | (uint32_t)j << 15 | (uint32_t)n << 22;
-}
+// An MG2L work list (one per wave), three times 64 words.  First the outputs:
+// P - |k| (0: two components of degree P) | output grid << 4 | degree |k| << 11;
+// then, output by output, the rows of the first multipole (8 bits) and of the
+// first table value of each run, two runs to a word; last what the wave stages,
+// and in its last word the number of outputs.  Rows are the components in column
+// order (by (a, b), then the z exponent).
+constexpr uint32_t MG2L_NONE = 255u;
+constexpr int MG2L_STEPS = 64, MG2L_LIST = 3 * MG2L_STEPS;  // words per list
+constexpr uint32_t mg2l_rows(int m, int d) { return (uint32_t)m | (uint32_t)d << 8; }
 
 __constant__ int c_e[MM_KMAX][3];         // exponents of component c
 __constant__ float c_ifact[MM_KMAX];      // 1 / (a! b! c!)
+__constant__ int c_le[MM_KMAX][3];        // exponents of the local expansions, in the order of their grids
+__constant__ float c_lifact[MM_KMAX];
 __constant__ int c_cols[MM_COLS_MAX][3];  // near set by column: dx, dy, half-height w in z
 
 struct MMIndex {
@@ -110,7 +105,7 @@ struct MMIndex {
 
 struct MMState {
     int nc = 0, P = 0, K = 0, nz = 0;  // nz = complex grids (K/2 rounded up)
-    int slen = 0, ncols = 0;
+    int ncols = 0;
     double* Dt = nullptr;  // [K][nc^3]
     size_t Dt_bytes = 0;
     float* Dt32 = nullptr;  // the same rounded to FP32, the rows MG2L reads
@@ -135,7 +130,7 @@ struct MMState {
     size_t scan_tmp_bytes = 0;
     double2* tabz = nullptr;  // one FP64 complex grid while the table is built
     size_t tabz_bytes = 0;
-    uint32_t* sched = nullptr;  // the MG2L lists [MM_SLOTS][mg2l_stride(slen)]
+    uint32_t* sched = nullptr;  // the MG2L lists [waves][MG2L_LIST]
     size_t sched_bytes = 0;
 };
 MMState g_mm;
@@ -436,81 +431,150 @@ __global__ __launch_bounds__(256) void mm_p2m(const uint4* __restrict__ P, const
 
 // ------------------------------------------------------------ MG2L
 
-// MM_QB wave vectors per workgroup: the transformed multipoles unpacked from
-// the paired grids (Z(q) and Z(-q)) and the table rows (rounded to FP32) in
-// LDS; thread (slot, qq) walks list `slot` (read through L1: every workgroup
-// reads the same lists) four products at a time, all lists of equal length,
-// each pair of components (2j, 2j+1) in one list, and writes L^_2j + i L^_2j+1
-// (paired like the multipoles, for the inverse transforms).  A group's four
-// products sum in FP32 (the multipoles are FP32 already), groups in FP64:
-// those with real D^_n into (ar, ai), those with imaginary D^_n (as M^ times
-// the real coefficient) into (br, bi); a component is (ar - bi) + i (ai + br).
-static_assert(MM_QB * sizeof(float2) == 128 && MM_QB * sizeof(float) == 64, "LDS rows of 128 and 64 bytes");
-__global__ __launch_bounds__(256) void mm_mg2l(const float2* __restrict__ Zm, const float* __restrict__ Dt32,
-                                               const uint32_t* __restrict__ sched, int nc, int K, int nz, int slen,
-                                               float2* __restrict__ Zl) {
-    __shared__ float2 Mh[MM_KMAX][MM_QB];
-    __shared__ float Dq[MM_KMAX + 1][MM_QB];
-    const size_t n3 = (size_t)nc * nc * nc;
-    const size_t q0 = (size_t)blockIdx.x * MM_QB;
-    const int t = threadIdx.x;
-    const int m = nc - 1;
-    for (int e = t; e < nz * MM_QB; e += 256) {
-        const int j = e / MM_QB, qq = e % MM_QB;
-        const size_t q = q0 + qq;
-        const int i0 = (int)(q / ((size_t)nc * nc)), i1 = (int)(q / nc % nc), i2 = (int)(q % nc);
-        const size_t qn = ((size_t)((-i0) & m) * nc + (size_t)((-i1) & m)) * nc + (size_t)((-i2) & m);
-        const float2 a = Zm[(size_t)j * n3 + q], b = Zm[(size_t)j * n3 + qn];
-        Mh[2 * j][qq] = make_float2(0.5f * (a.x + b.x), 0.5f * (a.y - b.y));          // (Z(q) + conj Z(-q)) / 2
-        if (2 * j + 1 < K) Mh[2 * j + 1][qq] = make_float2(0.5f * (a.y + b.y), 0.5f * (b.x - a.x));  // / 2i
-    }
-    for (int e = t; e < K * MM_QB; e += 256) {
-        const int c = e / MM_QB, qq = e % MM_QB;
-        Dq[c][qq] = Dt32[(size_t)c * n3 + q0 + qq];
-    }
-    if (t < MM_QB) Dq[K][t] = 0.0f;  // the pads' row
-    __syncthreads();
-    const int qq = t & (MM_QB - 1), slot = t / MM_QB;
-    const uint32_t* L = sched + slot * mg2l_stride(slen);
-    const char* mb = (const char*)&Mh[0][qq];
-    const char* db = (const char*)&Dq[0][qq];
-    double ar = 0.0, ai = 0.0, br = 0.0, bi = 0.0, er = 0.0, ei = 0.0;
-    uint4 gn = *(const uint4*)L;  // the next group's entries, read one group ahead
-    for (int i = 0; i < slen; i += 4) {
-        const uint4 g = gn;
-        if (i + 4 < slen) gn = *(const uint4*)(L + i + 4);
-        const uint32_t w[4] = {g.x, g.y, g.z, g.w};
-        float2 mv[4];
-        float d[4];
+// L^_k = sum_l M^_l D^_{k+l} per wave vector.  With M'_l = i^|l| M^_l and the
+// table's D^_n = i^|n| D'_n (D' real), L^_k = i^|k| sum_l M'_l D'_{k+l}: one
+// complex by real product per term, whatever the parities.  MM_QB wave vectors
+// per workgroup, one per lane: the transformed multipoles, unpacked from the
+// paired grids (Z(q) and Z(-q)) and turned by i^|l|, and the table rows with
+// their sign in LDS, in column order.  An output is the pair k, k + e_z (z
+// exponents kz, kz + 1, kz even): for every column (lx, ly) it takes the run of
+// R + 1 multipoles and of R + 1 table values from LDS once, for 2 R + 1 products.
+// Up to four products sum in FP32 (the multipoles are FP32 already), these sums
+// in FP64.  Written as i^|k| (S_k - S_{k+e_z}) = L^_k + i L^_{k+e_z}, ready for
+// the inverse transforms; the highest z exponents left over, of one product each,
+// in pairs (S_a + i S_b).  The waves of a workgroup walk lists of outputs of about
+// equal cost, the same for every workgroup, so that P - |k| is uniform and the
+// whole of an output unrolled.  A list of single products, read from LDS for each
+// (36 KB per wave vector at order 8, now 22 KB) with five instructions on its
+// address and parity, took 507 us on 64^3 cells; this 181.  Bound by LDS reads
+// (about 75 us) and by the conversions to FP64, at four waves per SIMD (the LDS).
+struct Mg2lSum {
+    double ar, ai;
+    float tr, ti;
+};
+
+// The runs of an output from the N-th of length R + 1 on, r = P - |k|: r - R + 1
+// of each length; Q products are done.  `at`: the output's first word of runs.
+template <int r, int R, int N, int Q>
+__device__ __forceinline__ void mg2l_runs(const float2 (*Mh)[MM_QB], const float (*Dq)[MM_QB], uint32_t rows, int at, int lane,
+                                          Mg2lSum& s) {
+    if constexpr (N <= r - R) {
+        constexpr int n = (r - R) * (r - R + 1) / 2 + N;  // runs done
+        const uint32_t w = (uint32_t)__builtin_amdgcn_readlane(rows, at + n / 2) >> 16 * (n & 1);
+        const float2* m = &Mh[w & 255u][lane];
+        const float* d = &Dq[w >> 8 & 255u][lane];
+        float2 mv[R + 1];
+        float dv[R + 1];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            mv[u] = *(const float2*)(mb + (w[u] & 0x7f80u));
-            d[u] = *(const float*)(db + ((w[u] >> 22) << 6));
+        for (int u = 0; u <= R; ++u) {
+            mv[u] = m[u * MM_QB];
+            dv[u] = d[u * MM_QB];
         }
-        float tr = 0.0f, ti = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            tr = fmaf(mv[u].x, d[u], tr);
-            ti = fmaf(mv[u].y, d[u], ti);
-        }
-        const uint32_t f = g.w;
-        if (f & G_ODD) {
-            br += (double)tr;
-            bi += (double)ti;
-        } else {
-            ar += (double)tr;
-            ai += (double)ti;
-        }
-        if (f & (G_SAVE | G_FLUSH)) {
-            double lr = ar - bi, li = ai + br;
-            ar = ai = br = bi = 0.0;
-            if (f & G_SAVE) {
-                er = lr;
-                ei = li;
-                lr = li = 0.0;
+        for (int p = 0; p < 2 * R + 1; ++p) {  // m_u d_u, then -m_u d_(u+1)
+            const float e = p & 1 ? -dv[p / 2 + 1] : dv[p / 2];
+            if (((Q + p) & 3) == 0) {
+                s.tr = mv[p / 2].x * e;
+                s.ti = mv[p / 2].y * e;
+            } else {
+                s.tr = fmaf(mv[p / 2].x, e, s.tr);
+                s.ti = fmaf(mv[p / 2].y, e, s.ti);
             }
-            if (f & G_FLUSH)  // L_2j + i L_2j+1
-                Zl[(size_t)((f >> 15) & 127) * n3 + q0 + qq] = make_float2((float)(er - li), (float)(ei + lr));
+            if (((Q + p) & 3) == 3) {
+                s.ar += (double)s.tr;
+                s.ai += (double)s.ti;
+            }
+        }
+        mg2l_runs<r, R, N + 1, Q + 2 * R + 1>(Mh, Dq, rows, at, lane, s);
+    } else if constexpr (R > 0) {
+        mg2l_runs<r, R - 1, 0, Q>(Mh, Dq, rows, at, lane, s);
+    } else if constexpr (Q & 3) {
+        s.ar += (double)s.tr;
+        s.ai += (double)s.ti;
+    }
+}
+
+// v i^d, d uniform
+__device__ __forceinline__ float2 turn(float2 v, uint32_t d) {
+    const float x = d & 1 ? v.y : v.x, y = d & 1 ? v.x : v.y;
+    return make_float2(__uint_as_float(__float_as_uint(x) ^ (d + 1 & 2) << 30), __uint_as_float(__float_as_uint(y) ^ (d & 2) << 30));
+}
+
+// PMAX: room for expansions up to that order; WAVES work lists.  At PMAX = 8 one
+// workgroup fills a CU's LDS, so the workgroups are persistent and hold the next
+// block's reads in registers while they work on this one.
+template <int PMAX, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void mm_mg2l(const float2* __restrict__ Zm, const float* __restrict__ Dt32,
+                                                      const uint32_t* __restrict__ sched, int nc, int K, int nz,
+                                                      float2* __restrict__ Zl) {
+    constexpr int KMAX = (PMAX + 1) * (PMAX + 2) * (PMAX + 3) / 6;
+    constexpr int NZ = ((KMAX + 1) / 2 + WAVES - 1) / WAVES, ND = (KMAX + WAVES - 1) / WAVES;
+    __shared__ float2 Mh[KMAX][MM_QB];
+    __shared__ float Dq[KMAX][MM_QB];
+    const int n3 = nc * nc * nc, blocks = n3 / MM_QB, m = nc - 1, lg = __ffs(nc) - 1;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t* list = sched + wave * MG2L_LIST;
+    uint32_t outs = list[lane], rows = list[MG2L_STEPS + lane], stage = list[2 * MG2L_STEPS + lane];
+    // here, so that no wait for them stands between the reads below and their use
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(outs), "+v"(rows), "+v"(stage));
+    const int count = (int)__builtin_amdgcn_readlane(stage, 63);
+    float2 za[NZ], zb[NZ];
+    float dv[ND];
+    const auto fetch = [&](int block) {
+        const int q = block * MM_QB + lane;
+        const int qn = ((-(q >> 2 * lg) & m) << 2 * lg) | ((-(q >> lg) & m) << lg) | (-q & m);
+#pragma unroll
+        for (int i = 0; i < NZ; ++i) {
+            const int j = min(wave + WAVES * i, nz - 1);
+            za[i] = Zm[(size_t)j * n3 + q];
+            zb[i] = Zm[(size_t)j * n3 + qn];
+        }
+#pragma unroll
+        for (int i = 0; i < ND; ++i) dv[i] = Dt32[(size_t)min(wave + WAVES * i, K - 1) * n3 + q];
+    };
+    fetch(blockIdx.x);
+    for (int block = blockIdx.x; block < blocks; block += gridDim.x) {
+        __syncthreads();  // the block before is done with the LDS
+#pragma unroll
+        for (int i = 0; i < NZ; ++i) {
+            const int j = wave + WAVES * i;
+            if (j >= nz) break;
+            const uint32_t s = __builtin_amdgcn_readlane(stage, i);  // rows and degrees of the components 2j, 2j + 1
+            const float2 a = za[i], b = zb[i];
+            // (Z(q) + conj Z(-q)) / 2 and / 2i
+            Mh[s & 255u][lane] = turn(make_float2(0.5f * (a.x + b.x), 0.5f * (a.y - b.y)), s >> 16);
+            if (2 * j + 1 < K)
+                Mh[s >> 8 & 255u][lane] = turn(make_float2(0.5f * (a.y + b.y), 0.5f * (b.x - a.x)), s >> 24);
+        }
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            if (wave + WAVES * i >= K) break;
+            const uint32_t s = __builtin_amdgcn_readlane(stage, 16 + i);  // row and sign of a table component
+            Dq[s & 255u][lane] = __uint_as_float(__float_as_uint(dv[i]) ^ (s & 0x80000000u));
+        }
+        __syncthreads();
+        if (block + (int)gridDim.x < blocks) fetch(block + gridDim.x);
+        for (int i = 0, at = 0; i < count; ++i) {
+            const uint32_t w = __builtin_amdgcn_readlane(outs, i);
+            const int r = (int)(w & 15u);
+            Mg2lSum s{0.0, 0.0, 0.0f, 0.0f};
+            switch (r) {
+#define CT2_MM_OUT(R) \
+    case R: \
+        if constexpr (R <= PMAX) mg2l_runs<R, R, 0, 0>(Mh, Dq, rows, at, lane, s); \
+        break;
+                CT2_MM_OUT(1) CT2_MM_OUT(2) CT2_MM_OUT(3) CT2_MM_OUT(4) CT2_MM_OUT(5) CT2_MM_OUT(6) CT2_MM_OUT(7) CT2_MM_OUT(8)
+#undef CT2_MM_OUT
+                default: {  // S_a and S_b of two components of degree P; the second maybe absent
+                    const uint32_t c = __builtin_amdgcn_readlane(rows, at);
+                    const float2 m0 = Mh[0][lane];
+                    const float da = Dq[c & 255u][lane], db = (c >> 8) == MG2L_NONE ? 0.0f : Dq[c >> 8][lane];
+                    s.ar = m0.x * da - m0.y * db;
+                    s.ai = m0.y * da + m0.x * db;
+                }
+            }
+            at += r ? ((r + 1) * (r + 2) / 2 + 1) / 2 : 1;
+            Zl[(size_t)(w >> 4 & 127u) * n3 + block * MM_QB + lane] = turn(make_float2((float)s.ar, (float)s.ai), w >> 11);
         }
     }
 }
@@ -702,8 +766,8 @@ __global__ __launch_bounds__(64 * MM_WAVES) void mm_near_l2p(const uint4* __rest
                 for (int hb = 0; hb < 2; ++hb) {
                     const int c = 2 * (j0 + j) + hb;
                     if (c >= K) continue;
-                    const float L = (hb ? zc[j].y : zc[j].x) * c_ifact[c];
-                    const int a = c_e[c][0], b = c_e[c][1], d = c_e[c][2];
+                    const float L = (hb ? zc[j].y : zc[j].x) * c_lifact[c];
+                    const int a = c_le[c][0], b = c_le[c][1], d = c_le[c][2];
                     phi = fmaf(L, pa[a] * pb[b] * pc[d], phi);
                     if (a) gx = fmaf(L * (float)a, pa[a - 1] * pb[b] * pc[d], gx);
                     if (b) gy = fmaf(L * (float)b, pa[a] * pb[b - 1] * pc[d], gy);
@@ -768,7 +832,15 @@ int mm_forces() {
     mm_p2m<<<(unsigned)(n3 / MM_P2M_CELLS), 256, 0, st>>>(s.Ps, s.start, lg, s.P, s.K, (size_t)n3, s.Zm);
     CT2_LAUNCH_CHECK();
     CT2_TRY(fft3d_batch(s.Zm, nc, 1, false, s.nz));
-    mm_mg2l<<<(unsigned)(n3 / MM_QB), 256, 0, st>>>(s.Zm, s.Dt32, s.sched, nc, s.K, s.nz, s.slen, s.Zl);
+#define CT2_MM_MG2L(PMAX, WAVES) \
+    mm_mg2l<PMAX, WAVES><<<(unsigned)std::min(n3 / MM_QB, 256 * (16 / WAVES)), 64 * WAVES, 0, st>>>(s.Zm, s.Dt32, s.sched, nc, s.K, s.nz, s.Zl)
+    if (s.P <= 4)
+        CT2_MM_MG2L(4, 4);
+    else if (s.P <= 6)
+        CT2_MM_MG2L(6, 8);
+    else
+        CT2_MM_MG2L(MM_PMAX, 16);
+#undef CT2_MM_MG2L
     CT2_LAUNCH_CHECK();
     CT2_TRY(fft3d_batch(s.Zl, nc, -1, false, s.nz));
     // near pairs + L2P
@@ -831,46 +903,88 @@ extern "C" int ct2_mm_init(int nc, int order) {
     MMState& s = g_mm;
     hipStream_t st = c.stream;
     s.nc = 0;  // unusable until the table is complete
-    // the MG2L lists: per component, its products split by the parity of |n|
-    // into groups of four (padded), grouped by component pair (2j, 2j+1); the
-    // pairs spread over MM_SLOTS lists by descending length (each to the
-    // shortest list), padded with empty groups to equal length
     const int nz = (I.K + 1) / 2;
-    std::vector<std::vector<uint32_t>> byj(nz);
-    for (int k = 0; k < I.K; ++k) {
-        std::vector<uint32_t>& out = byj[k >> 1];
-        for (int odd = 0; odd < 2; ++odd) {
-            std::vector<uint32_t> grp;
-            for (size_t p = 0; p < I.pa.size(); ++p)
-                if (I.pa[p] == k && (I.deg(I.pc[p]) & 1) == odd) grp.push_back(mg2l_entry(I.pb[p], I.pc[p], k >> 1, 0));
-            if (grp.empty()) continue;
-            while (grp.size() % 4) grp.push_back(mg2l_entry(0, I.K, k >> 1, 0));
-            for (size_t g = 3; g < grp.size(); g += 4) grp[g] |= odd ? G_ODD : 0u;
-            out.insert(out.end(), grp.begin(), grp.end());
+    // column order: the components of one (a, b) in a row, by z exponent
+    int col[MM_PMAX + 1][MM_PMAX + 1], row[MM_KMAX] = {}, rows = 0;
+    for (int e = 0; e <= order; ++e)
+        for (int a = e; a >= 0; --a) {
+            col[a][e - a] = rows;
+            for (int z = 0; z <= order - e; ++z) row[I.id[a][e - a][z]] = rows++;
         }
-        if (!(k & 1)) out.back() |= G_SAVE;  // the end of the even component
+    // the MG2L outputs: pairs of z exponents (kz, kz + 1), with a run for every
+    // (lx, ly), then the highest exponents left over (degree P) two by two; a
+    // list per wave, each output to the shortest list, the longest first
+    struct Output {
+        uint32_t head;
+        std::vector<uint32_t> runs;
+        int cost;
+    };
+    std::vector<Output> outs;
+    std::vector<int> lcomp, single;  // components in the order of the local grids
+    for (int e = 0; e <= order; ++e)
+        for (int a = e; a >= 0; --a) {
+            const int b = e - a;
+            for (int kz = 0; kz + 1 <= order - e; kz += 2) {
+                const int r = order - e - kz;
+                Output o{(uint32_t)r | (uint32_t)outs.size() << 4 | (uint32_t)(e + kz) << 11, {}, 40};
+                for (int le = 0, n = 0; le <= r; ++le)
+                    for (int la = le; la >= 0; --la, ++n) {
+                        const uint32_t w = mg2l_rows(col[la][le - la], col[a + la][b + le - la] + kz);
+                        if (n & 1)
+                            o.runs.back() |= w << 16;
+                        else
+                            o.runs.push_back(w);
+                        o.cost += 10 * (r - le) + 15;  // about its share of the time
+                    }
+                outs.push_back(o);
+                lcomp.push_back(I.id[a][b][kz]);
+                lcomp.push_back(I.id[a][b][kz + 1]);
+            }
+            if ((order - e) % 2 == 0) single.push_back(I.id[a][b][order - e]);
+        }
+    for (size_t k = 0; k < single.size(); k += 2) {
+        const bool both = k + 1 < single.size();
+        outs.push_back({(uint32_t)outs.size() << 4 | (uint32_t)order << 11,
+                        {mg2l_rows(row[single[k]], both ? row[single[k + 1]] : (int)MG2L_NONE)}, 60});
+        lcomp.push_back(single[k]);
+        if (both) lcomp.push_back(single[k + 1]);
     }
-    for (int j = 0; j < nz; ++j) byj[j].back() |= G_FLUSH;
-    std::vector<int> jorder(nz);
-    for (int j = 0; j < nz; ++j) jorder[j] = j;
-    std::stable_sort(jorder.begin(), jorder.end(), [&](int a, int b) { return byj[a].size() > byj[b].size(); });
-    std::vector<std::vector<uint32_t>> lists(MM_SLOTS);
-    for (int j : jorder) {
-        auto it = std::min_element(lists.begin(), lists.end(),
-                                   [](const std::vector<uint32_t>& a, const std::vector<uint32_t>& b) { return a.size() < b.size(); });
-        it->insert(it->end(), byj[j].begin(), byj[j].end());
+    if ((int)outs.size() != nz || (int)lcomp.size() != I.K)
+        return set_error(CT2_ERR_STATE, "MG2L outputs do not cover the %d components", I.K);
+    const int waves = order <= 4 ? 4 : order <= 6 ? 8 : 16;
+    std::stable_sort(outs.begin(), outs.end(), [](const Output& x, const Output& y) { return x.cost > y.cost; });
+    std::vector<uint32_t> sched((size_t)waves * MG2L_LIST, 0u);
+    std::vector<int> load(waves, 0), count(waves, 0);
+    std::vector<size_t> words(waves, 0);
+    for (const Output& o : outs) {
+        const int w = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+        if (count[w] == MG2L_STEPS || words[w] + o.runs.size() > MG2L_STEPS)
+            return set_error(CT2_ERR_STATE, "MG2L list longer than %d words", MG2L_STEPS);
+        uint32_t* list = sched.data() + (size_t)w * MG2L_LIST;
+        list[count[w]++] = o.head;
+        std::copy(o.runs.begin(), o.runs.end(), list + MG2L_STEPS + words[w]);
+        words[w] += o.runs.size();
+        load[w] += o.cost;
     }
-    size_t slen = 0;
-    for (auto& l : lists) slen = std::max(slen, l.size());
-    if (slen > (size_t)MM_SCHED_MAX) return set_error(CT2_ERR_INVALID, "MG2L list of %zu entries exceeds %d", slen, MM_SCHED_MAX);
-    const size_t sstride = (size_t)mg2l_stride((int)slen);
-    std::vector<uint32_t> sched((size_t)MM_SLOTS * sstride, mg2l_entry(0, I.K, 0, 0));
-    for (int sl = 0; sl < MM_SLOTS; ++sl) std::copy(lists[sl].begin(), lists[sl].end(), sched.begin() + (size_t)sl * sstride);
-    int ce[MM_KMAX][3] = {};
-    float cf[MM_KMAX] = {};
+    const auto degree = [&](int c) { return (uint32_t)(I.e[c][0] + I.e[c][1] + I.e[c][2]); };
+    for (int w = 0; w < waves; ++w) {
+        uint32_t* stage = sched.data() + (size_t)w * MG2L_LIST + 2 * MG2L_STEPS;
+        for (int i = 0, j = w; j < nz; ++i, j += waves) {
+            stage[i] = (uint32_t)row[2 * j] | degree(2 * j) << 16;
+            if (2 * j + 1 < I.K) stage[i] |= (uint32_t)row[2 * j + 1] << 8 | degree(2 * j + 1) << 24;
+        }
+        for (int i = 16, c = w; c < I.K; ++i, c += waves) stage[i] = (uint32_t)row[c] | (degree(c) & 2u) << 30;
+        stage[MG2L_STEPS - 1] = (uint32_t)count[w];
+    }
+    int ce[MM_KMAX][3] = {}, cle[MM_KMAX][3] = {};
+    float cf[MM_KMAX] = {}, clf[MM_KMAX] = {};
     for (int k = 0; k < I.K; ++k) {
-        for (int q = 0; q < 3; ++q) ce[k][q] = I.e[k][q];
+        for (int q = 0; q < 3; ++q) {
+            ce[k][q] = I.e[k][q];
+            cle[k][q] = I.e[lcomp[k]][q];
+        }
         cf[k] = (float)(1.0 / I.fact[k]);
+        clf[k] = (float)(1.0 / I.fact[lcomp[k]]);
     }
     // the near set |offset|^2 <= 10 as columns: (dx, dy) with dz in [-w, w]
     int cn[MM_COLS_MAX][3] = {};
@@ -887,6 +1001,8 @@ extern "C" int ct2_mm_init(int nc, int order) {
             }
     CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_e), ce, sizeof ce, 0, hipMemcpyHostToDevice, st));
     CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_ifact), cf, sizeof cf, 0, hipMemcpyHostToDevice, st));
+    CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_le), cle, sizeof cle, 0, hipMemcpyHostToDevice, st));
+    CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_lifact), clf, sizeof clf, 0, hipMemcpyHostToDevice, st));
     CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_cols), cn, sizeof cn, 0, hipMemcpyHostToDevice, st));
     // buffers
     CT2_TRY(ensure_scratch((void**)&s.sched, &s.sched_bytes, sizeof(uint32_t) * sched.size(), "MG2L lists"));
@@ -918,7 +1034,6 @@ extern "C" int ct2_mm_init(int nc, int order) {
     s.P = order;
     s.K = I.K;
     s.nz = nz;
-    s.slen = (int)slen;
     s.ncols = ncols;
     return CT2_OK;
 }

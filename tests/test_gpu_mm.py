@@ -63,6 +63,30 @@ def test_forces_vs_oracle(ct2, orc, nc, order, clustered):
     assert np.max(np.abs(pot - op)) < 1e-5 * np.abs(op).max()  # the periodic potential crosses zero
 
 
+@pytest.mark.parametrize("nc,order", [(8, 2), (8, 3), (16, 5), (16, 7)])
+def test_orders_and_cells_of_several_passes(ct2, orc, nc, order):
+    """The orders between those above (odd numbers of components, every length of
+    MG2L run), with cells of 15, 16, 17, 32, 33 and 70 particles among sparse
+    ones: P2M takes 16 particles of a cell per pass.  Bounds as above."""
+    x, y, z = random_set(600, order)
+    rng = np.random.default_rng(order + 1)
+    for i, k in enumerate((15, 16, 17, 32, 33, 70)):
+        c = np.array([i, (3 * i + 1) % nc, (nc - 1 + i) % nc])
+        p = (c + rng.random((k, 3))) / nc
+        x, y, z = (np.concatenate([u, to_fixed(p[:, q])]) for q, u in enumerate((x, y, z)))
+    n = len(x)
+    gm, soft = float(np.float32(1.0 / n)), float(np.float32(2e-3))
+    ct2.particle_allocate(n)
+    ct2.particles_upload(x, y, z)
+    ct2.set_force_options(soft, gm, ct2.KERNEL_PLUMMER)
+    ct2.mm_init(nc, order)
+    fx, fy, fz, pot = ct2.mm_forces()
+    ox, oy, oz, op = orc.mm_forces(x, y, z, nc, order, gm, soft)
+    e = rel_err(np.stack([fx, fy, fz]), np.stack([ox, oy, oz]))
+    assert np.median(e) < 3e-6 and np.percentile(e, 99) < 5e-5, (np.median(e), e.max())
+    assert np.max(np.abs(pot - op)) < 1e-5 * np.abs(op).max()
+
+
 def test_ct2_kernel_and_empty_cells(ct2, orc):
     """ct2's uniform-sphere kernel (kick.cpp:52-60) in the direct pairs, a
     16^3 grid with most cells empty, and particles on cell faces."""
