@@ -38,6 +38,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "epilogue.h"
+#include "fft_stages.h"
 #include "internal.h"
 
 namespace ct2 {
@@ -63,8 +64,6 @@ constexpr uint32_t mg2l_rows(int m, int d) { return (uint32_t)m | (uint32_t)d <<
 
 __constant__ int c_e[MM_KMAX][3];         // exponents of component c
 __constant__ float c_ifact[MM_KMAX];      // 1 / (a! b! c!)
-__constant__ int c_le[MM_KMAX][3];        // exponents of the local expansions, in the order of their grids
-__constant__ float c_lifact[MM_KMAX];
 __constant__ int c_cols[MM_COLS_MAX][3];  // near set by column: dx, dy, half-height w in z
 
 struct MMIndex {
@@ -132,6 +131,8 @@ struct MMState {
     size_t tabz_bytes = 0;
     uint32_t* sched = nullptr;  // the MG2L lists [waves][MG2L_LIST]
     size_t sched_bytes = 0;
+    float4* far = nullptr;  // far field per sorted particle, where Zm is too small for it
+    size_t far_bytes = 0;
 };
 MMState g_mm;
 
@@ -579,7 +580,90 @@ __global__ __launch_bounds__(64 * WAVES) void mm_mg2l(const float2* __restrict__
     }
 }
 
-// ------------------------------------------------------------ near pairs + L2P
+// ------------------------------------------------------------ L2P
+
+// Where the local expansion's components lie: pairs of z exponents (d, d + 1), d
+// even, column by column, then the highest exponents left over two by two.
+template <int P>
+struct LocalGrids {
+    int pair[P + 1][P + 1] = {};    // grid of a column's first pair
+    int single[P + 1][P + 1] = {};  // rank of a column's left-over component
+    int pairs = 0;
+    constexpr LocalGrids() {
+        int n = 0;
+        for (int e = 0; e <= P; ++e)
+            for (int a = e; a >= 0; --a) {
+                pair[a][e - a] = pairs;
+                pairs += (P - e + 1) / 2;
+                if ((P - e) % 2 == 0) single[a][e - a] = n++;
+            }
+    }
+};
+
+// The local expansion of a particle's cell at its offset from the centre, one
+// thread per particle in cell order: (d/dx, d/dy, d/dz) and the value, in cells.
+// Columns of z exponents by powers over factorials, so that a component costs two
+// multiply-adds, with every exponent a constant (order 8: 0.5 k instructions per
+// particle; by components with exponents read from a table, behind the near
+// pairs, it took 5 k and 220 us of 2^21 particles on 64^3 cells, this 95).
+// Bound by reading the grids once.
+template <int P>
+__global__ __launch_bounds__(256) void mm_l2p(const uint4* __restrict__ Ps, const float2* __restrict__ Zl, int n, int lg,
+                                              float4* __restrict__ far) {
+    static constexpr LocalGrids<P> G{};
+    const int i = (int)xcd_contiguous(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    if (i >= n) return;
+    const uint4 me = Ps[i];
+    const int sh = 32 - lg;
+    const uint32_t half = 1u << (sh - 1), low = (1u << sh) - 1u;
+    const size_t n3 = (size_t)1 << 3 * lg;
+    const float2* z = Zl + (((size_t)(me.x >> sh) << 2 * lg) | ((size_t)(me.y >> sh) << lg) | (size_t)(me.z >> sh));
+    const float inv = ldexpf(1.0f, -sh);
+    float px[P + 1], py[P + 1], pz[P + 1];
+    px[0] = py[0] = pz[0] = 1.0f;
+    const float ax = (float)(int32_t)((me.x & low) - half) * inv, ay = (float)(int32_t)((me.y & low) - half) * inv,
+                az = (float)(int32_t)((me.z & low) - half) * inv;
+#pragma unroll
+    for (int e = 1; e <= P; ++e) {
+        px[e] = px[e - 1] * ax * (1.0f / e);
+        py[e] = py[e - 1] * ay * (1.0f / e);
+        pz[e] = pz[e - 1] * az * (1.0f / e);
+    }
+    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int a = 0; a <= P; ++a) {
+        float v = 0.f, vy = 0.f, vz = 0.f;
+#pragma unroll
+        for (int b = 0; b <= P; ++b) {
+            if (a + b > P) continue;
+            const int top = P - a - b;
+            float f = 0.f, fz = 0.f;
+#pragma unroll
+            for (int d = 0; d <= P; d += 2) {
+                if (d > top) continue;
+                const int s = G.single[a][b];
+                float2 L = z[(size_t)(d < top ? G.pair[a][b] + d / 2 : G.pairs + s / 2) * n3];
+                if (d == top && s % 2) L.x = L.y;
+                f = fmaf(L.x, pz[d], f);
+                if (d) fz = fmaf(L.x, pz[d - 1], fz);
+                if (d < top) {
+                    f = fmaf(L.y, pz[d + 1], f);
+                    fz = fmaf(L.y, pz[d], fz);
+                }
+            }
+            v = fmaf(f, py[b], v);
+            vz = fmaf(fz, py[b], vz);
+            if (b) vy = fmaf(f, py[b - 1], vy);
+        }
+        g.w = fmaf(v, px[a], g.w);
+        g.y = fmaf(vy, px[a], g.y);
+        g.z = fmaf(vz, px[a], g.z);
+        if (a) g.x = fmaf(v, px[a - 1], g.x);
+    }
+    far[i] = g;
+}
+
+// ------------------------------------------------------------ near pairs
 
 struct NearK {
     float eps2u, h2u, hinvu, hinv3u;  // as the direct kick, in 2^-32 units
@@ -623,9 +707,6 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 constexpr int MM_STAGE = 256;  // sources per wave staged in LDS at a time
-#ifndef MM_L2P_CHUNK
-#define MM_L2P_CHUNK 4  // local-expansion grids read ahead at a time by L2P
-#endif
 #ifndef MM_NEAR_UNROLL
 #define MM_NEAR_UNROLL 4  // sources per step of a lane's run (LDS reads in flight)
 #endif
@@ -643,20 +724,18 @@ constexpr int MM_STAGE = 256;  // sources per wave staged in LDS at a time
 // every axis).  EXACT path (8^3 cells, where the window can cover the whole
 // column and a sink's run wrap inside it): every lane walks the window and
 // takes the sources within w of its own cell, with separations from the
-// fixed-point positions.  Each column's sum is folded in with TwoSum; then
-// the local expansion of the sink's cell.
+// fixed-point positions.  Each column's sum is folded in with TwoSum; then the
+// far field of the slot is added.
 template <int KERNEL, bool EXACT>
-__global__ __launch_bounds__(64 * MM_WAVES) void mm_near_l2p(const uint4* __restrict__ P, const int* __restrict__ start,
-                                                             const int* __restrict__ items, const int* __restrict__ nitems,
-                                                             const float2* __restrict__ Zl, int lg, int Pord, int K,
-                                                             int ncols, NearK kc, double fnear, double pnear,
-                                                             double ffar, double pfar, float* __restrict__ fx,
-                                                             float* __restrict__ fy, float* __restrict__ fz,
-                                                             float* __restrict__ pot) {
+__global__ __launch_bounds__(64 * MM_WAVES) void mm_near(const uint4* __restrict__ P, const int* __restrict__ start,
+                                                         const int* __restrict__ items, const int* __restrict__ nitems,
+                                                         const float4* __restrict__ far, int lg, int ncols, NearK kc,
+                                                         double fnear, double pnear, double ffar, double pfar,
+                                                         float* __restrict__ fx, float* __restrict__ fy,
+                                                         float* __restrict__ fz, float* __restrict__ pot) {
     __shared__ uint4 S[MM_WAVES][MM_STAGE];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int nc = 1 << lg, sh = 32 - lg, m = nc - 1;
-    const size_t n3 = (size_t)nc * nc * nc;
     const uint32_t half = 1u << (sh - 1);
     const int total = *nitems;
     for (int item = blockIdx.x * MM_WAVES + w; item < total; item += gridDim.x * MM_WAVES) {
@@ -739,48 +818,13 @@ __global__ __launch_bounds__(64 * MM_WAVES) void mm_near_l2p(const uint4* __rest
             two_sum_f(sz, czs, tz);
             two_sum_f(sp, cps, tp);
         }
-        // the local expansion of the sink's own cell at a = offset from its centre, in cells
-        const size_t cell = ((size_t)row << lg) | (size_t)zs;
-        const float inv = ldexpf(1.0f, -sh);
-        const float ax = (float)(int32_t)(me.x - rx) * inv, ay = (float)(int32_t)(me.y - ry) * inv,
-                    az = (float)(int32_t)(me.z - (((uint32_t)zs << sh) + half)) * inv;
-        float pa[MM_PMAX + 1], pb[MM_PMAX + 1], pc[MM_PMAX + 1];
-        pa[0] = pb[0] = pc[0] = 1.0f;
-        for (int e = 1; e <= Pord; ++e) {
-            pa[e] = pa[e - 1] * ax;
-            pb[e] = pb[e - 1] * ay;
-            pc[e] = pc[e - 1] * az;
-        }
-        float phi = 0.f, gx = 0.f, gy = 0.f, gz = 0.f;
-        // the component pairs (grids) read MM_L2P_CHUNK at a time, all in flight
-        // together, instead of one load per component on the critical path
-        const int nzg = (K + 1) >> 1;
-        for (int j0 = 0; j0 < nzg; j0 += MM_L2P_CHUNK) {
-            float2 zc[MM_L2P_CHUNK];
-#pragma unroll
-            for (int j = 0; j < MM_L2P_CHUNK; ++j)
-                if (j0 + j < nzg) zc[j] = Zl[(size_t)(j0 + j) * n3 + cell];
-#pragma unroll
-            for (int j = 0; j < MM_L2P_CHUNK; ++j) {
-#pragma unroll
-                for (int hb = 0; hb < 2; ++hb) {
-                    const int c = 2 * (j0 + j) + hb;
-                    if (c >= K) continue;
-                    const float L = (hb ? zc[j].y : zc[j].x) * c_lifact[c];
-                    const int a = c_le[c][0], b = c_le[c][1], d = c_le[c][2];
-                    phi = fmaf(L, pa[a] * pb[b] * pc[d], phi);
-                    if (a) gx = fmaf(L * (float)a, pa[a - 1] * pb[b] * pc[d], gx);
-                    if (b) gy = fmaf(L * (float)b, pa[a] * pb[b - 1] * pc[d], gy);
-                    if (d) gz = fmaf(L * (float)d, pa[a] * pb[b] * pc[d - 1], gz);
-                }
-            }
-        }
         if (live) {
             const uint32_t i = me.w;
-            fx[i] = (float)(((double)sx + (double)cxs) * fnear + (double)gx * ffar);
-            fy[i] = (float)(((double)sy + (double)cys) * fnear + (double)gy * ffar);
-            fz[i] = (float)(((double)sz + (double)czs) * fnear + (double)gz * ffar);
-            pot[i] = (float)(((double)sp + (double)cps) * pnear + (double)phi * pfar);
+            const float4 g = far[first + lane];
+            fx[i] = (float)(((double)sx + (double)cxs) * fnear + (double)g.x * ffar);
+            fy[i] = (float)(((double)sy + (double)cys) * fnear + (double)g.y * ffar);
+            fz[i] = (float)(((double)sz + (double)czs) * fnear + (double)g.z * ffar);
+            pot[i] = (float)(((double)sp + (double)cps) * pnear + (double)g.w * pfar);
         }
     }
 }
@@ -843,7 +887,21 @@ int mm_forces() {
 #undef CT2_MM_MG2L
     CT2_LAUNCH_CHECK();
     CT2_TRY(fft3d_batch(s.Zl, nc, -1, false, s.nz));
-    // near pairs + L2P
+    // L2P into the multipole grids, which the transforms are done with, where they hold every particle
+    float4* far = (float4*)s.Zm;
+    if (sizeof(float4) * (size_t)n > s.Z_bytes) {
+        CT2_TRY(ensure_scratch((void**)&s.far, &s.far_bytes, sizeof(float4) * (size_t)n, "far field"));
+        far = s.far;
+    }
+    switch (s.P) {
+#define CT2_MM_L2P(P) \
+    case P: mm_l2p<P><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(s.Ps, s.Zl, (int)n, lg, far); break;
+        CT2_MM_L2P(1) CT2_MM_L2P(2) CT2_MM_L2P(3) CT2_MM_L2P(4) CT2_MM_L2P(5) CT2_MM_L2P(6) CT2_MM_L2P(7)
+        default: mm_l2p<MM_PMAX><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(s.Ps, s.Zl, (int)n, lg, far);
+#undef CT2_MM_L2P
+    }
+    CT2_LAUNCH_CHECK();
+    // near pairs
     const double two32 = 4294967296.0, h = c.opts.hsoft, hu = h * two32, gm = c.opts.GM;
     NearK kc;
     kc.eps2u = (float)(hu * hu);
@@ -858,8 +916,8 @@ int mm_forces() {
     const unsigned grid = (unsigned)std::min<size_t>(65535, (max_items + MM_WAVES - 1) / MM_WAVES);
     const bool plummer = c.opts.kernel == CT2_KERNEL_PLUMMER, exact = nc < 16;
 #define CT2_MM_NEAR(KER, EX)                                                                                    \
-    mm_near_l2p<KER, EX><<<grid, 64 * MM_WAVES, 0, st>>>(s.Ps, s.start, s.items, s.nitems, s.Zl, lg, s.P, s.K, \
-                                                         s.ncols, kc, fnear, pnear, ffar, pfar, c.fx, c.fy, c.fz, c.pot)
+    mm_near<KER, EX><<<grid, 64 * MM_WAVES, 0, st>>>(s.Ps, s.start, s.items, s.nitems, far, lg, s.ncols, kc, fnear, pnear, \
+                                                     ffar, pfar, c.fx, c.fy, c.fz, c.pot)
     if (plummer && exact)
         CT2_MM_NEAR(CT2_KERNEL_PLUMMER, true);
     else if (plummer)
@@ -879,7 +937,7 @@ int mm_forces() {
 void release_mm() {
     MMState& s = g_mm;
     for (void* p : {(void*)s.Dt, (void*)s.Dt32, (void*)s.Zm, (void*)s.Zl, (void*)s.keys, s.sort_tmp, (void*)s.Ps, (void*)s.start,
-                    (void*)s.items, (void*)s.cnt, s.scan_tmp, (void*)s.tabz, (void*)s.sched})
+                    (void*)s.items, (void*)s.cnt, s.scan_tmp, (void*)s.tabz, (void*)s.sched, (void*)s.far})
         dev_free(p);
     s = MMState();
 }
@@ -920,7 +978,7 @@ extern "C" int ct2_mm_init(int nc, int order) {
         int cost;
     };
     std::vector<Output> outs;
-    std::vector<int> lcomp, single;  // components in the order of the local grids
+    std::vector<int> single;  // grids in LocalGrids' order
     for (int e = 0; e <= order; ++e)
         for (int a = e; a >= 0; --a) {
             const int b = e - a;
@@ -937,8 +995,6 @@ extern "C" int ct2_mm_init(int nc, int order) {
                         o.cost += 10 * (r - le) + 15;  // about its share of the time
                     }
                 outs.push_back(o);
-                lcomp.push_back(I.id[a][b][kz]);
-                lcomp.push_back(I.id[a][b][kz + 1]);
             }
             if ((order - e) % 2 == 0) single.push_back(I.id[a][b][order - e]);
         }
@@ -946,11 +1002,8 @@ extern "C" int ct2_mm_init(int nc, int order) {
         const bool both = k + 1 < single.size();
         outs.push_back({(uint32_t)outs.size() << 4 | (uint32_t)order << 11,
                         {mg2l_rows(row[single[k]], both ? row[single[k + 1]] : (int)MG2L_NONE)}, 60});
-        lcomp.push_back(single[k]);
-        if (both) lcomp.push_back(single[k + 1]);
     }
-    if ((int)outs.size() != nz || (int)lcomp.size() != I.K)
-        return set_error(CT2_ERR_STATE, "MG2L outputs do not cover the %d components", I.K);
+    if ((int)outs.size() != nz) return set_error(CT2_ERR_STATE, "%zu MG2L outputs for %d grids", outs.size(), nz);
     const int waves = order <= 4 ? 4 : order <= 6 ? 8 : 16;
     std::stable_sort(outs.begin(), outs.end(), [](const Output& x, const Output& y) { return x.cost > y.cost; });
     std::vector<uint32_t> sched((size_t)waves * MG2L_LIST, 0u);
@@ -976,15 +1029,11 @@ extern "C" int ct2_mm_init(int nc, int order) {
         for (int i = 16, c = w; c < I.K; ++i, c += waves) stage[i] = (uint32_t)row[c] | (degree(c) & 2u) << 30;
         stage[MG2L_STEPS - 1] = (uint32_t)count[w];
     }
-    int ce[MM_KMAX][3] = {}, cle[MM_KMAX][3] = {};
-    float cf[MM_KMAX] = {}, clf[MM_KMAX] = {};
+    int ce[MM_KMAX][3] = {};
+    float cf[MM_KMAX] = {};
     for (int k = 0; k < I.K; ++k) {
-        for (int q = 0; q < 3; ++q) {
-            ce[k][q] = I.e[k][q];
-            cle[k][q] = I.e[lcomp[k]][q];
-        }
+        for (int q = 0; q < 3; ++q) ce[k][q] = I.e[k][q];
         cf[k] = (float)(1.0 / I.fact[k]);
-        clf[k] = (float)(1.0 / I.fact[lcomp[k]]);
     }
     // the near set |offset|^2 <= 10 as columns: (dx, dy) with dz in [-w, w]
     int cn[MM_COLS_MAX][3] = {};
@@ -1001,8 +1050,6 @@ extern "C" int ct2_mm_init(int nc, int order) {
             }
     CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_e), ce, sizeof ce, 0, hipMemcpyHostToDevice, st));
     CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_ifact), cf, sizeof cf, 0, hipMemcpyHostToDevice, st));
-    CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_le), cle, sizeof cle, 0, hipMemcpyHostToDevice, st));
-    CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_lifact), clf, sizeof clf, 0, hipMemcpyHostToDevice, st));
     CT2_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_cols), cn, sizeof cn, 0, hipMemcpyHostToDevice, st));
     // buffers
     CT2_TRY(ensure_scratch((void**)&s.sched, &s.sched_bytes, sizeof(uint32_t) * sched.size(), "MG2L lists"));
