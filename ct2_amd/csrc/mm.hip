@@ -120,10 +120,9 @@ struct MMState {
     size_t Ps_bytes = 0;
     int* start = nullptr;  // cell starts (nc^3 + 1)
     size_t start_bytes = 0;
-    int* items = nullptr;  // near-field work items (row of cells, first sink, sinks) and their count
+    int2* items = nullptr;  // near-field work items (cell, group of its sinks), then their count
     size_t items_bytes = 0;
-    int* nitems = nullptr;
-    int* cnt = nullptr;  // items per row, then the rows' first item (exclusive sum)
+    int* cnt = nullptr;  // items per cell, then the cells' first item (exclusive sum)
     size_t cnt_bytes = 0;
     void* scan_tmp = nullptr;
     size_t scan_tmp_bytes = 0;
@@ -300,49 +299,21 @@ __global__ __launch_bounds__(256) void mm_bounds(const uint32_t* __restrict__ ke
     start[c] = lo;
 }
 
-// Work items of the near-set kernel: the sorted particles of each row of
-// cells (fixed x and y cell) cut into runs of at most 64 that span fewer than
-// zspan z cells.  One thread per row walks the row's cells; pass 0 counts the
-// row's items into cnt, pass 1 writes (row, first slot, sinks) at first[row].
-__global__ __launch_bounds__(256) void mm_row_items(const int* __restrict__ start, int lg, int zspan, int pass,
-                                                    int* __restrict__ cnt, const int* __restrict__ first,
-                                                    int* __restrict__ items, int* __restrict__ nitems) {
-    const int nc = 1 << lg, rows = nc * nc;
-    const int r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= rows) return;
-    int it = pass ? first[r] : 0;
-    int f = start[r * nc], c = 0, z0 = 0;
-    for (int z = 0; z < nc; ++z) {
-        int left = start[r * nc + z + 1] - start[r * nc + z];
-        while (left > 0) {
-            if (c == 64 || (c > 0 && z - z0 >= zspan)) {
-                if (pass) {
-                    items[3 * it] = r;
-                    items[3 * it + 1] = f;
-                    items[3 * it + 2] = c;
-                }
-                ++it;
-                f += c;
-                c = 0;
-            }
-            if (c == 0) z0 = z;
-            const int t = min(left, 64 - c);
-            c += t;
-            left -= t;
-        }
-    }
-    if (c > 0) {
-        if (pass) {
-            items[3 * it] = r;
-            items[3 * it + 1] = f;
-            items[3 * it + 2] = c;
-        }
-        ++it;
-    }
-    if (!pass)
-        cnt[r] = it;
-    else if (r == rows - 1)
-        *nitems = it;
+// Near-field work items: the sinks of a cell in groups of at most MM_SINKS, as
+// even as they go, each (cell, group).  Counts, then (after their exclusive sum)
+// the items and their number.
+constexpr int MM_SINKS = 10;
+__global__ __launch_bounds__(256) void mm_item_counts(const int* __restrict__ start, int n3, int* __restrict__ cnt) {
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c < n3) cnt[c] = (start[c + 1] - start[c] + MM_SINKS - 1) / MM_SINKS;
+}
+__global__ __launch_bounds__(256) void mm_items(const int* __restrict__ cnt, const int* __restrict__ first, int n3,
+                                                int2* __restrict__ items, int* __restrict__ nitems) {
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= n3) return;
+    const int k = cnt[c], f = first[c];
+    for (int g = 0; g < k; ++g) items[f + g] = make_int2(c, g);
+    if (c == n3 - 1) *nitems = f + k;
 }
 
 // ------------------------------------------------------------ P2M
@@ -669,26 +640,19 @@ struct NearK {
     float eps2u, h2u, hinvu, hinv3u;  // as the direct kick, in 2^-32 units
 };
 
-__device__ __forceinline__ void two_sum_f(float& s, float& c, float v) {
-#pragma clang fp contract(off)
-    const float t = s + v;
-    const float bp = t - s;
-    c += (s - (t - bp)) + (v - bp);
-    s = t;
-}
-
-// The pair term of the direct set: ddx, ddy, ddz in 2^-32 box units.
+// The pair term of the direct set: ddx, ddy, ddz in 2^-32 box units; pad is 0, or
+// infinite for a lane past the last source, which makes r^2 infinite and the term 0.
 template <int KERNEL>
-__device__ __forceinline__ void near_pair(float ddx, float ddy, float ddz, const NearK& kc, float& tx, float& ty,
+__device__ __forceinline__ void near_pair(float ddx, float ddy, float ddz, float pad, const NearK& kc, float& tx, float& ty,
                                           float& tz, float& tp) {
     float k, p;
     if constexpr (KERNEL == CT2_KERNEL_PLUMMER) {
-        const float r2 = fmaf(ddz, ddz, fmaf(ddy, ddy, fmaf(ddx, ddx, kc.eps2u)));
+        const float r2 = fmaf(ddz, ddz, fmaf(ddy, ddy, fmaf(ddx, ddx, kc.eps2u + pad)));
         const float wv = __builtin_amdgcn_rsqf(r2);
         k = (wv * wv) * wv;
         p = wv;
     } else {
-        const float r2 = fmaf(ddz, ddz, fmaf(ddy, ddy, ddx * ddx));
+        const float r2 = fmaf(ddz, ddz, fmaf(ddy, ddy, fmaf(ddx, ddx, pad)));
         const bool in = r2 < kc.h2u;
         const float wv = __builtin_amdgcn_rsqf(in ? kc.h2u : r2);
         k = in ? kc.hinv3u : (wv * wv) * wv;
@@ -706,125 +670,177 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-constexpr int MM_STAGE = 256;  // sources per wave staged in LDS at a time
-#ifndef MM_NEAR_UNROLL
-#define MM_NEAR_UNROLL 4  // sources per step of a lane's run (LDS reads in flight)
-#endif
+__device__ __forceinline__ float lane_value(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
 
-// One wave per work item (up to 64 consecutive sinks of a row of cells,
-// spanning fewer than zspan z cells); a wave takes items in turn, about one
-// when the grid covers the item count.  For each (dx, dy) column of the near set (half-height w
-// in z) the sources of the column's cells z_first - w .. z_last + w (the
-// window) are staged in the wave's LDS slot in window order, up to MM_STAGE
-// at a time.  FP32 path (nc >= 16, where the window is shorter than the
-// column): a sink's own cells z - w .. z + w are one contiguous run of the
-// window, so each lane loops over exactly its run; the separations are FP32
-// offsets from the centre of the item's first cell, which are the minimum
-// image when zspan + 3.5 < nc / 2 (a near pair is less than 4 cells apart on
-// every axis).  EXACT path (8^3 cells, where the window can cover the whole
-// column and a sink's run wrap inside it): every lane walks the window and
-// takes the sources within w of its own cell, with separations from the
-// fixed-point positions.  Each column's sum is folded in with TwoSum; then the
-// far field of the slot is added.
+// One source per lane and step, NS sinks in scalar registers; the partial sums of
+// the lanes are left in red[s][16 q + ..], q the component.
+constexpr int MM_RED = 68;  // floats per row: 64 and a shift of the banks
+template <int KERNEL, bool EXACT, int NS, typename Next>
+__device__ __forceinline__ void near_sinks(uint4 own, uint32_t rx, uint32_t ry, uint32_t rz, int steps, const Next& next,
+                                           const NearK& kc, int lane, float* __restrict__ red) {
+    uint32_t ix[NS], iy[NS], iz[NS];
+    float ux[NS], uy[NS], uz[NS], t[4 * NS];
+    const float ox = (float)(int32_t)(own.x - rx), oy = (float)(int32_t)(own.y - ry), oz = (float)(int32_t)(own.z - rz);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        if constexpr (EXACT) {
+            ix[s] = __builtin_amdgcn_readlane(own.x, s);
+            iy[s] = __builtin_amdgcn_readlane(own.y, s);
+            iz[s] = __builtin_amdgcn_readlane(own.z, s);
+        } else {
+            ux[s] = lane_value(ox, s);
+            uy[s] = lane_value(oy, s);
+            uz[s] = lane_value(oz, s);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4 * NS; ++i) t[i] = 0.0f;
+    float pad1;
+    uint4 q1 = next(0, pad1);
+    for (int k = 0; k < steps; ++k) {
+        const uint4 q = q1;
+        const float pad = pad1;
+        if (k + 1 < steps) q1 = next(k + 1, pad1);
+        if constexpr (EXACT) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                near_pair<KERNEL>((float)(int32_t)(q.x - ix[s]), (float)(int32_t)(q.y - iy[s]), (float)(int32_t)(q.z - iz[s]),
+                                  pad, kc, t[s], t[NS + s], t[2 * NS + s], t[3 * NS + s]);
+        } else {
+            const float qx = (float)(int32_t)(q.x - rx), qy = (float)(int32_t)(q.y - ry), qz = (float)(int32_t)(q.z - rz);
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                near_pair<KERNEL>(qx - ux[s], qy - uy[s], qz - uz[s], pad, kc, t[s], t[NS + s], t[2 * NS + s], t[3 * NS + s]);
+        }
+    }
+    // [aL aH], [bL bH] -> [aL + aH, bL + bH], first by halves of the wave, then by rows of 16
+#pragma unroll
+    for (int i = 0; i < 2 * NS; ++i) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(t[i]), __float_as_uint(t[i + 2 * NS]), false, false);
+        t[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t[s]), __float_as_uint(t[s + NS]), false, false);
+        red[s * MM_RED + lane] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+}
+
+// One wave per work item: up to MM_SINKS sinks of a cell, which all have the same
+// sources, the particles of the near set's cells.  They are the cells z - w .. z + w
+// of the set's (dx, dy) columns, a run of consecutive slots each (one that wraps
+// through z = 0 continues a column's length lower); a lane holds a column's run,
+// and the runs joined are the item's list, 64 sources to a step, whose lane finds
+// its run from the bits of the run heads up to it.  Sources are read and taken as
+// FP32 offsets from the cell's centre once for all sinks, so that a pair costs
+// its 13 instructions, with no lane idle but in the last step; a lane sums every
+// 64th source in FP32, then the lanes are summed.  Bound by those instructions at
+// the rate that five waves per SIMD issue them: a lane per sink that walked its own
+// runs in LDS (idle for a fifth of the time, with 135 instructions per column and
+// two per pair on top, but eight waves per SIMD) took 1,109 us for 2^21 particles on
+// 64^3 cells, and two small kernels 39 us to cut the rows into its items; this takes
+// 1,063 and 7.  12 sinks took 1,081 at five waves and 1,237 at four, 9 the same at
+// six; groups of 2 to 6 sinks interleaved by hand 1,177 to 1,320.  EXACT (8^3 cells,
+// whose offsets are too coarse): separations from the fixed-point positions.
+constexpr int MM_STEPS = 64;  // steps whose run heads are in LDS at a time
 template <int KERNEL, bool EXACT>
-__global__ __launch_bounds__(64 * MM_WAVES) void mm_near(const uint4* __restrict__ P, const int* __restrict__ start,
-                                                         const int* __restrict__ items, const int* __restrict__ nitems,
-                                                         const float4* __restrict__ far, int lg, int ncols, NearK kc,
+__global__ __launch_bounds__(64 * MM_WAVES, 5) void mm_near(const uint4* __restrict__ P, const int* __restrict__ start,
+                                                         const int2* __restrict__ items, const int* __restrict__ nitems,
+                                                         const float* __restrict__ far, int lg, int ncols, NearK kc,
                                                          double fnear, double pnear, double ffar, double pfar,
                                                          float* __restrict__ fx, float* __restrict__ fy,
                                                          float* __restrict__ fz, float* __restrict__ pot) {
-    __shared__ uint4 S[MM_WAVES][MM_STAGE];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    __shared__ uint32_t heads_lds[MM_WAVES][2 * MM_STEPS];
+    __shared__ __align__(16) float red_lds[MM_WAVES][MM_SINKS * MM_RED];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t* const heads = heads_lds[w];
+    float* const red = red_lds[w];
     const int nc = 1 << lg, sh = 32 - lg, m = nc - 1;
     const uint32_t half = 1u << (sh - 1);
     const int total = *nitems;
-    for (int item = blockIdx.x * MM_WAVES + w; item < total; item += gridDim.x * MM_WAVES) {
-        const int row = items[3 * item], first = items[3 * item + 1], cnt = items[3 * item + 2];
-        const int cx = row >> lg, cy = row & m;
-        const bool live = lane < cnt;
-        const uint4 me = P[first + (live ? lane : cnt - 1)];
-        const int zs = (int)(me.z >> sh);
-        const int zl = __builtin_amdgcn_readfirstlane(zs);
-        const int zh = __shfl(zs, cnt - 1);
-        const uint32_t rx = ((uint32_t)cx << sh) + half, ry = ((uint32_t)cy << sh) + half,
-                       rz = ((uint32_t)zl << sh) + half;
-        const float ux = (float)(int32_t)(me.x - rx), uy = (float)(int32_t)(me.y - ry), uz = (float)(int32_t)(me.z - rz);
-        float sx = 0.f, sy = 0.f, sz = 0.f, sp = 0.f, cxs = 0.f, cys = 0.f, czs = 0.f, cps = 0.f;
-        for (int col = 0; col < ncols; ++col) {
-            const int dx = c_cols[col][0], dy = c_cols[col][1], hw = c_cols[col][2];
-            const int srow = (((cx + dx) & m) << lg) | ((cy + dy) & m);
-            const int* st = start + (size_t)srow * nc;  // st[nc] is the end of the column
-            const int span = min(zh - zl + 2 * hw + 1, nc);
-            const int zlo = span == nc ? 0 : (zl - hw) & m;
-            // the window in order: cells zlo .. min(zlo + span, nc) - 1, then 0 .. zlo + span - nc - 1
-            const int s0 = st[zlo], w0 = st[min(zlo + span, nc)] - s0, s1 = st[0];
-            const int W = w0 + (zlo + span > nc ? st[zlo + span - nc] - s1 : 0);
-            int lo = 0, hi = 0;
-            if constexpr (!EXACT) {  // this sink's run: window cells zs - zl .. zs - zl + 2w
-                const int za = zlo + zs - zl, zb = za + 2 * hw + 1;
-                lo = za <= nc ? st[za] - s0 : w0 + st[za - nc] - s1;
-                hi = zb <= nc ? st[zb] - s0 : w0 + st[zb - nc] - s1;
-            }
-            const int zsw = zs - hw;  // EXACT: a source of cell zc counts iff (zc - zsw) mod nc <= 2 hw
-            float tx = 0.f, ty = 0.f, tz = 0.f, tp = 0.f;
-            for (int jb = 0; jb < W; jb += MM_STAGE) {
-                const int nj = min(MM_STAGE, W - jb);
-                // EXACT: 16-byte records (fixed-point position, cell z); FP32 path:
-                // planes of x, y and z offsets (4-byte entries: the runs of a wave's
-                // cells start at different banks)
-                float* const sf = (float*)&S[w][0];
-                for (int k = lane; k < nj; k += 64) {
-                    const int p = jb + k;
-                    const uint4 q = P[p < w0 ? s0 + p : s1 + (p - w0)];
-                    if constexpr (EXACT) {
-                        S[w][k] = make_uint4(q.x, q.y, q.z, q.z >> sh);
-                    } else {
-                        sf[k] = (float)(int32_t)(q.x - rx);
-                        sf[MM_STAGE + k] = (float)(int32_t)(q.y - ry);
-                        sf[2 * MM_STAGE + k] = (float)(int32_t)(q.z - rz);
-                    }
-                }
-                wave_sync();
-                if constexpr (EXACT) {
-                    for (int j = 0; j < nj; ++j) {
-                        const uint4 q = S[w][j];
-                        if ((((int)q.w - zsw) & m) > 2 * hw) continue;
-                        near_pair<KERNEL>((float)(int32_t)(q.x - me.x), (float)(int32_t)(q.y - me.y),
-                                          (float)(int32_t)(q.z - me.z), kc, tx, ty, tz, tp);
-                    }
-                } else {
-                    const int a = max(lo - jb, 0), b = min(hi - jb, nj);
-                    int j = a;
-                    for (; j + MM_NEAR_UNROLL - 1 < b; j += MM_NEAR_UNROLL) {
-                        float qx[MM_NEAR_UNROLL], qy[MM_NEAR_UNROLL], qz[MM_NEAR_UNROLL];
+    const unsigned blocks = ((unsigned)(total + MM_WAVES - 1) / MM_WAVES + 7u) & ~7u;
+    const int dx = lane < ncols ? c_cols[lane][0] : 0, dy = lane < ncols ? c_cols[lane][1] : 0,
+              hw = lane < ncols ? c_cols[lane][2] : 0;
+    for (unsigned b = blockIdx.x; b < blocks; b += gridDim.x) {
+        const int item = (int)xcd_contiguous(b, blocks) * MM_WAVES + w;
+        if (item >= total) continue;
+        const int cell = __builtin_amdgcn_readfirstlane(items[item].x), group = __builtin_amdgcn_readfirstlane(items[item].y);
+        const int cs = __builtin_amdgcn_readfirstlane(start[cell]), n = __builtin_amdgcn_readfirstlane(start[cell + 1]) - cs;
+        const int groups = (n + MM_SINKS - 1) / MM_SINKS;
+        const int f = (int)((int64_t)group * n / groups), ns = (int)((int64_t)(group + 1) * n / groups) - f;
+        const int cx = cell >> 2 * lg, cy = cell >> lg & m, cz = cell & m;
+        const uint4 own = P[cs + f + min(lane, ns - 1)];
+        // the lane's column
+        const int* st = start + ((((cx + dx) & m) << lg | ((cy + dy) & m)) << lg);  // st[nc] is the end of the column
+        const int za = cz - hw, zb = cz + hw + 1;
+        const int end = st[nc], count = end - st[0];
+        const int s0 = st[za & m];
+        int len = st[zb > nc ? zb - nc : zb] - s0 + (za < 0 || zb > nc ? count : 0);
+        if (lane >= ncols) len = 0;
+        int upto = len;  // of the columns to this one
 #pragma unroll
-                        for (int u = 0; u < MM_NEAR_UNROLL; ++u) {
-                            qx[u] = sf[j + u];
-                            qy[u] = sf[MM_STAGE + j + u];
-                            qz[u] = sf[2 * MM_STAGE + j + u];
-                        }
-#pragma unroll
-                        for (int u = 0; u < MM_NEAR_UNROLL; ++u)
-                            near_pair<KERNEL>(qx[u] - ux, qy[u] - uy, qz[u] - uz, kc, tx, ty, tz, tp);
-                    }
-                    for (; j < b; ++j)
-                        near_pair<KERNEL>(sf[j] - ux, sf[MM_STAGE + j] - uy, sf[2 * MM_STAGE + j] - uz, kc, tx, ty,
-                                          tz, tp);
-                }
-                wave_sync();
-            }
-            two_sum_f(sx, cxs, tx);
-            two_sum_f(sy, cys, ty);
-            two_sum_f(sz, czs, tz);
-            two_sum_f(sp, cps, tp);
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(upto, d);
+            if (lane >= d) upto += v;
         }
-        if (live) {
-            const uint32_t i = me.w;
-            const float4 g = far[first + lane];
-            fx[i] = (float)(((double)sx + (double)cxs) * fnear + (double)g.x * ffar);
-            fy[i] = (float)(((double)sy + (double)cys) * fnear + (double)g.y * ffar);
-            fz[i] = (float)(((double)sz + (double)czs) * fnear + (double)g.z * ffar);
-            pot[i] = (float)(((double)sp + (double)cps) * pnear + (double)g.w * pfar);
+        const int W = __builtin_amdgcn_readlane(upto, 63), at = upto - len;
+        // the columns that hold particles first: what a slot is more than its place in the list, and where the column ends
+        const uint64_t some = __ballot(len > 0);
+        const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(some >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)some, 0));
+        const int rank = len > 0 ? below : __popcll(some) + lane - below;
+        const int shift = __builtin_amdgcn_ds_permute(4 * rank, s0 - at);
+        const bool wraps = cz < 3 || cz + 3 >= nc;  // uniform
+        const int ends = __builtin_amdgcn_ds_permute(4 * rank, end), counts = __builtin_amdgcn_ds_permute(4 * rank, count);
+        const uint32_t rx = ((uint32_t)cx << sh) + half, ry = ((uint32_t)cy << sh) + half, rz = ((uint32_t)cz << sh) + half;
+        double sum = 0.0;
+        for (int j0 = 0; j0 < W; j0 += 64 * MM_STEPS) {
+            const int steps = min(MM_STEPS, (W - j0 + 63) / 64);
+            heads[lane] = heads[64 + lane] = 0;
+            wave_sync();
+            if (len > 0 && at >= j0 && at < j0 + 64 * MM_STEPS) atomicOr(&heads[(at - j0) >> 5], 1u << (at & 31));
+            wave_sync();
+            const uint32_t hl = heads[2 * lane], hh = heads[2 * lane + 1];  // of step `lane`
+            int run = __popcll(__ballot(len > 0 && at < j0));               // heads before the step
+            const auto next = [&](int k, float& pad) {
+                const uint64_t h = (uint64_t)__builtin_amdgcn_readlane(hh, k) << 32 | (uint32_t)__builtin_amdgcn_readlane(hl, k);
+                const uint64_t up = h >> 1;
+                const int r = run + (int)(h & 1) - 1 +
+                              (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(up >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)up, 0));
+                run += __popcll(h);
+                const int j = j0 + 64 * k + lane;
+                int slot = j + __builtin_amdgcn_ds_bpermute(4 * r, shift);
+                if (wraps) {
+                    const int e = __builtin_amdgcn_ds_bpermute(4 * r, ends), c = __builtin_amdgcn_ds_bpermute(4 * r, counts);
+                    if (slot >= e) slot -= c;
+                }
+                pad = j < W ? 0.0f : __builtin_inff();
+                return P[j < W ? slot : cs];
+            };
+            switch (ns) {
+#define CT2_MM_NS(NS) \
+    case NS: near_sinks<KERNEL, EXACT, NS>(own, rx, ry, rz, steps, next, kc, lane, red); break;
+                CT2_MM_NS(1) CT2_MM_NS(2) CT2_MM_NS(3) CT2_MM_NS(4) CT2_MM_NS(5) CT2_MM_NS(6) CT2_MM_NS(7) CT2_MM_NS(8)
+                CT2_MM_NS(9) CT2_MM_NS(10)
+#undef CT2_MM_NS
+            }
+            wave_sync();
+            if (lane < 4 * ns) {  // sink lane / 4, component lane % 4
+                const float4* r = (const float4*)(red + (lane >> 2) * MM_RED + 16 * (lane & 3));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float4 v = r[i];
+                    sum += ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w);
+                }
+            }
+            wave_sync();
+        }
+        const uint32_t i = __shfl(own.w, lane >> 2);
+        if (lane < 4 * ns) {
+            const int q = lane & 3;
+            float* const out = q == 0 ? fx : q == 1 ? fy : q == 2 ? fz : pot;
+            out[i] = (float)(sum * (q < 3 ? fnear : pnear) + (double)far[4 * (size_t)(cs + f) + lane] * (q < 3 ? ffar : pfar));
         }
     }
 }
@@ -844,12 +860,10 @@ int mm_forces() {
     CT2_TRY(ensure_scratch((void**)&s.keys, &s.keys_bytes, sizeof(uint32_t) * 4 * (size_t)n, "multipole-mesh keys"));
     CT2_TRY(ensure_scratch((void**)&s.Ps, &s.Ps_bytes, sizeof(uint4) * (size_t)n, "multipole-mesh particles"));
     CT2_TRY(ensure_scratch((void**)&s.start, &s.start_bytes, sizeof(int) * ((size_t)n3 + 1), "cell starts"));
-    const int rows = nc * nc;
-    CT2_TRY(ensure_scratch((void**)&s.cnt, &s.cnt_bytes, sizeof(int) * 2 * (size_t)rows, "item counts"));
-    const int zspan = nc >= 32 ? 8 : nc >= 16 ? 4 : nc;  // the FP32 offsets stay minimum images
-    const size_t max_items = (size_t)n / 64 + (size_t)n3 / (size_t)std::min(zspan, nc) + (size_t)rows + 1;
-    CT2_TRY(ensure_scratch((void**)&s.items, &s.items_bytes, sizeof(int) * (3 * max_items + 1), "work items"));
-    s.nitems = s.items + 3 * max_items;
+    CT2_TRY(ensure_scratch((void**)&s.cnt, &s.cnt_bytes, sizeof(int) * 2 * (size_t)n3, "item counts"));
+    const size_t max_items = (size_t)n / MM_SINKS + (size_t)std::min(n, n3);
+    CT2_TRY(ensure_scratch((void**)&s.items, &s.items_bytes, sizeof(int2) * max_items + sizeof(int), "work items"));
+    int* const nitems = (int*)(s.items + max_items);
     uint32_t *kin = s.keys, *kout = s.keys + n, *vin = s.keys + 2L * n, *vout = s.keys + 3L * n;
     const unsigned pb = (unsigned)((n + 255) / 256);
     mm_keys<<<pb, 256, 0, st>>>(c.x, c.y, c.z, n, lg, kin, vin);
@@ -862,15 +876,15 @@ int mm_forces() {
     CT2_LAUNCH_CHECK();
     mm_bounds<<<(unsigned)((n3 + 256) / 256), 256, 0, st>>>(kout, n, n3, s.start);
     CT2_LAUNCH_CHECK();
-    int* first = s.cnt + rows;
-    const unsigned rb = (unsigned)((rows + 255) / 256);
-    mm_row_items<<<rb, 256, 0, st>>>(s.start, lg, zspan, 0, s.cnt, first, s.items, s.nitems);
+    int* first = s.cnt + n3;
+    const unsigned cb = (unsigned)((n3 + 255) / 256);
+    mm_item_counts<<<cb, 256, 0, st>>>(s.start, n3, s.cnt);
     CT2_LAUNCH_CHECK();
     tmp = 0;
-    CT2_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, s.cnt, first, rows, st));
+    CT2_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, s.cnt, first, n3, st));
     CT2_TRY(ensure_scratch(&s.scan_tmp, &s.scan_tmp_bytes, std::max<size_t>(tmp, 256), "item scan"));
-    CT2_HIP(hipcub::DeviceScan::ExclusiveSum(s.scan_tmp, tmp, s.cnt, first, rows, st));
-    mm_row_items<<<rb, 256, 0, st>>>(s.start, lg, zspan, 1, s.cnt, first, s.items, s.nitems);
+    CT2_HIP(hipcub::DeviceScan::ExclusiveSum(s.scan_tmp, tmp, s.cnt, first, n3, st));
+    mm_items<<<cb, 256, 0, st>>>(s.cnt, first, n3, s.items, nitems);
     CT2_LAUNCH_CHECK();
     // far field
     mm_p2m<<<(unsigned)(n3 / MM_P2M_CELLS), 256, 0, st>>>(s.Ps, s.start, lg, s.P, s.K, (size_t)n3, s.Zm);
@@ -910,14 +924,12 @@ int mm_forces() {
     kc.hinv3u = (float)(1.0 / (hu * hu * hu));
     const double fnear = gm * two32 * two32, pnear = gm * two32;
     const double ffar = gm * (double)nc * nc, pfar = gm * (double)nc;
-    // about one work item per wave (max_items bounds the count the device
-    // computes; waves past it exit at once): measured faster than 2,048 to
-    // 8,192 persistent workgroups taking items in turn (unequal items)
-    const unsigned grid = (unsigned)std::min<size_t>(65535, (max_items + MM_WAVES - 1) / MM_WAVES);
+    // a wave per work item (max_items bounds the count that the device computes; waves past it exit at once)
+    const unsigned grid = (unsigned)((max_items + MM_WAVES - 1) / MM_WAVES + 7) & ~7u;
     const bool plummer = c.opts.kernel == CT2_KERNEL_PLUMMER, exact = nc < 16;
-#define CT2_MM_NEAR(KER, EX)                                                                                    \
-    mm_near<KER, EX><<<grid, 64 * MM_WAVES, 0, st>>>(s.Ps, s.start, s.items, s.nitems, far, lg, s.ncols, kc, fnear, pnear, \
-                                                     ffar, pfar, c.fx, c.fy, c.fz, c.pot)
+#define CT2_MM_NEAR(KER, EX)                                                                                        \
+    mm_near<KER, EX><<<grid, 64 * MM_WAVES, 0, st>>>(s.Ps, s.start, s.items, nitems, (const float*)far, lg, s.ncols, \
+                                                     kc, fnear, pnear, ffar, pfar, c.fx, c.fy, c.fz, c.pot)
     if (plummer && exact)
         CT2_MM_NEAR(CT2_KERNEL_PLUMMER, true);
     else if (plummer)

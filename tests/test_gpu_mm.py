@@ -87,6 +87,34 @@ def test_orders_and_cells_of_several_passes(ct2, orc, nc, order):
     assert np.max(np.abs(pot - op)) < 1e-5 * np.abs(op).max()
 
 
+@pytest.mark.parametrize("nc,kernel", [(8, "KERNEL_PLUMMER"), (16, "KERNEL_PLUMMER"), (16, "KERNEL_CT2")])
+def test_near_groups_and_long_lists(ct2, orc, nc, kernel):
+    """Near pairs at the edges of their split: cells of 9, 10, 11, 20, 21 and 31
+    sinks (ten to a work item), a cell of 4,500 particles at z = 0 (lists of more
+    than 4,096 sources for its neighbours, some continued through z = 0), and
+    columns without particles.  Bounds as above; order 2 keeps the far field small."""
+    rng = np.random.default_rng(nc)
+    cells = [(1, 2, z, k) for z, k in zip((0, 2, 3, 5, 6, 7), (9, 10, 11, 20, 21, 31))]
+    cells += [(2, 2, 0, 4500), (2, 3, nc - 1, 3), (0, 2, nc - 1, 64), (nc - 1, 2, 1, 65), (4, 4, 4, 1)]
+    p = np.concatenate([(np.array(c[:3]) + rng.random((c[3], 3))) / nc for c in cells])
+    p = p[rng.permutation(len(p))]
+    x, y, z = [to_fixed(p[:, q]) for q in range(3)]
+    n = len(x)
+    gm, soft = float(np.float32(1.0 / n)), float(np.float32(2e-3))
+    ct2.particle_allocate(n)
+    ct2.particles_upload(x, y, z)
+    ct2.set_force_options(soft, gm, getattr(ct2, kernel))
+    try:
+        ct2.mm_init(nc, 2)
+        fx, fy, fz, pot = ct2.mm_forces()
+        ox, oy, oz, op = orc.mm_forces(x, y, z, nc, 2, gm, soft, kernel=getattr(orc, kernel))
+    finally:
+        ct2.set_force_options(soft, gm, ct2.KERNEL_PLUMMER)
+    e = rel_err(np.stack([fx, fy, fz]), np.stack([ox, oy, oz]))
+    assert np.median(e) < 3e-6 and np.percentile(e, 99) < 5e-5, (np.median(e), e.max())
+    assert np.max(np.abs(pot - op)) < 1e-5 * np.abs(op).max()
+
+
 def test_ct2_kernel_and_empty_cells(ct2, orc):
     """ct2's uniform-sphere kernel (kick.cpp:52-60) in the direct pairs, a
     16^3 grid with most cells empty, and particles on cell faces."""
