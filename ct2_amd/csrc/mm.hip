@@ -37,6 +37,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include "cellsort.h"
 #include "epilogue.h"
 #include "fft_stages.h"
 #include "internal.h"
@@ -112,8 +113,8 @@ struct MMState {
     float2* Zm = nullptr;  // multipole grids [nz][nc^3], then their transforms
     float2* Zl = nullptr;  // local-expansion grids
     size_t Z_bytes = 0;
-    uint32_t* keys = nullptr;  // sort keys / values in and out (4 n)
-    size_t keys_bytes = 0;
+    uint4* other = nullptr;    // the sort's second buffer (n)
+    size_t other_bytes = 0;
     void* sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
     uint4* Ps = nullptr;  // sorted (x, y, z, index)
@@ -264,40 +265,19 @@ __global__ __launch_bounds__(256) void mm_table_finish(const double2* __restrict
 
 // ------------------------------------------------------------ binning
 
-__global__ __launch_bounds__(256) void mm_keys(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
-                                               const uint32_t* __restrict__ Z, int n, int lg, uint32_t* __restrict__ key,
-                                               uint32_t* __restrict__ idx) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int sh = 32 - lg;
-    key[i] = (((X[i] >> sh) << lg | (Y[i] >> sh)) << lg) | (Z[i] >> sh);
-    idx[i] = (uint32_t)i;
-}
-
-__global__ __launch_bounds__(256) void mm_gather(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
-                                                 const uint32_t* __restrict__ Z, const uint32_t* __restrict__ idx, int n,
-                                                 uint4* __restrict__ P) {
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= n) return;
-    const uint32_t i = idx[s];
-    P[s] = make_uint4(X[i], Y[i], Z[i], i);
-}
-
-// start[c] = first sorted slot of cell c (lower bound of key c), start[n3] = n
-__global__ __launch_bounds__(256) void mm_bounds(const uint32_t* __restrict__ key, int n, int n3,
-                                                 int* __restrict__ start) {
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c > n3) return;
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (key[mid] < (uint32_t)c)
-            lo = mid + 1;
-        else
-            hi = mid;
+struct MMCellKey {
+    int lg;
+    __device__ __forceinline__ uint32_t operator()(const uint4& p) const {
+        const int sh = 32 - lg;
+        return (((p.x >> sh) << lg | (p.y >> sh)) << lg) | (p.z >> sh);
     }
-    start[c] = lo;
-}
+};
+
+// start[c] = first sorted slot of cell c, start[n3] = n
+struct PutCell {
+    int* start;
+    __device__ __forceinline__ void operator()(long c, long e) const { start[c] = (int)e; }
+};
 
 // Near-field work items: the sinks of a cell in groups of at most MM_SINKS, as
 // even as they go, each (cell, group).  Counts, then (after their exclusive sum)
@@ -857,30 +837,21 @@ int mm_forces() {
     const int n = (int)c.n, nc = s.nc, lg = ilog2(nc);
     const int n3 = nc * nc * nc;
     hipStream_t st = c.stream;
-    CT2_TRY(ensure_scratch((void**)&s.keys, &s.keys_bytes, sizeof(uint32_t) * 4 * (size_t)n, "multipole-mesh keys"));
+    CT2_TRY(ensure_scratch((void**)&s.other, &s.other_bytes, sizeof(uint4) * (size_t)n, "multipole-mesh sort"));
     CT2_TRY(ensure_scratch((void**)&s.Ps, &s.Ps_bytes, sizeof(uint4) * (size_t)n, "multipole-mesh particles"));
     CT2_TRY(ensure_scratch((void**)&s.start, &s.start_bytes, sizeof(int) * ((size_t)n3 + 1), "cell starts"));
     CT2_TRY(ensure_scratch((void**)&s.cnt, &s.cnt_bytes, sizeof(int) * 2 * (size_t)n3, "item counts"));
     const size_t max_items = (size_t)n / MM_SINKS + (size_t)std::min(n, n3);
     CT2_TRY(ensure_scratch((void**)&s.items, &s.items_bytes, sizeof(int2) * max_items + sizeof(int), "work items"));
     int* const nitems = (int*)(s.items + max_items);
-    uint32_t *kin = s.keys, *kout = s.keys + n, *vin = s.keys + 2L * n, *vout = s.keys + 3L * n;
-    const unsigned pb = (unsigned)((n + 255) / 256);
-    mm_keys<<<pb, 256, 0, st>>>(c.x, c.y, c.z, n, lg, kin, vin);
-    CT2_LAUNCH_CHECK();
-    size_t tmp = 0;
-    CT2_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, kin, kout, vin, vout, n, 0, 3 * lg, st));
-    CT2_TRY(ensure_scratch(&s.sort_tmp, &s.sort_tmp_bytes, std::max<size_t>(tmp, 256), "multipole-mesh sort"));
-    CT2_HIP(hipcub::DeviceRadixSort::SortPairs(s.sort_tmp, tmp, kin, kout, vin, vout, n, 0, 3 * lg, st));
-    mm_gather<<<pb, 256, 0, st>>>(c.x, c.y, c.z, vout, n, s.Ps);
-    CT2_LAUNCH_CHECK();
-    mm_bounds<<<(unsigned)((n3 + 256) / 256), 256, 0, st>>>(kout, n, n3, s.start);
-    CT2_LAUNCH_CHECK();
+    const MMCellKey key{lg};
+    CT2_TRY(cell_sort(c.x, c.y, c.z, n, key, 3 * lg, s.Ps, s.other, &s.sort_tmp, &s.sort_tmp_bytes, st));
+    CT2_TRY(cell_starts(s.Ps, key, n, n3, PutCell{s.start}, st));
     int* first = s.cnt + n3;
     const unsigned cb = (unsigned)((n3 + 255) / 256);
     mm_item_counts<<<cb, 256, 0, st>>>(s.start, n3, s.cnt);
     CT2_LAUNCH_CHECK();
-    tmp = 0;
+    size_t tmp = 0;
     CT2_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, s.cnt, first, n3, st));
     CT2_TRY(ensure_scratch(&s.scan_tmp, &s.scan_tmp_bytes, std::max<size_t>(tmp, 256), "item scan"));
     CT2_HIP(hipcub::DeviceScan::ExclusiveSum(s.scan_tmp, tmp, s.cnt, first, n3, st));
@@ -948,7 +919,7 @@ int mm_forces() {
 
 void release_mm() {
     MMState& s = g_mm;
-    for (void* p : {(void*)s.Dt, (void*)s.Dt32, (void*)s.Zm, (void*)s.Zl, (void*)s.keys, s.sort_tmp, (void*)s.Ps, (void*)s.start,
+    for (void* p : {(void*)s.Dt, (void*)s.Dt32, (void*)s.Zm, (void*)s.Zl, (void*)s.other, s.sort_tmp, (void*)s.Ps, (void*)s.start,
                     (void*)s.items, (void*)s.cnt, s.scan_tmp, (void*)s.tabz, (void*)s.sched, (void*)s.far})
         dev_free(p);
     s = MMState();

@@ -13,15 +13,14 @@
 // PM + near field tends to the periodic direct sum.
 //
 // Pipeline (all on the library stream, deterministic):
-//   near_key      slice key of each particle: (x, y) column, then z slice
-//                 (NEAR_SUB slices per cell), and its index
-//   radix sort    hipCUB's stable LSD sort of (key, index): the order is
-//                 (column, slice, particle index) for any scheduling and any
-//                 clustering, so the summation order never depends on atomics
-//   near_bounds   start of every slice and cell (a binary search each)
+//   cell_sort     the particles as (x, y, z, index) records, sorted stably by
+//                 slice key ((x, y) column, then z slice, NEAR_SUB per cell):
+//                 the order is (column, slice, particle index) for any
+//                 scheduling and any clustering, so the summation order never
+//                 depends on atomics (cellsort.h)
+//   cell_starts   start of every slice and cell
 //   near_scan     exclusive scan over the rows -> work-item prefix (runs of
 //                 NEAR_SINKS sinks per row)
-//   near_gather   the sorted (x, y, z, index)
 //   near_items    the (row, run) of every work item
 //   near_force    one wave per work item: 16 sinks, each in four lanes that
 //                 take every fourth source; the 9 (or 25) neighbouring rows'
@@ -39,8 +38,7 @@
 #include <utility>
 #include <vector>
 
-#include <hipcub/hipcub.hpp>
-
+#include "cellsort.h"
 #include "internal.h"
 
 namespace ct2 {
@@ -80,11 +78,9 @@ struct NearState {
     double rcut_rs = 0.0;  // 0 = off
     int nc = 0;
     size_t cap = 0;                // particles the buffers hold
-    uint32_t* key = nullptr;       // [cap] slice key of each particle
-    int* idx = nullptr;            // [cap] particle indices (sort values)
-    uint4* P0 = nullptr;           // [cap] sorted keys and indices (8 of its 16 B per particle)
+    uint4* P0 = nullptr;           // [cap] the sort's second buffer
     uint4* P = nullptr;            // [cap] sorted (x, y, z, index)
-    void* sort_tmp = nullptr;      // radix sort scratch
+    void* sort_tmp = nullptr;      // its counts
     size_t sort_tmp_bytes = 0;
     size_t ncell_cap = 0, nrow_cap = 0;  // cells and (x, y) columns the index buffers hold
     int* start = nullptr;          // [nc^3 + 1]
@@ -115,47 +111,25 @@ __device__ __forceinline__ uint32_t slice_of(uint32_t z, uint32_t nzs) {
     return (uint32_t)(((uint64_t)z * nzs) >> 32);
 }
 
-// Sort key of each particle: its (x, y) column row = cx nxy + cy and its z
+// Sort key of a particle: its (x, y) column row = cx nxy + cy and its z
 // slice u along the row, key = row nzs + u -- the index of its slice in
 // subst (cells: (row nc + u / NEAR_SUB) = key / NEAR_SUB).
-__global__ __launch_bounds__(256) void near_key(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
-                                                const uint32_t* __restrict__ Z, int n, uint32_t nxy, uint32_t nzs,
-                                                uint32_t* __restrict__ key, int* __restrict__ idx) {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= n) return;
-    key[p] = (cell_of(X[p], nxy) * nxy + cell_of(Y[p], nxy)) * nzs + slice_of(Z[p], nzs);
-    idx[p] = p;
-}
-
-// After the stable sort by key: subst[q] = first sorted position with key >=
-// q (q = 0 .. nkeys, subst[nkeys] = n), and the cell starts start[c] =
-// subst[c NEAR_SUB].  One binary search per slice, so empty slices cost the
-// same as full ones.
-__global__ __launch_bounds__(256) void near_bounds(const uint32_t* __restrict__ key, int n, int nkeys,
-                                                   int* __restrict__ subst, int* __restrict__ start) {
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    if (q > nkeys) return;
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (key[mid] < (uint32_t)q)
-            lo = mid + 1;
-        else
-            hi = mid;
+struct SliceKey {
+    uint32_t nxy, nzs;
+    __device__ __forceinline__ uint32_t operator()(const uint4& p) const {
+        return (cell_of(p.x, nxy) * nxy + cell_of(p.y, nxy)) * nzs + slice_of(p.z, nzs);
     }
-    subst[q] = lo;
-    if (q % NEAR_SUB == 0) start[q / NEAR_SUB] = lo;
-}
+};
 
-// The sorted particles: P[i] = (x, y, z, index) of sorted entry i.
-__global__ __launch_bounds__(256) void near_gather(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
-                                                   const uint32_t* __restrict__ Z, const int* __restrict__ idx, int n,
-                                                   uint4* __restrict__ P) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int p = idx[i];
-    P[i] = make_uint4(X[p], Y[p], Z[p], (uint32_t)p);
-}
+// subst[q] = first sorted position with key >= q (q = 0 .. nkeys, subst[nkeys]
+// = n), and the cell starts start[c] = subst[c NEAR_SUB].
+struct PutSlice {
+    int *subst, *start;
+    __device__ __forceinline__ void operator()(long q, long e) const {
+        subst[q] = (int)e;
+        if (q % NEAR_SUB == 0) start[q / NEAR_SUB] = (int)e;
+    }
+};
 
 // Exclusive scan (one workgroup) of the work items per row: out[0..len],
 // out[len] = total; row i holds ceil(m / NEAR_SINKS) items, m = in[(i+1)*nc] -
@@ -438,8 +412,6 @@ __global__ __launch_bounds__(64 * NEAR_WAVES) void near_force(
 }
 
 void free_near_buffers() {
-    dev_free(g_near.key);
-    dev_free(g_near.idx);
     dev_free(g_near.P0);
     dev_free(g_near.P);
     dev_free(g_near.sort_tmp);
@@ -453,8 +425,6 @@ void free_near_buffers() {
     dev_free(g_near.table);
     g_near.table = nullptr;
     g_near.table_rsu = g_near.table_rcu = 0.0;
-    g_near.key = nullptr;
-    g_near.idx = nullptr;
     g_near.P0 = g_near.P = nullptr;
     g_near.start = g_near.row_chunk = nullptr;
     g_near.item = nullptr;
@@ -465,17 +435,11 @@ void free_near_buffers() {
 
 int ensure_buffers(size_t n, size_t ncell, size_t nrow) {
     if (n > g_near.cap) {
-        dev_free(g_near.key);
-        dev_free(g_near.idx);
         dev_free(g_near.P0);
         dev_free(g_near.P);
-        g_near.key = nullptr;
-        g_near.idx = nullptr;
         g_near.P0 = g_near.P = nullptr;
         g_near.cap = 0;
-        CT2_TRY(dev_alloc((void**)&g_near.key, n * sizeof(uint32_t), "near-field sort keys"));
-        CT2_TRY(dev_alloc((void**)&g_near.idx, n * sizeof(int), "near-field sort values"));
-        CT2_TRY(dev_alloc((void**)&g_near.P0, n * sizeof(uint4), "near-field sorted keys"));
+        CT2_TRY(dev_alloc((void**)&g_near.P0, n * sizeof(uint4), "near-field sort"));
         CT2_TRY(dev_alloc((void**)&g_near.P, n * sizeof(uint4), "near-field sorted particles"));
         g_near.cap = n;
     }
@@ -609,29 +573,17 @@ int near_forces(double rs) {
     const int c3 = nxy * nxy * nc, nrow = nxy * nxy;
     CT2_TRY(ensure_buffers(c.n, (size_t)c3, (size_t)nrow));
     g_near.nc = nc;
-    const unsigned pb = (unsigned)((n + 255) / 256);
     hipStream_t st = c.stream;
-    // (slice key, particle index) pairs sorted stably by key: the order is
-    // (row, z slice, particle index) whatever the scheduling
+    // sorted stably by slice: the order is (row, z slice, particle index)
+    // whatever the scheduling
     const uint32_t nzs = (uint32_t)(nc * NEAR_SUB);
     const int nkeys = c3 * NEAR_SUB;  // = nrow nzs < 2^25
     int bits = 1;
     while ((1 << bits) < nkeys) ++bits;
-    uint32_t* kin = g_near.key;
-    int* vin = g_near.idx;
-    uint32_t* kout = (uint32_t*)g_near.P0;  // P0 (16 B per particle) holds the sorted keys and indices
-    int* vout = (int*)g_near.P0 + n;
-    near_key<<<pb, 256, 0, st>>>(c.x, c.y, c.z, n, (uint32_t)nxy, nzs, kin, vin);
-    CT2_LAUNCH_CHECK();
-    size_t tmp = 0;
-    CT2_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, kin, kout, vin, vout, n, 0, bits, st));
-    CT2_TRY(ensure_scratch(&g_near.sort_tmp, &g_near.sort_tmp_bytes, std::max<size_t>(tmp, 256), "near-field sort"));
-    CT2_HIP(hipcub::DeviceRadixSort::SortPairs(g_near.sort_tmp, tmp, kin, kout, vin, vout, n, 0, bits, st));
-    near_bounds<<<(unsigned)((nkeys + 256) / 256), 256, 0, st>>>(kout, n, nkeys, g_near.subst, g_near.start);
-    CT2_LAUNCH_CHECK();
+    const SliceKey key{(uint32_t)nxy, nzs};
+    CT2_TRY(cell_sort(c.x, c.y, c.z, n, key, bits, g_near.P, g_near.P0, &g_near.sort_tmp, &g_near.sort_tmp_bytes, st));
+    CT2_TRY(cell_starts(g_near.P, key, n, nkeys, PutSlice{g_near.subst, g_near.start}, st));
     near_scan<<<1, SCAN_THREADS, 0, st>>>(g_near.start, nrow, nc, g_near.row_chunk);
-    CT2_LAUNCH_CHECK();
-    near_gather<<<pb, 256, 0, st>>>(c.x, c.y, c.z, vout, n, g_near.P);
     CT2_LAUNCH_CHECK();
 
     const double u = 0x1p32;

@@ -45,6 +45,34 @@ def test_to_grid_is_a_stable_cell_sort(ct2, n, nc, minrung):
     assert starts[-1] == last
 
 
+@pytest.mark.parametrize("n", [2, 2047, 2048, 2049, 4097, 65536, 65537, 2 ** 21 - 1, 2 ** 21 + 8191])
+@pytest.mark.parametrize("nc", [1, 2, 13, 64, 129, 162, 256])
+@pytest.mark.parametrize("one_cell", [False, True])
+def test_cell_sort_tiles_and_passes(ct2, n, nc, one_cell):
+    """Records in one tile, in few (their counts summed by the placement) and many,
+    full and not; keys of one, two and three passes; all particles but one in a
+    cell in the middle (long runs of empty cells before and after it)."""
+    rng = np.random.default_rng(n + nc)
+    x, y, z = (rng.integers(0, TWO32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
+    if one_cell:
+        x[1:], y[1:], z[1:] = (rng.integers(TWO32 // 2, TWO32 // 2 + 1000, n - 1, dtype=np.uint64).astype(np.uint32)
+                               for _ in range(3))
+    vx = np.arange(n, dtype=np.float32)
+    ct2.particle_allocate(n)
+    ct2.particles_upload(x, y, z, vx, -vx, 2 * vx, (np.arange(n) % 5).astype(np.int8))
+    ct2.particle_sort_by_rung(0)
+    starts = ct2.particles_to_grid(nc)
+    p = ct2.particles_download()
+    key = cell_of(x, y, z, nc)
+    order = np.argsort(key, kind="stable")
+    assert np.array_equal(p.vx, vx[order])
+    assert np.array_equal(p.vy, -vx[order]) and np.array_equal(p.vz, 2 * vx[order])
+    assert np.array_equal(p.rung, order % 5)
+    for a, b in ((p.x, x), (p.y, y), (p.z, z)):
+        assert np.array_equal(a, b[order])
+    assert np.array_equal(starts, np.searchsorted(key[order], np.arange(nc ** 3 + 1), side="left"))
+
+
 def test_to_grid_rejects_bad_sizes(ct2):
     from ct2_amd import Ct2Error
     ct2.particle_allocate(10)
