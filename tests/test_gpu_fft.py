@@ -49,6 +49,20 @@ def test_fft3d_fp32_vs_numpy_fp64(ct2, n):
     assert rel_l2(back, z.astype(np.complex128)) < 1e-5
 
 
+@pytest.mark.parametrize("f64", [False, True])
+@pytest.mark.parametrize("d", [1, -1])
+def test_fft3d_in_groups_of_planes(ct2, f64, d):
+    """Cubes of 1 GB and more take their z and y passes by groups of planes (512^3:
+    96 or 48 planes, the last group smaller): a product of three random lines,
+    whose transform is the product of theirs."""
+    n, rng = 512, np.random.default_rng(5)
+    a = rng.standard_normal((3, n)) + 1j * rng.standard_normal((3, n))
+    t = np.fft.fft(a) if d > 0 else np.fft.ifft(a, norm="forward")
+    cube = [(v[0][:, None, None] * v[1][:, None]) * v[2] for v in (a, t)]
+    got = ct2.fft3d(cube[0] if f64 else cube[0].astype(np.complex64), d)
+    assert rel_l2(got, cube[1]) < (1e-14 if f64 else 1e-6)
+
+
 def test_fft3d_512_round_trip_and_delta(ct2):
     """512^3 (the PM grid of the clustered and stepping configurations):
     delta -> constant, and forward/inverse round trip."""
