@@ -72,11 +72,40 @@ __device__ __forceinline__ void epilogue(float f0, float f1, float f2, float& vx
     }
 }
 
+// The container's sinks as an epilogue updates them: `first` and those after it.
+struct Sinks {
+    EpiConst e;
+    int first;
+    float *vx, *vy, *vz;
+    int8_t* rung;
+    int* maxrung;
+
+    __device__ __forceinline__ void apply(int i, float f0, float f1, float f2, int& rmax) const {
+        float u = vx[i], v = vy[i], w = vz[i];
+        int8_t r = rung[i];
+        epilogue(f0, f1, f2, u, v, w, r, e, rmax);
+        vx[i] = u;
+        vy[i] = v;
+        vz[i] = w;
+        rung[i] = r;
+    }
+    // every lane of the wave
+    __device__ __forceinline__ void store_max(int rmax) const {
+        for (int off = 32; off > 0; off >>= 1) rmax = max(rmax, __shfl_xor(rmax, off));
+        if ((threadIdx.x & 63) == 0 && rmax > 0) atomicMax(maxrung, rmax);
+    }
+};
+
 // Validates the kick parameters the epilogue will use.
 int check_kick_params(const ct2_kick_params* p);
 
 // Launches the epilogue over the stored forces of the context (used by the
 // mesh-based kicks; the direct sum fuses it into its finalize kernel).
 int run_epilogue(const ct2_kick_params* p, int* max_rung);
+// The same in two halves, for a force whose last kernel may apply it: the max-rung
+// counter made ready before the force, and the epilogue (unless `applied`) and
+// kick()'s return value after it.
+int begin_epilogue(const ct2_kick_params* p, Sinks* sinks);
+int finish_epilogue(const ct2_kick_params* p, const Sinks& sinks, bool applied, int* max_rung);
 
 }  // namespace ct2

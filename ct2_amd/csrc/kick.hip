@@ -245,23 +245,11 @@ __global__ __launch_bounds__(256) void kick_finalize(PartialSums s0, PartialSums
 
 // Epilogue over stored forces (mesh-based kicks).
 __global__ __launch_bounds__(256) void epilogue_kernel(const float* __restrict__ fx, const float* __restrict__ fy,
-                                                       const float* __restrict__ fz, int n, int i0, EpiConst e,
-                                                       float* __restrict__ vx, float* __restrict__ vy,
-                                                       float* __restrict__ vz, int8_t* __restrict__ rung,
-                                                       int* __restrict__ maxrung) {
-    const int i = i0 + blockIdx.x * 256 + threadIdx.x;
+                                                       const float* __restrict__ fz, int n, Sinks sinks) {
+    const int i = sinks.first + blockIdx.x * 256 + threadIdx.x;
     int rmax = 0;
-    if (i < n) {
-        float u = vx[i], v = vy[i], w = vz[i];
-        int8_t r = rung[i];
-        epilogue(fx[i], fy[i], fz[i], u, v, w, r, e, rmax);
-        vx[i] = u;
-        vy[i] = v;
-        vz[i] = w;
-        rung[i] = r;
-    }
-    for (int off = 32; off > 0; off >>= 1) rmax = max(rmax, __shfl_xor(rmax, off));
-    if ((threadIdx.x & 63) == 0 && rmax > 0) atomicMax(maxrung, rmax);
+    if (i < n) sinks.apply(i, fx[i], fy[i], fz[i], rmax);
+    sinks.store_max(rmax);
 }
 
 __global__ void zero_int(int* p) { *p = 0; }
@@ -1042,20 +1030,28 @@ int check_kick_params(const ct2_kick_params* p) {
     return CT2_OK;
 }
 
-int run_epilogue(const ct2_kick_params* p, int* max_rung) {
+int begin_epilogue(const ct2_kick_params* p, Sinks* sinks) {
     Context& c = ctx();
     if (!c.maxrung) CT2_TRY(dev_alloc((void**)&c.maxrung, sizeof(int), "max rung"));
     CT2_TRY(clear_max_rung(c, p, c.maxrung));
-    if (epilogue_active(p)) {
-        const EpiConst e = make_epilogue(p, c.opts.hsoft);
-        const int n = (int)c.n, i0 = (int)c.rung_begin;
-        if (n > i0) {
-            epilogue_kernel<<<(n - i0 + 255) / 256, 256, 0, c.stream>>>(c.fx, c.fy, c.fz, n, i0, e, c.vx, c.vy, c.vz,
-                                                                         c.rung, c.maxrung);
-            CT2_LAUNCH_CHECK();
-        }
+    *sinks = Sinks{make_epilogue(p, c.opts.hsoft), (int)c.rung_begin, c.vx, c.vy, c.vz, c.rung, c.maxrung};
+    return CT2_OK;
+}
+
+int finish_epilogue(const ct2_kick_params* p, const Sinks& sinks, bool applied, int* max_rung) {
+    Context& c = ctx();
+    const int n = (int)c.n;
+    if (epilogue_active(p) && !applied && n > sinks.first) {
+        epilogue_kernel<<<(n - sinks.first + 255) / 256, 256, 0, c.stream>>>(c.fx, c.fy, c.fz, n, sinks);
+        CT2_LAUNCH_CHECK();
     }
     return return_max_rung(c, p, c.maxrung, max_rung);
+}
+
+int run_epilogue(const ct2_kick_params* p, int* max_rung) {
+    Sinks sinks;
+    CT2_TRY(begin_epilogue(p, &sinks));
+    return finish_epilogue(p, sinks, false, max_rung);
 }
 
 }  // namespace ct2

@@ -245,7 +245,8 @@ __device__ __forceinline__ int block_scan(int nt, const IN& in, const OUT& out) 
 
 // Binning, second half: every workgroup scans the tile totals (workgroup 0
 // writes them out as tstart) and places its particles' entries, grouped by
-// tile, in order.  Which of a tile's slots an entry gets depends on scheduling;
+// tile, in order.  total null: no bin_prefix has run, and every workgroup sums
+// the counts as they are (bin_in_lds).  Which of a tile's slots an entry gets depends on scheduling;
 // the set does not.
 template <int ORDER, int TILES>
 __global__ __launch_bounds__(BIN_THREADS) void bin_scatter(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
@@ -253,13 +254,31 @@ __global__ __launch_bounds__(BIN_THREADS) void bin_scatter(const uint32_t* __res
                                                           const int* __restrict__ cnt, const int* __restrict__ total,
                                                           int* __restrict__ tstart, int* __restrict__ order) {
     __shared__ int h[TILES];
-    const int* mine = cnt + (size_t)blockIdx.x * nt;
     const bool first = blockIdx.x == 0;
-    const int sum = block_scan(nt, [&](int t) { return total[t]; },
-                               [&](int t, int s) {
-                                   h[t] = s + mine[t];
-                                   if (first) tstart[t] = s;
-                               });
+    int sum;
+    if (total) {
+        const int* mine = cnt + (size_t)blockIdx.x * nt;
+        sum = block_scan(nt, [&](int t) { return total[t]; },
+                         [&](int t, int s) {
+                             h[t] = s + mine[t];
+                             if (first) tstart[t] = s;
+                         });
+    } else {  // at most one tile a thread
+        int before = 0, all = 0;
+        const int t = threadIdx.x, nw = gridDim.x;
+        if (t < nt)
+#pragma unroll 8
+            for (int w = 0; w < nw; ++w) {
+                const int v = cnt[(size_t)w * nt + t];
+                before += w < (int)blockIdx.x ? v : 0;
+                all += v;
+            }
+        sum = block_scan(nt, [&](int) { return all; },
+                         [&](int k, int s) {
+                             h[k] = s + before;
+                             if (first) tstart[k] = s;
+                         });
+    }
     if (first && threadIdx.x == 0) tstart[nt] = sum;
     __syncthreads();
     const int p1 = (int)min((long)n, (long)(blockIdx.x + 1) * per);
@@ -360,13 +379,20 @@ __global__ __launch_bounds__(TILE_THREADS) void dep_tile(const uint32_t* __restr
 // cell in 205 us; with the half-spectrum z and y passes before it the
 // transforms of one force on 256^3 went from 453 to 327 us, on 64^3 from 36 to
 // 22 us (ten launches to four).
+// On 64^3 grids the columns of the cubes' passes make 66 workgroups; 8 of them
+// (64-byte segments) make 264: 9.1 -> 7.8 us.
 template <int N>
-__global__ __launch_bounds__((Cfg<float, N, N / 2>::P * Cfg<float, N, N / 2>::COLS)) void pm_xpass(
+constexpr int xpass_cols() {
+    return N == 64 ? 8 : Cfg<float, N, N / 2>::COLS;
+}
+
+template <int N>
+__global__ __launch_bounds__((Cfg<float, N, N / 2>::P * xpass_cols<N>())) void pm_xpass(
     const float2* __restrict__ half, float2* __restrict__ A, const double* __restrict__ G,
     const float2* __restrict__ twg) {
     constexpr int H = N / 2;
     using CF = Cfg<float, N, H>;
-    constexpr int COLS = CF::COLS;
+    constexpr int COLS = xpass_cols<N>();
     constexpr unsigned MAIN = (unsigned)N * (H / COLS);
     constexpr double twopi = 6.283185307179586476925;
     __shared__ float2 sm[N * COLS];
@@ -394,11 +420,16 @@ __global__ __launch_bounds__((Cfg<float, N, N / 2>::P * Cfg<float, N, N / 2>::CO
     const double wy = ky == H ? 0.0 : twopi * my, wz = kz == H ? 0.0 : twopi * kz;
     double2 phi[CF::RM];
     const double* Gc = G + (long)abs(my) * (H + 1) + kz;
+    double g[CF::RM];  // read ahead of the transform they wait for
+#pragma unroll
+    for (int m = 0; m < CF::RM; ++m) {
+        const int i = p + m * CF::P;
+        g[m] = Gc[(long)(i < H ? i : N - i) * (H + 1) * (H + 1)];
+    }
     run_stages<float, N, 1, false, false>(
         [&](int i, int) { return d[(long)i * stride]; },
         [&](int i, int m, float2 v) {
-            const double g = Gc[(long)(i < H ? i : N - i) * (H + 1) * (H + 1)];
-            phi[m] = double2{g * (double)v.x, g * (double)v.y};
+            phi[m] = double2{g[m] * (double)v.x, g[m] * (double)v.y};
         },
         ix, sm, tw, p);
     constexpr long N2 = (long)N * N, N3 = N2 * N;
@@ -441,7 +472,8 @@ int xpass_launch(const float2* half, float2* A, const double* G, hipStream_t st)
     using CF = Cfg<float, N, N / 2>;
     const float2* tw = nullptr;
     CT2_TRY(fft_table_f32(N, &tw));
-    pm_xpass<N><<<N * (N / 2) / CF::COLS + N / CF::COLS, CF::P * CF::COLS, 0, st>>>(half, A, G, tw);
+    constexpr int COLS = xpass_cols<N>();
+    pm_xpass<N><<<N * (N / 2) / COLS + N / COLS, CF::P * COLS, 0, st>>>(half, A, G, tw);
     CT2_LAUNCH_CHECK();
     return CT2_OK;
 }
@@ -460,14 +492,16 @@ int xpass(int n, const float2* half, float2* A, const double* G, hipStream_t st)
     }
 }
 
-template <int ORDER>
+// EPI: a kick of nothing but this force goes on to its epilogue, a launch and 13
+// bytes read again per particle fewer.
+template <int ORDER, bool EPI>
 __global__ __launch_bounds__(PM_BLOCK) void mesh_interp(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
                                                        const uint32_t* __restrict__ Z, int n, int g,
                                                        const float2* __restrict__ A, const float2* __restrict__ B,
                                                        float* __restrict__ fx, float* __restrict__ fy,
-                                                       float* __restrict__ fz, float* __restrict__ pot) {
-    const int p = blockIdx.x * PM_BLOCK + threadIdx.x;
-    if (p >= n) return;
+                                                       float* __restrict__ fz, float* __restrict__ pot, Sinks epi) {
+    const int t = blockIdx.x * PM_BLOCK + threadIdx.x;
+    const int p = min(t, n - 1);
     const int s = 32 - g;
     const uint32_t ng = 1u << g, mask = ng - 1;
     uint32_t i0, j0, k0;
@@ -494,10 +528,17 @@ __global__ __launch_bounds__(PM_BLOCK) void mesh_interp(const uint32_t* __restri
                 acc3 = fmaf(w, b.y, acc3);
             }
         }
-    fx[p] = acc0;
-    fy[p] = acc1;
-    fz[p] = acc2;
-    pot[p] = acc3;
+    if (t < n) {
+        fx[p] = acc0;
+        fy[p] = acc1;
+        fz[p] = acc2;
+        pot[p] = acc3;
+    }
+    if constexpr (EPI) {
+        int rmax = 0;
+        if (t < n && t >= epi.first) epi.apply(t, acc0, acc1, acc2, rmax);
+        epi.store_max(rmax);
+    }
 }
 
 // Interpolation in tile order, for grids with enough particles per tile: a
@@ -607,10 +648,15 @@ int bin_in_lds(const Context& c) {
     const int per = (n + nw - 1) / nw;
     bin_count<ORDER, TILES><<<nw, BIN_THREADS, 0, c.stream>>>(c.x, c.y, c.z, n, per, g, nt, g_pm.bins);
     CT2_LAUNCH_CHECK();
-    bin_prefix<<<(nt + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, c.stream>>>(g_pm.bins, nw, nt, g_pm.tcount);
     CT2_LAUNCH_CHECK();
-    bin_scatter<ORDER, TILES><<<nw, BIN_THREADS, 0, c.stream>>>(c.x, c.y, c.z, n, per, g, nt, g_pm.bins, g_pm.tcount,
-                                                                g_pm.tstart, g_pm.order);
+    // few counts: cheaper summed by every workgroup than by one more launch
+    const bool few = nw <= 16 && nt <= BIN_THREADS;
+    if (!few) {
+        bin_prefix<<<(nt + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, c.stream>>>(g_pm.bins, nw, nt, g_pm.tcount);
+        CT2_LAUNCH_CHECK();
+    }
+    bin_scatter<ORDER, TILES><<<nw, BIN_THREADS, 0, c.stream>>>(c.x, c.y, c.z, n, per, g, nt, g_pm.bins,
+                                                                few ? nullptr : g_pm.tcount, g_pm.tstart, g_pm.order);
     CT2_LAUNCH_CHECK();
     return CT2_OK;
 }
@@ -711,7 +757,8 @@ int pm_require() {
 }
 
 // The PM force and potential of the container into the context force arrays.
-int pm_forces() {
+// epi: the sinks to kick where the interpolation can do it (then *applied).
+static int pm_forces(const Sinks* epi, bool* applied) {
     CT2_TRY(pm_require());
     CT2_TRY(ensure_table());
     Context& c = ctx();
@@ -734,15 +781,25 @@ int pm_forces() {
     else if (tiled)
         interp_tile<2><<<tiles, TILE_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.A, c.fx,
                                                              c.fy, c.fz, c.pot);
-    else if (g_assign == 1)
-        mesh_interp<1><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.A, g_pm.B, c.fx, c.fy, c.fz, c.pot);
-    else
-        mesh_interp<2><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.A, g_pm.B, c.fx, c.fy, c.fz, c.pot);
+    else {
+        const bool fuse = epi && !near_enabled();
+        auto interp = [&](auto kernel) {
+            kernel<<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.A, g_pm.B, c.fx, c.fy, c.fz, c.pot,
+                                                  fuse ? *epi : Sinks{});
+        };
+        if (g_assign == 1)
+            fuse ? interp(mesh_interp<1, true>) : interp(mesh_interp<1, false>);
+        else
+            fuse ? interp(mesh_interp<2, true>) : interp(mesh_interp<2, false>);
+        if (applied) *applied = fuse;
+    }
     CT2_LAUNCH_CHECK();
     if (near_enabled()) CT2_TRY(near_forces(g_pm.rs_cells / g_pm.ng));
     c.forces_valid = true;
     return CT2_OK;
 }
+
+int pm_forces() { return pm_forces(nullptr, nullptr); }
 
 // Device grids for the learned correction's feature gather.
 void pm_config(int* ng, double* rs_cells, int* order, double* rcut_rs) {
@@ -824,9 +881,12 @@ extern "C" int ct2_kick_pm(const ct2_kick_params* p, unsigned flags, int* max_ru
     CT2_TRY(pm_require());
     CT2_TRY(check_kick_params(p));
     if (flags & ~(unsigned)CT2_KICK_STORE) return set_error(CT2_ERR_INVALID, "unknown flags 0x%x", flags);
-    CT2_TRY(pm_forces());
+    Sinks sinks;
+    bool applied = false;
+    CT2_TRY(begin_epilogue(p, &sinks));
+    CT2_TRY(pm_forces(epilogue_active(p) ? &sinks : nullptr, &applied));
     ctx().last_path = near_enabled() ? CT2_PATH_PM_NEAR : CT2_PATH_PM;
-    return run_epilogue(p, max_rung);
+    return finish_epilogue(p, sinks, applied, max_rung);
 }
 
 extern "C" int ct2_pm_density_download(uint64_t* host) {

@@ -252,3 +252,56 @@ def test_tsc_pm_forces_vs_fp64_oracle(ct2, orc, tsc, ng, rs):
     rms = np.sqrt(np.mean(O ** 2))
     assert np.max(np.abs(F - O)) < 2e-5 * rms * np.sqrt(ng), np.max(np.abs(F - O)) / rms
     assert np.max(np.abs(pot - op)) < 1e-5 * np.abs(op).max()
+
+
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("n,ng", [(65, 16), (5000, 64), (40000, 32)])
+@pytest.mark.parametrize("descending", [False, True])
+def test_kick_pm_applies_the_epilogue_to_the_range(ct2, orc, order, n, ng, descending):
+    """The interpolation's own epilogue (the first two) and the separate kernel
+    (tiled interpolation), on a rung range that starts inside a wave."""
+    rng = np.random.default_rng(n + order)
+    x, y, z = (rng.integers(0, 2 ** 32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
+    rung = rng.integers(0, 3, n).astype(np.int8)
+    v = [(0.01 * rng.standard_normal(n)).astype(np.float32) for _ in range(3)]
+    ct2.particle_allocate(n)
+    ct2.particles_upload(x, y, z, *v, rung)
+    gm, soft = float(np.float32(1.0 / n)), float(np.float32(2e-3))
+    ct2.set_force_options(soft, gm, ct2.KERNEL_PLUMMER)
+    ct2.particle_sort_by_rung(1)
+    first, _ = ct2.particle_current_range()
+    p0 = ct2.particles_download()
+    params = ct2.kick_params(ascending=True, descending=descending, top=True, rung=1, t0=0.01)
+    ct2.pm_assignment(order)
+    try:
+        ct2.pm_init(ng, 1.25)
+        mr = ct2.kick_pm(params)
+    finally:
+        ct2.pm_assignment(1)
+    f = ct2.forces_download()
+    p1 = ct2.particles_download()
+    for a in ("vx", "vy", "vz", "rung"):
+        assert np.array_equal(getattr(p1, a)[:first], getattr(p0, a)[:first]), a
+    want = [getattr(p0, a)[first:].copy() for a in ("vx", "vy", "vz", "rung")]
+    op = orc.KickParams(*[getattr(params, k) for k, _ in params._fields_])
+    omr = orc.kick_epilogue(f[0][first:], f[1][first:], f[2][first:], *want, op, soft)
+    for a, w in zip(("vx", "vy", "vz", "rung"), want):
+        assert np.array_equal(getattr(p1, a)[first:], w), a
+    assert mr == omr
+
+
+@pytest.mark.parametrize("n,ng,order", [(16 * 4096 + 4095, 64, 2), (17 * 4096, 64, 1), (17 * 4096 - 1, 128, 1), (9001, 256, 2)])
+def test_deposit_few_binning_counts_bit_exact(ct2, orc, n, ng, order):
+    """16 and 17 binning workgroups, 64, 512 and 4,096 tiles: the counts summed by
+    the placement or by a kernel of their own."""
+    rng = np.random.default_rng(n)
+    x, y, z = (rng.integers(0, 2 ** 32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
+    load(ct2, x, y, z)
+    ct2.set_force_options(1e-3, 1.0 / n, 0)
+    ct2.pm_assignment(order)
+    try:
+        ct2.pm_init(ng, 1.25)
+        ct2.pm_forces()
+    finally:
+        ct2.pm_assignment(1)
+    assert np.array_equal(ct2.pm_density_download().ravel(), orc.mesh_deposit(x, y, z, ng.bit_length() - 1, order).ravel())
