@@ -684,10 +684,11 @@ int bin_particles(const Context& c) {
 // faster (us per PM force, per particle / tiled: CIC 4,096 particles on 32^3
 // 23.1 / 32.6, 8,000 on 64^3 32.3 / 42.7, 32,768 on 64^3 36.3 / 40.0 from a
 // lattice and 52.5 / 45.5 clustered; TSC 4,096 on 32^3 27.0 / 37.1, 32,768 on 64^3
-// 52.1 / 44.2).
+// 52.1 / 44.2).  Entries are counted in int, which up to MAX_COPIES for each of
+// 2^28 particles and more could exceed.
 template <int ORDER>
 bool tiles_pay(long n, int g) {
-    return g >= TILE_MIN_G && n * (ORDER == 1 ? 8 : 27) > 1L << 17;
+    return g >= TILE_MIN_G && n < (1L << 31) / MAX_COPIES && n * (ORDER == 1 ? 8 : 27) > 1L << 17;
 }
 
 // Density of the container's particles into g_pm.W.
