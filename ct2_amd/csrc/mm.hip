@@ -121,9 +121,9 @@ struct MMState {
     size_t Ps_bytes = 0;
     int* start = nullptr;  // cell starts (nc^3 + 1)
     size_t start_bytes = 0;
-    int2* items = nullptr;  // near-field work items (cell, group of its sinks), then their count
+    int2* items = nullptr;  // near-field work items, then their count
     size_t items_bytes = 0;
-    int* cnt = nullptr;  // items per cell, then the cells' first item (exclusive sum)
+    int* cnt = nullptr;  // items per cell, the cells' first item (exclusive sum), 16 bits per cell for the runs
     size_t cnt_bytes = 0;
     void* scan_tmp = nullptr;
     size_t scan_tmp_bytes = 0;
@@ -279,21 +279,78 @@ struct PutCell {
     __device__ __forceinline__ void operator()(long c, long e) const { start[c] = (int)e; }
 };
 
-// Near-field work items: the sinks of a cell in groups of at most MM_SINKS, as
-// even as they go, each (cell, group).  Counts, then (after their exclusive sum)
-// the items and their number.
-constexpr int MM_SINKS = 10;
-__global__ __launch_bounds__(256) void mm_item_counts(const int* __restrict__ start, int n3, int* __restrict__ cnt) {
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c < n3) cnt[c] = (start[c + 1] - start[c] + MM_SINKS - 1) / MM_SINKS;
+// Near-field work items.  The sinks of a row of cells (fixed x and y), in cell
+// order, form runs of at most MM_RUN that span fewer than zspan cells, and the
+// separations of a run are FP32 offsets from the centre of its first cell.  The
+// runs are part of the result, not of the split: the rounding of a close pair's
+// separation grows with its distance from that centre, so other centres move the
+// forces of a set's closest pairs by up to 1e-5 of the whole (2-norm).  An item is
+// at most MM_SINKS sinks of one cell and one run, as even as they go:
+// (cell | cells from the run's first to it << 24 | sinks << 27, first sink).
+constexpr int MM_SINKS = 10, MM_RUN = 64;
+constexpr int mm_zspan(int nc) { return nc >= 32 ? 8 : nc >= 16 ? 4 : 1; }  // the offsets stay minimum images (8^3: exact, no runs)
+constexpr int MM_HEAD_BITS = 7;  // of a part: MM_RUN sinks and none
+
+__device__ __forceinline__ int mm_groups(int sinks) { return (sinks + MM_SINKS - 1) / MM_SINKS; }
+
+// A wave per row walks its cells.  part[c]: how many of the cell's sinks at most
+// still belong to the run that holds its first one, and that run's first cell (so
+// many cells before | << MM_HEAD_BITS); later runs start in the cell, every MM_RUN
+// sinks.  cnt[c]: its items.
+__global__ __launch_bounds__(256) void mm_item_counts(const int* __restrict__ start, int lg, int zspan,
+                                                      int* __restrict__ cnt, uint16_t* __restrict__ part) {
+    const int nc = 1 << lg, lane = threadIdx.x & 63;
+    const int row = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    const int* st = start + ((size_t)row << lg);
+    int end = 0, ref = 0;  // of the run so far
+    for (int z0 = 0; z0 < nc; z0 += 64) {
+        const int z = z0 + lane;
+        const bool in = z < nc;
+        const int a = in ? st[z] : 0, b = in ? st[z + 1] : 0, reach = in ? st[min(z + zspan, nc)] : 0;
+        int head = 0, from = 0;
+        for (uint64_t m = __ballot(a < b); m; m &= m - 1) {
+            const int l = __ffsll((unsigned long long)m) - 1;
+            const int ca = __builtin_amdgcn_readlane(a, l), cb = __builtin_amdgcn_readlane(b, l),
+                      cr = __builtin_amdgcn_readlane(reach, l);
+            if (ca >= end) {
+                ref = z0 + l;
+                end = ca + min(MM_RUN, cr - ca);
+            }
+            if (lane == l) {
+                head = end - ca;
+                from = ref;
+            }
+            if (end < cb) {  // the last run that starts in this cell
+                ref = z0 + l;
+                const uint32_t more = ((uint32_t)(cb - end) + MM_RUN - 1) / MM_RUN * MM_RUN;
+                end += (int)min(more, (uint32_t)(cr - end));
+            }
+        }
+        if (!in) continue;
+        const int c = (row << lg) + z, later = max(b - a - head, 0);
+        cnt[c] = mm_groups(min(b - a, head)) + later / MM_RUN * mm_groups(MM_RUN) + mm_groups(later % MM_RUN);
+        part[c] = (uint16_t)(min(head, MM_RUN) | (z - from) << MM_HEAD_BITS);
+    }
 }
-__global__ __launch_bounds__(256) void mm_items(const int* __restrict__ cnt, const int* __restrict__ first, int n3,
+
+// After the counts' exclusive sum: the items and their number.
+__global__ __launch_bounds__(256) void mm_items(const int* __restrict__ start, const int* __restrict__ cnt,
+                                                const uint16_t* __restrict__ part, const int* __restrict__ first, int n3,
                                                 int2* __restrict__ items, int* __restrict__ nitems) {
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (c >= n3) return;
-    const int k = cnt[c], f = first[c];
-    for (int g = 0; g < k; ++g) items[f + g] = make_int2(c, g);
-    if (c == n3 - 1) *nitems = f + k;
+    int f = first[c];
+    if (c == n3 - 1) *nitems = f + cnt[c];
+    if (cnt[c] == 0) return;
+    int a = start[c], back = part[c] >> MM_HEAD_BITS, len = part[c] & ((1 << MM_HEAD_BITS) - 1);
+    for (const int b = start[c + 1]; a < b; back = 0, len = MM_RUN) {
+        const int n = min(b - a, len), groups = mm_groups(n);
+        for (int g = 0; g < groups; ++g) {
+            const int s0 = g * n / groups, s1 = (g + 1) * n / groups;
+            items[f++] = make_int2(c | back << 24 | (s1 - s0) << 27, a + s0);
+        }
+        a += n;
+    }
 }
 
 // ------------------------------------------------------------ P2M
@@ -714,7 +771,7 @@ __device__ __forceinline__ void near_sinks(uint4 own, uint32_t rx, uint32_t ry, 
 // through z = 0 continues a column's length lower); a lane holds a column's run,
 // and the runs joined are the item's list, 64 sources to a step, whose lane finds
 // its run from the bits of the run heads up to it.  Sources are read and taken as
-// FP32 offsets from the cell's centre once for all sinks, so that a pair costs
+// FP32 offsets (mm_item_counts says from where) once for all sinks, so that a pair costs
 // its 13 instructions, with no lane idle but in the last step; a lane sums every
 // 64th source in FP32, then the lanes are summed.  Bound by those instructions at
 // the rate that five waves per SIMD issue them: a lane per sink that walked its own
@@ -746,12 +803,10 @@ __global__ __launch_bounds__(64 * MM_WAVES, 5) void mm_near(const uint4* __restr
     for (unsigned b = blockIdx.x; b < blocks; b += gridDim.x) {
         const int item = (int)xcd_contiguous(b, blocks) * MM_WAVES + w;
         if (item >= total) continue;
-        const int cell = __builtin_amdgcn_readfirstlane(items[item].x), group = __builtin_amdgcn_readfirstlane(items[item].y);
-        const int cs = __builtin_amdgcn_readfirstlane(start[cell]), n = __builtin_amdgcn_readfirstlane(start[cell + 1]) - cs;
-        const int groups = (n + MM_SINKS - 1) / MM_SINKS;
-        const int f = (int)((int64_t)group * n / groups), ns = (int)((int64_t)(group + 1) * n / groups) - f;
+        const int it = __builtin_amdgcn_readfirstlane(items[item].x), first = __builtin_amdgcn_readfirstlane(items[item].y);
+        const int cell = it & 0xffffff, back = it >> 24 & 7, ns = it >> 27;
         const int cx = cell >> 2 * lg, cy = cell >> lg & m, cz = cell & m;
-        const uint4 own = P[cs + f + min(lane, ns - 1)];
+        const uint4 own = P[first + min(lane, ns - 1)];
         // the lane's column
         const int* st = start + ((((cx + dx) & m) << lg | ((cy + dy) & m)) << lg);  // st[nc] is the end of the column
         const int za = cz - hw, zb = cz + hw + 1;
@@ -773,7 +828,7 @@ __global__ __launch_bounds__(64 * MM_WAVES, 5) void mm_near(const uint4* __restr
         const int shift = __builtin_amdgcn_ds_permute(4 * rank, s0 - at);
         const bool wraps = cz < 3 || cz + 3 >= nc;  // uniform
         const int ends = __builtin_amdgcn_ds_permute(4 * rank, end), counts = __builtin_amdgcn_ds_permute(4 * rank, count);
-        const uint32_t rx = ((uint32_t)cx << sh) + half, ry = ((uint32_t)cy << sh) + half, rz = ((uint32_t)cz << sh) + half;
+        const uint32_t rx = ((uint32_t)cx << sh) + half, ry = ((uint32_t)cy << sh) + half, rz = ((uint32_t)(cz - back) << sh) + half;
         double sum = 0.0;
         for (int j0 = 0; j0 < W; j0 += 64 * MM_STEPS) {
             const int steps = min(MM_STEPS, (W - j0 + 63) / 64);
@@ -796,7 +851,7 @@ __global__ __launch_bounds__(64 * MM_WAVES, 5) void mm_near(const uint4* __restr
                     if (slot >= e) slot -= c;
                 }
                 pad = j < W ? 0.0f : __builtin_inff();
-                return P[j < W ? slot : cs];
+                return P[j < W ? slot : first];
             };
             switch (ns) {
 #define CT2_MM_NS(NS) \
@@ -820,7 +875,7 @@ __global__ __launch_bounds__(64 * MM_WAVES, 5) void mm_near(const uint4* __restr
         if (lane < 4 * ns) {
             const int q = lane & 3;
             float* const out = q == 0 ? fx : q == 1 ? fy : q == 2 ? fz : pot;
-            out[i] = (float)(sum * (q < 3 ? fnear : pnear) + (double)far[4 * (size_t)(cs + f) + lane] * (q < 3 ? ffar : pfar));
+            out[i] = (float)(sum * (q < 3 ? fnear : pnear) + (double)far[4 * (size_t)first + lane] * (q < 3 ? ffar : pfar));
         }
     }
 }
@@ -840,22 +895,23 @@ int mm_forces() {
     CT2_TRY(ensure_scratch((void**)&s.other, &s.other_bytes, sizeof(uint4) * (size_t)n, "multipole-mesh sort"));
     CT2_TRY(ensure_scratch((void**)&s.Ps, &s.Ps_bytes, sizeof(uint4) * (size_t)n, "multipole-mesh particles"));
     CT2_TRY(ensure_scratch((void**)&s.start, &s.start_bytes, sizeof(int) * ((size_t)n3 + 1), "cell starts"));
-    CT2_TRY(ensure_scratch((void**)&s.cnt, &s.cnt_bytes, sizeof(int) * 2 * (size_t)n3, "item counts"));
-    const size_t max_items = (size_t)n / MM_SINKS + (size_t)std::min(n, n3);
+    CT2_TRY(ensure_scratch((void**)&s.cnt, &s.cnt_bytes, (2 * sizeof(int) + sizeof(uint16_t)) * (size_t)n3, "item counts"));
+    // a part of at most MM_SINKS - 1 sinks beyond full items in each cell and at each end of a run inside one
+    const size_t max_items = (size_t)n / MM_SINKS + (size_t)std::min(n, n3) + (size_t)n / MM_RUN;
     CT2_TRY(ensure_scratch((void**)&s.items, &s.items_bytes, sizeof(int2) * max_items + sizeof(int), "work items"));
     int* const nitems = (int*)(s.items + max_items);
     const MMCellKey key{lg};
     CT2_TRY(cell_sort(c.x, c.y, c.z, n, key, 3 * lg, s.Ps, s.other, &s.sort_tmp, &s.sort_tmp_bytes, st));
     CT2_TRY(cell_starts(s.Ps, key, n, n3, PutCell{s.start}, st));
     int* first = s.cnt + n3;
-    const unsigned cb = (unsigned)((n3 + 255) / 256);
-    mm_item_counts<<<cb, 256, 0, st>>>(s.start, n3, s.cnt);
+    uint16_t* const part = (uint16_t*)(first + n3);
+    mm_item_counts<<<(unsigned)(nc * nc / 4), 256, 0, st>>>(s.start, lg, mm_zspan(nc), s.cnt, part);
     CT2_LAUNCH_CHECK();
     size_t tmp = 0;
     CT2_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, s.cnt, first, n3, st));
     CT2_TRY(ensure_scratch(&s.scan_tmp, &s.scan_tmp_bytes, std::max<size_t>(tmp, 256), "item scan"));
     CT2_HIP(hipcub::DeviceScan::ExclusiveSum(s.scan_tmp, tmp, s.cnt, first, n3, st));
-    mm_items<<<cb, 256, 0, st>>>(s.cnt, first, n3, s.items, nitems);
+    mm_items<<<(unsigned)((n3 + 255) / 256), 256, 0, st>>>(s.start, s.cnt, part, first, n3, s.items, nitems);
     CT2_LAUNCH_CHECK();
     // far field
     mm_p2m<<<(unsigned)(n3 / MM_P2M_CELLS), 256, 0, st>>>(s.Ps, s.start, lg, s.P, s.K, (size_t)n3, s.Zm);

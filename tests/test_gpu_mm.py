@@ -115,6 +115,82 @@ def test_near_groups_and_long_lists(ct2, orc, nc, kernel):
     assert np.max(np.abs(pot - op)) < 1e-5 * np.abs(op).max()
 
 
+def first_cell_of_runs(x, y, z, nc):
+    """The z cell whose centre a sink's near separations are taken from: the particles of a row of cells (fixed x and
+    y), in order of (z cell, index), form runs of at most 64 that span fewer than 8 cells (4 on 16^3 grids), and a
+    run's separations are FP32 offsets from the centre of its first cell."""
+    sh, span = 32 - int(np.log2(nc)), 4 if nc == 16 else 8
+    row, cz = (x >> sh).astype(np.int64) * nc + (y >> sh), (z >> sh).astype(np.int64)
+    ref = np.empty(x.size, np.int64)
+    last, c, z0 = -1, 0, 0
+    for i in np.argsort(row * nc + cz, kind="stable"):
+        if row[i] != last or c == 64 or cz[i] - z0 >= span:
+            last, c, z0 = row[i], 0, cz[i]
+        ref[i] = z0
+        c += 1
+    return ref
+
+
+@pytest.mark.parametrize("nc,kernel", [(16, "KERNEL_PLUMMER"), (32, "KERNEL_PLUMMER"), (32, "KERNEL_CT2")])
+def test_close_pairs_take_their_separation_from_the_runs_first_cell(ct2, nc, kernel):
+    """Close pairs (about 2,000 units of 2^-32 apart, 1e9 times the force of anything else) whose separation carries
+    the rounding of FP32 offsets from their run's first cell: a pair at every z cell of two rows, rows whose runs end
+    at 64 particles inside a cell, one cell of 150, and pairs behind 62 to 65 particles of an earlier cell.  The
+    pair's force in FP64 from those rounded offsets; tolerance: FP32 r^2, rsqrt (1 ulp) cubed and the products,
+    below 1e-6.  From any other cell's centre the separations differ by up to 64 units."""
+    rng = np.random.default_rng(nc)
+    sh = 32 - int(np.log2(nc))
+    cells = [(1, 2, c, 1) for c in range(nc)] + [(3, 0, c, 1) for c in range(2, nc, 3)]  # pairs per cell
+    fill = []                                                                              # lone particles per cell
+    for i, k in enumerate((61, 62, 63, 64)):
+        fill.append((5, 2 * i, 1, k))
+        cells += [(5, 2 * i, 1, 1), (5, 2 * i, 2, 2), (5, 2 * i, 6, 1)]
+    fill.append((8, 8, 3, 146))
+    cells += [(8, 8, 3, 2), (8, 8, 5, 1)]
+
+    def place(c):
+        return [(int(c[a]) << sh) + int(rng.integers(1 << (sh - 4), 15 << (sh - 4))) for a in range(3)]
+
+    pos, mate = [], []
+    for c in fill:
+        for _ in range(c[3]):
+            pos.append(place(c))
+            mate.append(-1)
+    for c in cells:
+        for _ in range(c[3]):
+            q = place(c)
+            d = [int(rng.choice([-1, 1]) * rng.integers(900, 1300)) for _ in range(3)]
+            k = len(pos)
+            pos += [q, [u + v for u, v in zip(q, d)]]
+            mate += [k + 1, k]
+    pos, mate = np.array(pos, dtype=np.int64), np.array(mate)
+    perm = rng.permutation(len(pos))
+    back = np.argsort(perm)
+    pos, mate = pos[perm], np.where(mate[perm] >= 0, back[mate[perm]], -1)
+    x, y, z = [pos[:, a].astype(np.uint32) for a in range(3)]
+    n = len(x)
+    gm, soft = float(np.float32(1.0 / n)), float(np.float32(300 / TWO32))
+    ct2.particle_allocate(n)
+    ct2.particles_upload(x, y, z)
+    ct2.set_force_options(soft, gm, getattr(ct2, kernel))
+    try:
+        ct2.mm_init(nc, 2)
+        F = np.stack(ct2.mm_forces()[:3]).astype(np.float64)
+    finally:
+        ct2.set_force_options(float(np.float32(2e-3)), gm, ct2.KERNEL_PLUMMER)
+    i = np.nonzero(mate >= 0)[0]
+    half = 1 << (sh - 1)
+    centre = [((x[i].astype(np.int64) >> sh) << sh) + half, ((y[i].astype(np.int64) >> sh) << sh) + half,
+              (first_cell_of_runs(x, y, z, nc)[i] << sh) + half]
+    off = lambda v, c: (v.astype(np.int64) - c).astype(np.float32)
+    d = np.stack([(off(v[mate[i]], c) - off(v[i], c)).astype(np.float64) for v, c in zip((x, y, z), centre)])
+    r2 = (d * d).sum(0) + (300.0 ** 2 if kernel == "KERNEL_PLUMMER" else 0.0)
+    W = gm * TWO32 ** 2 * d / r2 ** 1.5
+    e = rel_err(F[:, i], W)
+    print(f"{nc}^3 {kernel}: {i.size} sinks, largest error {e.max():.2e}", flush=True)
+    assert e.max() < 1e-6, (np.sort(e)[-5:], i[np.argsort(e)[-5:]])
+
+
 def test_ct2_kernel_and_empty_cells(ct2, orc):
     """ct2's uniform-sphere kernel (kick.cpp:52-60) in the direct pairs, a
     16^3 grid with most cells empty, and particles on cell faces."""
