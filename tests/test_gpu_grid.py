@@ -73,6 +73,47 @@ def test_cell_sort_tiles_and_passes(ct2, n, nc, one_cell):
     assert np.array_equal(starts, np.searchsorted(key[order], np.arange(nc ** 3 + 1), side="left"))
 
 
+def cell_centres(key, nc):
+    return [((2 * (k.astype(np.uint64)) + 1) * TWO32 // (2 * nc)).astype(np.uint32)
+            for k in (key // (nc * nc), key // nc % nc, key % nc)]
+
+
+@pytest.mark.parametrize("occupied", [
+    [0], [32767], [1023], [1024], [16384], [1023, 2047], [1024, 2048], [1022, 2047], [1023, 2046, 4000],
+    [5, 1028], [5, 1029], [5, 1030], [100, 1123, 2147, 3172, 32000], [0, 15, 31, 48, 1072, 2097, 32767]])
+def test_starts_across_long_runs_of_empty_cells(ct2, occupied):
+    """32^3 cells, 9,000 particles in a few of them: runs of 15 to 32,767 empty cells, 1,023 to 1,025 of them
+    starting and ending at, before and after multiples of 1,024 (starts are then written 1,024 to a wave)."""
+    nc, n = 32, 9000
+    key = np.array(occupied)[np.random.default_rng(len(occupied)).integers(0, len(occupied), n)]
+    ct2.particle_allocate(n)
+    ct2.particles_upload(*cell_centres(key, nc))
+    starts = ct2.particles_to_grid(nc)
+    assert np.array_equal(starts, np.searchsorted(np.sort(key), np.arange(nc ** 3 + 1), side="left"))
+
+
+def test_to_grid_of_a_set_in_a_corner_takes_no_longer(ct2):
+    """2^21 particles on 128^3 cells, in 1/50 of the box along each axis and in all of it: the empty cells' starts
+    must not be one wave's work.  About equal times are expected, 3x allowed."""
+    import time
+
+    from ct2_amd import _lib as L
+    n, nc = 2 ** 21, 128
+    rng = np.random.default_rng(4)
+    took = []
+    for part in (1, 50):
+        ct2.particle_allocate(n)
+        ct2.particles_upload(*(rng.integers(0, TWO32 // part, n, dtype=np.uint64).astype(np.uint32) for _ in range(3)))
+        best = np.inf
+        for _ in range(8):
+            t = time.perf_counter()
+            L.check(L.load().ct2_particles_to_grid(nc, None))
+            best = min(best, time.perf_counter() - t)
+        took.append(best)
+    print(f"all of the box {took[0] * 1e6:.0f} us, a corner {took[1] * 1e6:.0f} us", flush=True)
+    assert took[1] < 3 * took[0], took
+
+
 def test_to_grid_rejects_bad_sizes(ct2):
     from ct2_amd import Ct2Error
     ct2.particle_allocate(10)
