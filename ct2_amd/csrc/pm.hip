@@ -52,7 +52,7 @@ struct PmState {
     int* tcount = nullptr;  // [ntile]
     int* tstart = nullptr;  // [ntile + 1]
     int* bins = nullptr;    // [BIN_WGS][ntile] counts per binning workgroup
-    size_t cap = 0;         // particles order has room for
+    size_t cap = 0;         // particles order has room for (of one slab)
     int* order = nullptr;   // [cap MAX_COPIES] particle indices grouped by tile
 } g_pm;
 int g_assign = 1;  // mass assignment: 1 CIC, 2 TSC (kept across ct2_pm_init)
@@ -138,6 +138,10 @@ constexpr int BIN_THREADS = 1024;
 constexpr int BIN_WGS = 128;            // binning workgroups at most
 constexpr int BIN_TILES = 32768;        // tiles whose counters fit in LDS (512^3 grids)
 constexpr int MAX_COPIES = 8;           // tiles a stencil can touch
+// Entries are counted in int, and none can be refused: a list holds MAX_COPIES for
+// each of its particles.  Containers of more particles than this go slab by slab,
+// each adding its density to the last one's; the lists then take 8.6 GB.
+constexpr long SLAB_MAX = (1L << 31) / MAX_COPIES - 1;
 
 template <int ORDER>
 __device__ __forceinline__ uint32_t anchor_node(uint32_t x, int s) {
@@ -321,7 +325,7 @@ __global__ __launch_bounds__(BIN_THREADS) void tile_scan(int* __restrict__ in, i
 template <int ORDER>
 __global__ __launch_bounds__(TILE_THREADS) void dep_tile(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
                                                         const uint32_t* __restrict__ Z, const int* __restrict__ order,
-                                                        const int* __restrict__ tstart, int g,
+                                                        const int* __restrict__ tstart, int g, bool add,
                                                         unsigned long long* __restrict__ W) {
     __shared__ unsigned long long acc[TS * TS * TROW];
     const int tile = (int)xcd_contiguous(blockIdx.x, gridDim.x), tid = threadIdx.x;
@@ -360,7 +364,9 @@ __global__ __launch_bounds__(TILE_THREADS) void dep_tile(const uint32_t* __restr
     __syncthreads();
     for (int i = tid; i < TS * TS * TS; i += TILE_THREADS) {
         const int lz = i % TS, ly = i / TS % TS, lx = i / (TS * TS);
-        W[((((size_t)(ox + lx) << g) + (oy + ly)) << g) + (oz + lz)] = acc[(lx * TS + ly) * TROW + lz];
+        unsigned long long* const w = W + (((((size_t)(ox + lx) << g) + (oy + ly)) << g) + (oz + lz));
+        const unsigned long long v = acc[(lx * TS + ly) * TROW + lz];
+        *w = add ? *w + v : v;
     }
 }
 
@@ -627,7 +633,7 @@ void free_pm() {
     g_pm = PmState{};
 }
 
-// The tile lists' entries, grown to what the container can need.
+// The tile lists' entries, grown to what n particles can need.
 int ensure_deposit(size_t n) {
     if (n <= g_pm.cap) return CT2_OK;
     dev_free(g_pm.order);
@@ -638,43 +644,54 @@ int ensure_deposit(size_t n) {
     return CT2_OK;
 }
 
-// The container's particles grouped by tile: g_pm.tstart, g_pm.order.
+// Slab k of count: the container's particles [k per, (k + 1) per), per = ceil(n / count).
+struct Slab {
+    const uint32_t *x, *y, *z;
+    long first;
+    int n;
+};
+int slab_count(const Context& c) { return (int)(((long)c.n + SLAB_MAX - 1) / SLAB_MAX); }
+Slab slab(const Context& c, int k) {
+    const long count = slab_count(c), per = ((long)c.n + count - 1) / count, p0 = k * per;
+    return {c.x + p0, c.y + p0, c.z + p0, p0, (int)std::min(per, (long)c.n - p0)};
+}
+
+// A slab's particles grouped by tile: g_pm.tstart, g_pm.order (indices in the slab).
 template <int ORDER, int TILES>
-int bin_in_lds(const Context& c) {
-    const int n = (int)c.n, g = g_pm.g, nt = g_pm.ntile;
+int bin_in_lds(const Slab& p, hipStream_t st) {
+    const int n = p.n, g = g_pm.g, nt = g_pm.ntile;
     // at least 4 particles per thread, at most BIN_WGS workgroups: the counts of
     // each are a row that bin_prefix walks
     const int nw = std::max(1, std::min(BIN_WGS, n / (4 * BIN_THREADS)));
     const int per = (n + nw - 1) / nw;
-    bin_count<ORDER, TILES><<<nw, BIN_THREADS, 0, c.stream>>>(c.x, c.y, c.z, n, per, g, nt, g_pm.bins);
-    CT2_LAUNCH_CHECK();
+    bin_count<ORDER, TILES><<<nw, BIN_THREADS, 0, st>>>(p.x, p.y, p.z, n, per, g, nt, g_pm.bins);
     CT2_LAUNCH_CHECK();
     // few counts: cheaper summed by every workgroup than by one more launch
     const bool few = nw <= 16 && nt <= BIN_THREADS;
     if (!few) {
-        bin_prefix<<<(nt + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, c.stream>>>(g_pm.bins, nw, nt, g_pm.tcount);
+        bin_prefix<<<(nt + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, st>>>(g_pm.bins, nw, nt, g_pm.tcount);
         CT2_LAUNCH_CHECK();
     }
-    bin_scatter<ORDER, TILES><<<nw, BIN_THREADS, 0, c.stream>>>(c.x, c.y, c.z, n, per, g, nt, g_pm.bins,
-                                                                few ? nullptr : g_pm.tcount, g_pm.tstart, g_pm.order);
+    bin_scatter<ORDER, TILES><<<nw, BIN_THREADS, 0, st>>>(p.x, p.y, p.z, n, per, g, nt, g_pm.bins,
+                                                          few ? nullptr : g_pm.tcount, g_pm.tstart, g_pm.order);
     CT2_LAUNCH_CHECK();
     return CT2_OK;
 }
 
 template <int ORDER>
-int bin_particles(const Context& c) {
-    CT2_TRY(ensure_deposit(c.n));
-    const int n = (int)c.n, g = g_pm.g, nt = g_pm.ntile;
-    if (nt <= BIN_TILES / 8) return bin_in_lds<ORDER, BIN_TILES / 8>(c);
-    if (nt <= BIN_TILES) return bin_in_lds<ORDER, BIN_TILES>(c);
+int bin_particles(const Slab& p, hipStream_t st) {
+    CT2_TRY(ensure_deposit((size_t)p.n));
+    const int n = p.n, g = g_pm.g, nt = g_pm.ntile;
+    if (nt <= BIN_TILES / 8) return bin_in_lds<ORDER, BIN_TILES / 8>(p, st);
+    if (nt <= BIN_TILES) return bin_in_lds<ORDER, BIN_TILES>(p, st);
     const unsigned pb = (unsigned)((n + PM_BLOCK - 1) / PM_BLOCK);
-    fill_i32<<<(nt + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, c.stream>>>(g_pm.tcount, nt);
+    fill_i32<<<(nt + PM_BLOCK - 1) / PM_BLOCK, PM_BLOCK, 0, st>>>(g_pm.tcount, nt);
     CT2_LAUNCH_CHECK();
-    bin_global<ORDER, false><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.tcount, nullptr);
+    bin_global<ORDER, false><<<pb, PM_BLOCK, 0, st>>>(p.x, p.y, p.z, n, g, g_pm.tcount, nullptr);
     CT2_LAUNCH_CHECK();
-    tile_scan<<<1, BIN_THREADS, 0, c.stream>>>(g_pm.tcount, nt, g_pm.tstart);
+    tile_scan<<<1, BIN_THREADS, 0, st>>>(g_pm.tcount, nt, g_pm.tstart);
     CT2_LAUNCH_CHECK();
-    bin_global<ORDER, true><<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.tcount, g_pm.order);
+    bin_global<ORDER, true><<<pb, PM_BLOCK, 0, st>>>(p.x, p.y, p.z, n, g, g_pm.tcount, g_pm.order);
     CT2_LAUNCH_CHECK();
     return CT2_OK;
 }
@@ -684,11 +701,10 @@ int bin_particles(const Context& c) {
 // faster (us per PM force, per particle / tiled: CIC 4,096 particles on 32^3
 // 23.1 / 32.6, 8,000 on 64^3 32.3 / 42.7, 32,768 on 64^3 36.3 / 40.0 from a
 // lattice and 52.5 / 45.5 clustered; TSC 4,096 on 32^3 27.0 / 37.1, 32,768 on 64^3
-// 52.1 / 44.2).  Entries are counted in int, which up to MAX_COPIES for each of
-// 2^28 particles and more could exceed.
+// 52.1 / 44.2).
 template <int ORDER>
 bool tiles_pay(long n, int g) {
-    return g >= TILE_MIN_G && n < (1L << 31) / MAX_COPIES && n * (ORDER == 1 ? 8 : 27) > 1L << 17;
+    return g >= TILE_MIN_G && n * (ORDER == 1 ? 8 : 27) > 1L << 17;
 }
 
 // Density of the container's particles into g_pm.W.
@@ -703,10 +719,28 @@ int deposit(const Context& c) {
         CT2_LAUNCH_CHECK();
         return CT2_OK;
     }
-    CT2_TRY(bin_particles<ORDER>(c));
-    const int nt = g_pm.ntile;
-    dep_tile<ORDER><<<nt, TILE_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.W);
-    CT2_LAUNCH_CHECK();
+    const int nt = g_pm.ntile, count = slab_count(c);
+    for (int k = 0; k < count; ++k) {
+        const Slab p = slab(c, k);
+        CT2_TRY(bin_particles<ORDER>(p, c.stream));
+        dep_tile<ORDER><<<nt, TILE_THREADS, 0, c.stream>>>(p.x, p.y, p.z, g_pm.order, g_pm.tstart, g, k > 0, g_pm.W);
+        CT2_LAUNCH_CHECK();
+    }
+    return CT2_OK;
+}
+
+// Force and potential by tiles; the lists of the last slab are in place.
+template <int ORDER>
+int interp_by_tiles(const Context& c) {
+    const int count = slab_count(c);
+    for (int k = count - 1; k >= 0; --k) {
+        const Slab p = slab(c, k);
+        if (k < count - 1) CT2_TRY(bin_particles<ORDER>(p, c.stream));
+        interp_tile<ORDER><<<dim3(g_pm.ntile, 2), TILE_THREADS, 0, c.stream>>>(
+            p.x, p.y, p.z, g_pm.order, g_pm.tstart, g_pm.g, g_pm.A, c.fx + p.first, c.fy + p.first, c.fz + p.first,
+            c.pot + p.first);
+        CT2_LAUNCH_CHECK();
+    }
     return CT2_OK;
 }
 
@@ -775,14 +809,9 @@ static int pm_forces(const Sinks* epi, bool* applied) {
     // half in Plummer spheres 12.7 / 10.7, random field 4.98 / 5.06.
     const bool tiled = (g_assign == 1 ? tiles_pay<1>(n, g) : tiles_pay<2>(n, g)) && g <= 9 &&
                        (long)n * (g_assign == 1 ? 8 : 27) > 2L * TL_NODES * g_pm.ntile;
-    const dim3 tiles(g_pm.ntile, 2);
-    if (tiled && g_assign == 1)
-        interp_tile<1><<<tiles, TILE_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.A, c.fx,
-                                                             c.fy, c.fz, c.pot);
-    else if (tiled)
-        interp_tile<2><<<tiles, TILE_THREADS, 0, c.stream>>>(c.x, c.y, c.z, g_pm.order, g_pm.tstart, g, g_pm.A, c.fx,
-                                                             c.fy, c.fz, c.pot);
-    else {
+    if (tiled) {
+        CT2_TRY(g_assign == 1 ? interp_by_tiles<1>(c) : interp_by_tiles<2>(c));
+    } else {
         const bool fuse = epi && !near_enabled();
         auto interp = [&](auto kernel) {
             kernel<<<pb, PM_BLOCK, 0, c.stream>>>(c.x, c.y, c.z, n, g, g_pm.A, g_pm.B, c.fx, c.fy, c.fz, c.pot,
@@ -792,9 +821,9 @@ static int pm_forces(const Sinks* epi, bool* applied) {
             fuse ? interp(mesh_interp<1, true>) : interp(mesh_interp<1, false>);
         else
             fuse ? interp(mesh_interp<2, true>) : interp(mesh_interp<2, false>);
+        CT2_LAUNCH_CHECK();
         if (applied) *applied = fuse;
     }
-    CT2_LAUNCH_CHECK();
     if (near_enabled()) CT2_TRY(near_forces(g_pm.rs_cells / g_pm.ng));
     c.forces_valid = true;
     return CT2_OK;

@@ -305,3 +305,56 @@ def test_deposit_few_binning_counts_bit_exact(ct2, orc, n, ng, order):
     finally:
         ct2.pm_assignment(1)
     assert np.array_equal(ct2.pm_density_download().ravel(), orc.mesh_deposit(x, y, z, ng.bit_length() - 1, order).ravel())
+
+
+def fill_with_copies(ct2, base, copies):
+    """A container of `copies` times the base positions, one after the other."""
+    import ctypes as C
+
+    from ct2_amd import _lib as L
+    m = base[0].size
+    ct2.particle_allocate(m * copies)
+    ptr = L.ParticlePtrs()
+    L.check(L.load().ct2_particles_device_ptrs(C.byref(ptr)))
+    for dst, src in zip((ptr.x, ptr.y, ptr.z), base):
+        for k in range(copies):
+            L.check(L.load().ct2_memcpy_h2d(dst + 4 * m * k, src.ctypes.data_as(C.c_void_p), 4 * m))
+
+
+def test_containers_beyond_one_tile_list(ct2):
+    """2^28 particles (a tile list counts eight entries of each in an int, so the deposit takes more than one), 1,024
+    copies of 2^18 on a 256^3 grid with TSC: density and force are 2^10 times one copy's exactly, whatever the list,
+    and take about as long as for one copy fewer, which one list holds (2x allowed: binning runs again before the
+    interpolation; one global atomic per particle and node took several times as long)."""
+    import time
+
+    from ct2_amd import _lib as L
+    m, copies = 2 ** 18, 1024
+    rng = np.random.default_rng(28)
+    base = [rng.integers(0, 2 ** 32, m, dtype=np.uint64).astype(np.uint32) for _ in range(3)]
+    ct2.set_force_options(1e-3, 2.0 ** -28, ct2.KERNEL_PLUMMER)
+    ct2.pm_assignment(2)
+    try:
+        ct2.pm_init(256, 1.5)
+        ct2.particle_allocate(m)
+        ct2.particles_upload(*base)
+        one = ct2.pm_forces()
+        w = ct2.pm_density_download()
+        took = []
+        for k in (copies - 1, copies):
+            fill_with_copies(ct2, base, k)
+            best = np.inf
+            for _ in range(3):
+                t = time.perf_counter()
+                L.check(L.load().ct2_pm_forces())
+                ct2.synchronize()
+                best = min(best, time.perf_counter() - t)
+            took.append(best)
+            print(f"{k} copies: {best * 1e3:.1f} ms", flush=True)
+        assert np.array_equal(ct2.pm_density_download(), w * np.uint64(copies))
+        for f, g in zip(ct2.forces_download(), one):
+            assert (f.reshape(copies, m) == g * np.float32(copies)).all()
+    finally:
+        ct2.pm_assignment(1)
+        ct2.particle_allocate(16)
+    assert took[1] < 2 * took[0], took
