@@ -53,7 +53,7 @@ struct PmState {
     int* tstart = nullptr;  // [ntile + 1]
     int* bins = nullptr;    // [BIN_WGS][ntile] counts per binning workgroup
     size_t cap = 0;         // particles order has room for (of one slab)
-    int* order = nullptr;   // [cap MAX_COPIES] particle indices grouped by tile
+    int* order = nullptr;   // [cap MAX_COPIES] particle indices grouped by tile, ~index where at home in another
 } g_pm;
 int g_assign = 1;  // mass assignment: 1 CIC, 2 TSC (kept across ct2_pm_init)
 
@@ -132,7 +132,10 @@ constexpr int TS = 1 << TILE_B;
 constexpr int TROW = TS + 1;                 // padded LDS row
 constexpr int TL = TS + 2;                   // side of the grown tile
 constexpr int TL_NODES = TL * TL * TL;
-constexpr int TILE_THREADS = 512;
+// The tiles' kernels: two workgroups per CU.  A set in a corner of the box is a few
+// tiles' work: 2^21 particles in 1/1000 of it on 128^3 (TSC) take 9.8 ms a force,
+// with 512 threads to a tile 16.7; sets that fill the box are the same with either.
+constexpr int TILE_THREADS = 1024;
 constexpr int TILE_MIN_G = TILE_B + 1;  // grids of at least 2^5 nodes a side
 constexpr int BIN_THREADS = 1024;
 constexpr int BIN_WGS = 128;            // binning workgroups at most
@@ -287,7 +290,7 @@ __global__ __launch_bounds__(BIN_THREADS) void bin_scatter(const uint32_t* __res
     __syncthreads();
     const int p1 = (int)min((long)n, (long)(blockIdx.x + 1) * per);
     for (int p = blockIdx.x * per + threadIdx.x; p < p1; p += BIN_THREADS)
-        for_tiles<ORDER>(X[p], Y[p], Z[p], g, [&](int t, bool) { order[atomicAdd(&h[t], 1)] = p; });
+        for_tiles<ORDER>(X[p], Y[p], Z[p], g, [&](int t, bool home) { order[atomicAdd(&h[t], 1)] = home ? p : ~p; });
 }
 
 // The same for grids of more tiles than LDS holds counters for, with global
@@ -309,7 +312,7 @@ __global__ __launch_bounds__(PM_BLOCK) void bin_global(const uint32_t* __restric
                 home = t;
             } else {
                 const int k = atomicAdd(counter + t, 1);
-                if (PLACE) order[k] = p;
+                if (PLACE) order[k] = ~p;
             }
         });
     const int k = run_increment(counter, home);  // every lane of the wave takes part
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(TILE_THREADS) void dep_tile(const uint32_t* __restr
     for (int i = tid; i < TS * TS * TROW; i += TILE_THREADS) acc[i] = 0ull;
     __syncthreads();
     for (int k = b + tid; k < e; k += TILE_THREADS) {
-        const int p = order[k];
+        const int o = order[k], p = o < 0 ? ~o : o;
         const uint32_t x = X[p], y = Y[p], z = Z[p];
         uint32_t lo;
         uint32_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
@@ -549,7 +552,7 @@ __global__ __launch_bounds__(PM_BLOCK) void mesh_interp(const uint32_t* __restri
 
 // Interpolation in tile order, for grids with enough particles per tile: a
 // workgroup per deposit tile and grid (blockIdx.y: A = (Fx, Fy), B = (Fz, pot))
-// stages the grown tile's 18^3 nodes in LDS (47 KB, three workgroups per CU) and
+// stages the grown tile's 18^3 nodes in LDS (47 KB) and
 // interpolates the particles at home in it.  The same weights and summation
 // order as mesh_interp, so the results are identical.  Bound by the reads of the
 // grown tiles (rows of 144 bytes, 2.1 lines each): 130 us for 2^21 particles on
@@ -591,6 +594,7 @@ __global__ __launch_bounds__(TILE_THREADS) void interp_tile(const uint32_t* __re
     const float q = 0x1p-21f;
     for (int k = b + tid; k < e; k += TILE_THREADS) {
         const int p = order[k];
+        if (p < 0) continue;  // at home in a neighbour
         const uint32_t x = X[p], y = Y[p], z = Z[p];
         uint32_t lo;
         uint32_t ax[ORDER + 1], ay[ORDER + 1], az[ORDER + 1];
@@ -599,7 +603,6 @@ __global__ __launch_bounds__(TILE_THREADS) void interp_tile(const uint32_t* __re
         assign_axis<ORDER>(z, s, lo, az);
         const uint32_t hx = anchor_node<ORDER>(x, s) - ox, hy = anchor_node<ORDER>(y, s) - oy,
                        hz = anchor_node<ORDER>(z, s) - oz;
-        if ((hx | hy | hz) >= (uint32_t)TS) continue;  // at home in a neighbour
         const int lx = (int)(hx + SHIFT), ly = (int)(hy + SHIFT), lz = (int)(hz + SHIFT);
         float acc0 = 0.f, acc1 = 0.f;
 #pragma unroll
@@ -807,7 +810,10 @@ static int pm_forces(const Sinks* epi, bool* applied) {
     // that beats one L2 read per particle and stencil node.  Measured, PM force
     // per particle / tiled (TSC): 2^24 particles on 512^3, lattice 6.06 / 5.12 ms,
     // half in Plummer spheres 12.7 / 10.7, random field 4.98 / 5.06.
-    const bool tiled = (g_assign == 1 ? tiles_pay<1>(n, g) : tiles_pay<2>(n, g)) && g <= 9 &&
+    // CIC's eight nodes are fewer reads than the lists' on 512^3: 2^26 particles, per
+    // particle / tiled: lattice 6.27 / 6.35 ms, cell order 7.53 / 6.44, random order
+    // 23.4 / 30.4, half in 64 spheres 21.8 / 34.9.
+    const bool tiled = (g_assign == 1 ? tiles_pay<1>(n, g) && g <= 8 : tiles_pay<2>(n, g) && g <= 9) &&
                        (long)n * (g_assign == 1 ? 8 : 27) > 2L * TL_NODES * g_pm.ntile;
     if (tiled) {
         CT2_TRY(g_assign == 1 ? interp_by_tiles<1>(c) : interp_by_tiles<2>(c));
