@@ -91,7 +91,7 @@ __device__ __forceinline__ void f1_step(double2* s, int threads, int T, int lm, 
     __syncthreads();
 }
 
-// T = E / M transforms per workgroup of E / 8 threads, in LDS: transform t,
+// T <= E / M transforms per workgroup of E / 8 threads, in LDS: transform t,
 // element e at t pitch + e + e/8 (the padding keeps the radix-8 steps' strided
 // accesses, and the lanes of a group, off one bank group).  A transform holds 2 M doubles in memory, M = 2^lm:
 //   complex (N = M): row r of a group's 2 M x L array is part r % 2 of element
@@ -158,6 +158,56 @@ __global__ __launch_bounds__(E / 8) void fft1d_ct2(double* __restrict__ X, int l
         } else {
             const int e = r >> 1;
             X[address(d)] = ((const double*)&row[e + (e >> 3)])[(r & 1) ^ swap];
+        }
+    }
+}
+
+// A transform per workgroup, log2 N radix-2 steps of a butterfly a thread: the
+// shortest chain, for batches that leave the chip idle (a radix-8 step is three
+// trips to LDS and the twiddles fewer, but a few waves' long arithmetic).  us per
+// call in a row of them, of which 3.6 for the launch, this / fft1d_ct2: 100 real
+// transforms of 256 4.0 / 9.1 (5.1 with one transform per workgroup there too),
+// 1,000 complex ones of 512 7.6 / 8.4, 17 x 4 complex ones of 512 6.2 / 7.7.
+constexpr int F1_FEW_MAXN = 1024;
+
+// The rule: where this measured no slower (N = 8 to 1,024, 1 to 100,000 transforms).
+constexpr bool fft1d_is_small(bool real, int lanes, int N, long nt) {
+    const long elements = nt * (real ? N / 2 : N);
+    return lanes == 1 ? N <= (real ? 512 : F1_FEW_MAXN) && nt <= (real ? 2048 : 4096) && elements <= 1L << 19
+                      : N <= 512 && nt <= 512 && elements <= 1L << 16;
+}
+
+template <bool REAL>
+__global__ __launch_bounds__(256) void fft1d_few(double* __restrict__ X, int N, int lanes, int dir,
+                                                 const double2* __restrict__ W) {
+    __shared__ double2 s[F1_FEW_MAXN];
+    const int l = (int)(blockIdx.x % lanes), tid = threadIdx.x;
+    X += (long)(blockIdx.x / lanes) * lanes * N * (REAL ? 1 : 2) + l;
+    for (int n = tid; n < N; n += 256)
+        s[n] = REAL ? make_double2(X[(long)lanes * n], 0.0)
+                    : make_double2(X[2L * lanes * n], X[2L * lanes * n + lanes]);
+    __syncthreads();
+    for (int half = 1; half < N; half <<= 1) {
+        const int stride = N / (2 * half);
+        for (int q = tid; q < N / 2; q += 256) {
+            const int k = q & (half - 1), i0 = ((q - k) << 1) + k, i1 = i0 + half;
+            double2 w = W[k * stride];
+            if (dir < 0) w.y = -w.y;
+            const double2 a = s[i0], c = cmul(s[i1], w);
+            s[i0] = cadd(a, c);
+            s[i1] = csub(a, c);
+        }
+        __syncthreads();
+    }
+    if (REAL) {
+        for (int k = tid; k <= N / 2; k += 256) {
+            X[(long)lanes * k] = s[k].x;
+            if (k > 0 && k < N / 2) X[(long)lanes * (N - k)] = s[k].y;
+        }
+    } else {
+        for (int n = tid; n < N; n += 256) {
+            X[2L * lanes * n] = s[n].x;
+            X[2L * lanes * n + lanes] = s[n].y;
         }
     }
 }
@@ -239,8 +289,13 @@ int fft1d_launch(double* X, int N, int dir, size_t batch) {
     const double2* W;
     CT2_TRY(twiddles(N, &W));
     const int lm = ilog2(N) - (REAL ? 1 : 0);
-    const int T = E >> lm;
     const long nt = (long)batch * L;
+    // fewer to a workgroup where there would not be one for every CU (300 x 4 real
+    // transforms of 128: 8.0 -> 4.7 us), but a group's lanes together unless the
+    // data are small (17 x 4 complex ones of 2,048: 18.2 -> 12.7 us one by one;
+    // 100 x 4: 19 -> 30)
+    int T = E >> lm;
+    while (T > 1 && (nt + T - 1) / T < 256 && (T > L || nt <= 128)) T /= 2;
     fft1d_ct2<REAL, L, E><<<(unsigned)((nt + T - 1) / T), E / 8, 0, ctx().stream>>>(X, lm, nt, T, dir, W);
     CT2_LAUNCH_CHECK();
     return CT2_OK;
@@ -250,6 +305,13 @@ int fft1d_launch(double* X, int N, int dir, size_t batch) {
 // where a group's lanes or a single transform need it.
 template <bool REAL, int L>
 int fft1d_elements(double* X, int N, int dir, size_t batch) {
+    if (fft1d_is_small(REAL, L, N, (long)batch * L)) {
+        const double2* W;
+        CT2_TRY(twiddles(N, &W));
+        fft1d_few<REAL><<<(unsigned)(batch * L), 256, 0, ctx().stream>>>(X, N, L, dir, W);
+        CT2_LAUNCH_CHECK();
+        return CT2_OK;
+    }
     const int need = (REAL ? N / 2 : N) * L;
     if (need <= 2048) return fft1d_launch<REAL, L, 2048>(X, N, dir, batch);
     if (need <= 4096) return fft1d_launch<REAL, L, 4096>(X, N, dir, batch);

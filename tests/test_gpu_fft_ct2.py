@@ -54,6 +54,52 @@ def test_fft_1d_ragged_batches(ct2, orc, N, lanes, batch, dir):
         assert relerr(g, w) < 1e-14
 
 
+@pytest.mark.parametrize("N,lanes,batch", [
+    (2, 1, 2049), (8, 1, 4097), (16, 4, 129), (32, 4, 128), (32, 4, 129), (64, 1, 2048), (64, 1, 4097), (128, 1, 255),
+    (128, 4, 64), (128, 4, 300), (256, 1, 2049), (256, 4, 65), (512, 1, 1025), (512, 4, 33), (1024, 1, 512), (1024, 1, 513),
+    (1024, 4, 32), (1024, 4, 33), (2048, 1, 257), (2048, 4, 32), (2048, 4, 65), (4096, 4, 33)])
+def test_fft_1d_at_the_edges_of_the_small_batches(ct2, orc, N, lanes, batch):
+    """Batches at and past the sizes where a transform has a workgroup of its own, and where a workgroup takes fewer
+    transforms than it could (down to a group's lanes, and to single ones).  Bounds as above."""
+    rng = np.random.default_rng(N * lanes + batch)
+    X = rng.standard_normal(batch * lanes * N)
+    Z = rng.standard_normal(2 * batch * lanes * N)
+    for dir in (1, -1):
+        for got, want in ((ct2.fft_real(X, N, dir, lanes), [orc.fft_real(g, N, dir, lanes) for g in np.split(X, batch)]),
+                          (ct2.fft_complex(Z, N, dir, lanes), [orc.fft_complex(g, N, dir, lanes) for g in np.split(Z, batch)])):
+            d, w = np.split(got, batch) - np.array(want), np.array(want)
+            assert (np.linalg.norm(d, axis=1) < 1e-14 * np.linalg.norm(w, axis=1)).all()
+
+
+def test_small_1d_batches_take_little_more_than_a_launch(ct2):
+    """200 calls in a row: 100 real transforms of 256 points against one of 2 points, which is a launch and little
+    else (3.6 us; 4.0 are expected for the batch, 1.8 times the launch allowed)."""
+    import ctypes as C
+    import time
+
+    from ct2_amd import _lib as L
+    buf = C.c_void_p()
+    L.check(L.load().ct2_dev_alloc(100 * 256 * 8, C.byref(buf)))
+    try:
+        zero = np.zeros(100 * 256)
+        L.check(L.load().ct2_memcpy_h2d(buf, zero.ctypes.data_as(C.c_void_p), zero.nbytes))
+        took = []
+        for N, batch in ((2, 1), (256, 100)):
+            best = np.inf
+            for _ in range(12):
+                ct2.synchronize()
+                t = time.perf_counter()
+                for _ in range(200):
+                    L.check(L.load().ct2_fft_real_1d(buf, N, 1, 1, batch))
+                ct2.synchronize()
+                best = min(best, (time.perf_counter() - t) / 200)
+            took.append(best)
+    finally:
+        L.check(L.load().ct2_dev_free(buf))
+    print(f"one of 2: {took[0] * 1e6:.2f} us, 100 of 256: {took[1] * 1e6:.2f} us", flush=True)
+    assert took[1] < 1.8 * took[0], took
+
+
 def test_fft_real_matches_numpy_after_scramble(ct2, orc):
     """End to end in ct2's order of calls (fft_test.cpp:108-127): scramble on
     the device, then fft_real; the half-complex result equals numpy's rfft."""
