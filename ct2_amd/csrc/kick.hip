@@ -182,15 +182,15 @@ struct PartialSums {
     int nsplit, first, count;
 };
 
-// Sums, for every sink i in [i0, n), the planes of each of the (up to three)
-// partial-sum sets that cover i, in the set order given.  A workgroup takes SW
+// Sums, for every sink i in [i0, n), the planes of the (up to two) partial-sum
+// sets that cover i, in the set order given.  A workgroup takes SW
 // sinks: 4 threads a sink for the components, times 64 / SW that walk the planes
 // in turn; the fewer the sinks (and the more the planes), the smaller SW (one
 // thread a sink took 29 us for 32,768 sinks of 32 planes, and 800 us of the 870
 // for 100 sinks of 977).
 template <int SW>
-__global__ __launch_bounds__(256) void kick_finalize(PartialSums s0, PartialSums s1, PartialSums s2,
-                                                     int n, int i0, double fscale, double pscale, EpiConst e,
+__global__ __launch_bounds__(256) void kick_finalize(PartialSums s0, PartialSums s1, int n,
+                                                     int i0, double fscale, double pscale, EpiConst e,
                                                      float* __restrict__ vx, float* __restrict__ vy,
                                                      float* __restrict__ vz, int8_t* __restrict__ rung,
                                                      float* __restrict__ fx, float* __restrict__ fy,
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256) void kick_finalize(PartialSums s0, PartialSums
     const int t = blockIdx.x * SW + k;
     const int i = i0 + t;
     double a = 0.0;
-    for (const PartialSums& ps : {s0, s1, s2}) {
+    for (const PartialSums& ps : {s0, s1}) {
         const int r = i - ps.first;
         if (t >= ns || !ps.part || r < 0 || r >= ps.count) continue;
         const double* p = ps.part + (long)c * ps.nsplit * ps.count + r;
@@ -960,18 +960,29 @@ int finish_kick(Context& c, const ct2_kick_params* p, const PartialSums* sets, i
     // force in box units: sum(dxu * w3u) * 2^64 * GM; potential: sum(wu) * 2^32 * GM
     const double fscale = (double)c.opts.GM * two32 * two32;
     const double pscale = (double)c.opts.GM * two32;
-    const int planes = std::max({sets[0].nsplit, sets[1].nsplit, sets[2].nsplit});
-    auto launch = [&](auto kernel, int sw) {
-        kernel<<<(n - i0 + sw - 1) / sw, 256, 0, c.stream>>>(sets[0], sets[1], sets[2], n, i0, fscale, pscale, e, c.vx,
-                                                             c.vy, c.vz, c.rung, c.fx, c.fy, c.fz, c.pot, maxrung);
+    // sinks [a, b) of sets x and y
+    auto finalize = [&](int a, int b, const PartialSums& x, const PartialSums& y) {
+        auto launch = [&](auto kernel, int sw) {
+            kernel<<<(b - a + sw - 1) / sw, 256, 0, c.stream>>>(x, y, b, a, fscale, pscale, e, c.vx, c.vy, c.vz, c.rung,
+                                                                c.fx, c.fy, c.fz, c.pot, maxrung);
+        };
+        const int planes = std::max(x.nsplit, y.nsplit);
+        if (planes >= 128)
+            launch(kick_finalize<4>, 4);
+        else if (planes >= 32)
+            launch(kick_finalize<16>, 16);
+        else
+            launch(kick_finalize<64>, 64);
+        CT2_LAUNCH_CHECK();
+        return CT2_OK;
     };
-    if (planes >= 128)
-        launch(kick_finalize<4>, 4);
-    else if (planes >= 32)
-        launch(kick_finalize<16>, 16);
-    else
-        launch(kick_finalize<64>, 64);
-    CT2_LAUNCH_CHECK();
+    // The few sinks before a symmetric core have hundreds of planes, the core one or
+    // two: together, four sinks to a workgroup and an atomic to a wave of four, they
+    // took 370 us longer (131,073 sinks, descending).
+    const PartialSums& rest = sets[2];
+    const int core = i0 + rest.count;
+    if (rest.part) CT2_TRY(finalize(i0, core, rest, PartialSums{nullptr, 0, 0, 0}));
+    CT2_TRY(finalize(core, n, sets[0], sets[1]));
     c.forces_valid = true;
     c.last_path = CT2_PATH_DIRECT;
     return return_max_rung(c, p, maxrung, max_rung);

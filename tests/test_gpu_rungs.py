@@ -96,6 +96,79 @@ def test_kicks_act_on_the_current_range(ct2, orc):
     assert not np.array_equal(p2.vx[first:], p1.vx[first:])
 
 
+@pytest.mark.parametrize("active", [1, 63, 65, 100, 1500, 2400])
+@pytest.mark.parametrize("kernel", [0, 1])
+def test_few_active_sinks_of_a_large_container(ct2, orc, active, kernel):
+    """A rung of a few sinks in 200,003 particles (196 planes of partial sums, 131 and 98 for the last two): force and potential against the FP64 judge, velocities, rungs and
+    the returned maximum as the FP32 epilogue makes them of that force, ascending and descending, everything below the
+    range untouched; the same from ct2_kick_noalloc."""
+    n = 200003
+    rng = np.random.default_rng(active)
+    x, y, z = (rng.integers(0, TWO32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
+    v = [(0.01 * rng.standard_normal(n)).astype(np.float32) for _ in range(3)]
+    rung = np.zeros(n, np.int8)
+    rung[rng.choice(n, active, replace=False)] = 2
+    gm, soft = float(np.float32(1.0 / n)), float(np.float32(1e-3))
+    ct2.set_force_options(soft, gm, kernel)
+    try:
+        ct2.particle_allocate(n)
+        for kick in (ct2.kick, ct2.kick_noalloc):
+            for descending in (False, True):
+                ct2.particles_upload(x, y, z, *v, rung)
+                ct2.particle_sort_by_rung(0)
+                ct2.particle_sort_by_rung(2)
+                first, last = ct2.particle_current_range()
+                assert last - first == active
+                p0 = ct2.particles_download()
+                params = ct2.kick_params(ascending=True, descending=descending, top=True, rung=2, t0=0.01)
+                mr = kick(params, ct2.KICK_STORE)
+                f = ct2.forces_download()
+                W = ct2.kick_sample_fp64(np.arange(first, n))
+                F = np.stack(f[:3])[:, first:]
+                e = np.linalg.norm(F - np.stack(W[:3]), axis=0) / np.linalg.norm(np.stack(W[:3]), axis=0)
+                assert np.median(e) < 2e-6 and e.max() < 1e-4, (np.median(e), e.max())
+                assert np.max(np.abs(f[3][first:] / W[3] - 1)) < 1e-6
+                p1 = ct2.particles_download()
+                for a in ("x", "y", "z", "vx", "vy", "vz", "rung"):
+                    assert np.array_equal(getattr(p1, a)[:first], getattr(p0, a)[:first]), a
+                own = [getattr(p0, a)[first:].copy() for a in ("vx", "vy", "vz", "rung")]
+                op = orc.KickParams(*[getattr(params, k) for k, _ in params._fields_])
+                omr = orc.kick_epilogue(*F, *own, op, soft)
+                for a, w in zip(("vx", "vy", "vz", "rung"), own):
+                    assert np.array_equal(getattr(p1, a)[first:], w), a
+                assert mr == (omr if descending else 0)
+    finally:
+        ct2.set_force_options(soft, gm, 0)
+        ct2.particle_sort_by_rung(0)
+
+
+def test_descending_kick_with_sinks_before_the_symmetric_core(ct2, orc):
+    """65,543 particles in a symmetric core of 65,536 and seven sinks with hundreds of planes, summed apart from the
+    core's: all velocities and rungs as the epilogue makes them of the stored force, and the maximum rung."""
+    n = 65543
+    rng = np.random.default_rng(6)
+    x, y, z = (rng.integers(0, TWO32, n, dtype=np.uint64).astype(np.uint32) for _ in range(3))
+    v = [(0.01 * rng.standard_normal(n)).astype(np.float32) for _ in range(3)]
+    rung = rng.integers(0, 3, n).astype(np.int8)
+    gm, soft = float(np.float32(1.0 / n)), float(np.float32(1e-3))
+    ct2.set_force_options(soft, gm, 0)
+    ct2.particle_allocate(n)
+    ct2.particles_upload(x, y, z, *v, rung)
+    params = ct2.kick_params(ascending=True, descending=True, top=True, rung=1, t0=0.01)
+    mr = ct2.kick(params, ct2.KICK_STORE)
+    f = ct2.forces_download()
+    idx = np.concatenate([np.arange(16), rng.choice(n, 500, replace=False)])
+    W = np.stack(ct2.kick_sample_fp64(idx)[:3])
+    e = np.linalg.norm(np.stack(f[:3])[:, idx] - W, axis=0) / np.linalg.norm(W, axis=0)
+    assert np.median(e) < 2e-6 and e.max() < 1e-4, (np.median(e), e.max())
+    p = ct2.particles_download()
+    own = [a.copy() for a in (*v, rung)]
+    omr = orc.kick_epilogue(*f[:3], *own, orc.KickParams(*[getattr(params, k) for k, _ in params._fields_]), soft)
+    for a, w in zip((p.vx, p.vy, p.vz, p.rung), own):
+        assert np.array_equal(a, w)
+    assert mr == omr
+
+
 @pytest.mark.parametrize("flag_name", ["KICK_SYMMETRIC", "KICK_ORDERED"])
 def test_subset_kick_with_symmetric_core(ct2, orc, flag_name):
     """Active range [first, n) of 3,000 + 2,500 particles: with
