@@ -106,27 +106,30 @@ __global__ __launch_bounds__(KICK_BLOCK) void kick_direct(const uint32_t* __rest
     const uint32_t xi = X[ic], yi = Y[ic], zi = Z[ic];
     const int part = __builtin_amdgcn_readfirstlane(tid / K::SINKS);
 
-    const int j0 = blockIdx.y * jchunk;
-    const int j1 = min(nsrc, j0 + jchunk);
+    // the chunk's sources, counted from its first and without sign: nsrc may be 2^31 - 1
+    const uint32_t j0 = blockIdx.y * (uint32_t)jchunk, len = min((uint32_t)nsrc - j0, (uint32_t)jchunk);
+    X += j0;
+    Y += j0;
+    Z += j0;
     float sx = 0.f, sy = 0.f, sz = 0.f, sp = 0.f;
     float cx = 0.f, cy = 0.f, cz = 0.f, cp = 0.f;
 
     uint4 pre[K::LOADS];
-    auto fetch = [&](int jt) {
+    auto fetch = [&](uint32_t jt) {
 #pragma unroll
         for (int u = 0; u < K::LOADS; ++u) {
-            const int j = jt + u * KICK_BLOCK + tid;
-            if (j < j1) pre[u] = make_uint4(X[j], Y[j], Z[j], 0u);
+            const uint32_t j = jt + u * KICK_BLOCK + tid;
+            if (j < len) pre[u] = make_uint4(X[j], Y[j], Z[j], 0u);
         }
     };
-    fetch(j0);
+    fetch(0);
     int buf = 0;
-    for (int jt = j0; jt < j1; jt += K::TILE) {
+    for (uint32_t jt = 0; jt < len; jt += K::TILE) {
 #pragma unroll
         for (int u = 0; u < K::LOADS; ++u) tile[buf][u * KICK_BLOCK + tid] = pre[u];
         __syncthreads();
         fetch(jt + K::TILE);
-        const int cnt = min(PART, j1 - jt - part * PART);
+        const int cnt = min(PART, (int)min(len - jt, (uint32_t)K::TILE) - part * PART);
         float tx = 0.f, ty = 0.f, tz = 0.f, tp = 0.f;
         if (NAIVE) {
             tx = sx;
@@ -813,7 +816,7 @@ int ordered_pass(Context& c, int i0, int i1, int nsrc, bool naive, bool plummer,
                  size_t* bytes, PartialSums* out, double* fixed = nullptr, size_t fixed_bytes = 0) {
     const int ns = i1 - i0;
     const int sinks = naive ? Kick<true>::SINKS : Kick<false>::SINKS, tile = naive ? Kick<true>::TILE : Kick<false>::TILE;
-    const int nb = (ns + sinks - 1) / sinks;
+    const int nb = (int)(((long)ns + sinks - 1) / sinks);
     // 16,384 workgroups even out the last ones to finish (8 waves of them are in
     // flight at a time): 15,625 sinks x 1,000,003 sources 4.87 ms, with 8,192
     // 4.94, with 4,096 5.39; 32,768 x 32,768 0.355 / 0.358 / 0.381.  Below 5e8
@@ -824,9 +827,8 @@ int ordered_pass(Context& c, int i0, int i1, int nsrc, bool naive, bool plummer,
     int nsplit = std::min(max_split, std::max(1, naive ? (4096 + nb - 1) / nb : want / nb));
     const size_t per_split = sizeof(double) * 4 * (size_t)ns;
     if (fixed) nsplit = (int)std::max<size_t>(1, std::min<size_t>(nsplit, fixed_bytes / per_split));
-    int jchunk = (nsrc + nsplit - 1) / nsplit;
-    jchunk = (jchunk + tile - 1) / tile * tile;
-    const int nsplit_eff = (nsrc + jchunk - 1) / jchunk;
+    const long whole = ((long)nsrc + nsplit - 1) / nsplit, rounded = (whole + tile - 1) / tile * tile;
+    const int jchunk = (int)std::min<long>(rounded, nsrc), nsplit_eff = (int)(((long)nsrc + jchunk - 1) / jchunk);
     double* part = fixed;
     if (fixed) {
         if (per_split * nsplit_eff > fixed_bytes)

@@ -169,6 +169,38 @@ def test_descending_kick_with_sinks_before_the_symmetric_core(ct2, orc):
     assert mr == omr
 
 
+def test_kick_of_one_sink_in_the_largest_container(ct2):
+    """2^31 - 1 particles, the last one active: the source chunks end at 2^31 - 1, past which no index may go.  All
+    sources sit at the sink but the last 1,000, a quarter of the box away along x: their pull on it in closed form
+    (FP32 pair terms: 1e-6)."""
+    import ctypes as C
+
+    from ct2_amd import _lib as L
+    n, far = 2 ** 31 - 1, 1000
+    gm, soft = float(np.float32(1e-3)), float(np.float32(1e-2))
+    ct2.set_force_options(soft, gm, 0)
+    try:
+        ct2.particle_allocate(n)  # all zero
+        ptr = L.ParticlePtrs()
+        L.check(L.load().ct2_particles_device_ptrs(C.byref(ptr)))
+        x, rung = np.full(far, 2 ** 30, np.uint32), np.ones(1, np.int8)
+        L.check(L.load().ct2_memcpy_h2d(ptr.x + 4 * (n - 1 - far), x.ctypes.data_as(C.c_void_p), x.nbytes))
+        L.check(L.load().ct2_memcpy_h2d(ptr.rung + n - 1, rung.ctypes.data_as(C.c_void_p), 1))
+        ct2.particle_sort_by_rung(1)
+        assert ct2.particle_current_range() == (n - 1, n)
+        ct2.kick(ct2.kick_params(ascending=True, top=True, rung=1, t0=1.0))
+        v = np.empty(1, np.float32)
+        got = []
+        for a in (ptr.vx, ptr.vy, ptr.vz):
+            L.check(L.load().ct2_memcpy_d2h(v.ctypes.data_as(C.c_void_p), a + 4 * (n - 1), 4))
+            got.append(float(v[0]))
+    finally:
+        ct2.finalize()  # 140 GB
+        ct2.init(0)
+    want = 0.25 * gm * far * 0.25 / (0.0625 + soft ** 2) ** 1.5  # half of t0 / 2^rung times the force
+    assert abs(got[0] / want - 1) < 1e-6 and got[1] == got[2] == 0.0, (got, want)
+
+
 @pytest.mark.parametrize("flag_name", ["KICK_SYMMETRIC", "KICK_ORDERED"])
 def test_subset_kick_with_symmetric_core(ct2, orc, flag_name):
     """Active range [first, n) of 3,000 + 2,500 particles: with
