@@ -951,8 +951,9 @@ int mm_forces() {
     kc.hinv3u = (float)(1.0 / (hu * hu * hu));
     const double fnear = gm * two32 * two32, pnear = gm * two32;
     const double ffar = gm * (double)nc * nc, pfar = gm * (double)nc;
-    // a wave per work item (max_items bounds the count that the device computes; waves past it exit at once)
-    const unsigned grid = (unsigned)((max_items + MM_WAVES - 1) / MM_WAVES + 7) & ~7u;
+    // a wave per work item (max_items bounds the count that the device computes; waves past it exit at once), as
+    // far as a launch takes them: the waves of 2^31 threads go on with the rest
+    const unsigned grid = (unsigned)std::min<size_t>((max_items + MM_WAVES - 1) / MM_WAVES + 7, (1u << 31) / (64 * MM_WAVES)) & ~7u;
     const bool plummer = c.opts.kernel == CT2_KERNEL_PLUMMER, exact = nc < 16;
 #define CT2_MM_NEAR(KER, EX)                                                                                        \
     mm_near<KER, EX><<<grid, 64 * MM_WAVES, 0, st>>>(s.Ps, s.start, s.items, nitems, (const float*)far, lg, s.ncols, \

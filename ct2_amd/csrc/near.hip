@@ -248,7 +248,7 @@ __global__ __launch_bounds__(64 * NEAR_WAVES) void near_force(
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int b = blockIdx.x * NEAR_WAVES + w;
+    const int b = (int)(blockIdx.y * gridDim.x + blockIdx.x) * NEAR_WAVES + w;
     if (b >= row_chunk[nxy * nxy]) return;  // uniform across the wave; no workgroup barrier follows
     int(*rng)[2] = rngs[w];
     uint4* ring = rings[w];
@@ -615,9 +615,12 @@ int near_forces(double rs) {
     // slices a partner within rcut can be away along z (rcut <= 1 / nc: R <= NEAR_SUB)
     const int R = std::min(NEAR_SUB, (int)std::ceil(rcut * nc * NEAR_SUB));
     // work items: at most one partial one per row beyond n / NEAR_SINKS full ones
-    const unsigned items = (unsigned)((n + NEAR_SINKS - 1) / NEAR_SINKS + nrow);
+    const unsigned items = (unsigned)(((long)n + NEAR_SINKS - 1) / NEAR_SINKS + nrow);
+    // at most 2^31 threads along x: a launch takes less than 2^32, and 2^30 particles need more
+    const unsigned blocks = (items + NEAR_WAVES - 1) / NEAR_WAVES, across = std::min(blocks, (1u << 31) / (64 * NEAR_WAVES));
+    const dim3 grid(across, (blocks + across - 1) / across);
 #define CT2_NEAR(KER)                                                                                          \
-    near_force<KER><<<(items + NEAR_WAVES - 1) / NEAR_WAVES, 64 * NEAR_WAVES, 0, st>>>(                        \
+    near_force<KER><<<grid, 64 * NEAR_WAVES, 0, st>>>(                                                         \
         g_near.P, g_near.start, g_near.subst, g_near.row_chunk, g_near.item, nxy, nc, F, R, q, g_near.table,   \
         fscale, pscale, pconst, c.fx, c.fy, c.fz, c.pot)
     if (c.opts.kernel == CT2_KERNEL_PLUMMER)

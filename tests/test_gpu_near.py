@@ -179,3 +179,56 @@ def test_near_field_argument_checks(ct2):
     with pytest.raises(Ct2Error):
         ct2.pm_near(2.0)  # no Gaussian split
     ct2.pm_near(0.0)
+
+
+def fill_with_copies(ct2, base, copies):
+    """A container of `copies` times the base positions, one after the other; returns its device pointers."""
+    import ctypes as C
+
+    from ct2_amd import _lib as L
+    m = base[0].size
+    ct2.particle_allocate(m * copies)
+    ptr = L.ParticlePtrs()
+    L.check(L.load().ct2_particles_device_ptrs(C.byref(ptr)))
+    for dst, src in zip((ptr.x, ptr.y, ptr.z), base):
+        for k in range(copies):
+            L.check(L.load().ct2_memcpy_h2d(dst + 4 * m * k, src.ctypes.data_as(C.c_void_p), 4 * m))
+    return ptr
+
+
+def velocities(ptr, first, count):
+    import ctypes as C
+
+    from ct2_amd import _lib as L
+    v = np.empty((3, count), np.float32)
+    for a, p in zip(v, (ptr.vx, ptr.vy, ptr.vz)):
+        L.check(L.load().ct2_memcpy_d2h(a.ctypes.data_as(C.c_void_p), p + 4 * first, 4 * count))
+    return v.astype(np.float64)
+
+
+def test_near_field_of_more_work_items_than_a_launch_takes(ct2):
+    """2^30 + 2^20 particles, 1,025 copies of 2^20 (a wave per 16 sinks: more than 2^32 threads): every copy's
+    velocities after a half-kick equal the first's to the FP32 sums' rounding (about 10^5 terms; 1e-5 of their size),
+    and they are those of the same mass in one copy."""
+    m, copies = 2 ** 20, 1025
+    rng = np.random.default_rng(30)
+    base = [rng.integers(0, TWO32, m, dtype=np.uint64).astype(np.uint32) for _ in range(3)]
+    kick = ct2.kick_params(ascending=True, top=True, rung=0, t0=2.0)
+    soft = f32(1e-3)
+    try:
+        ct2.pm_init(128, 1.0)
+        ct2.pm_near(0.5)
+        got = []
+        for k in (1, copies):
+            ct2.set_force_options(soft, f32(1.0 / (m * k)), ct2.KERNEL_PLUMMER)
+            ptr = fill_with_copies(ct2, base, k)
+            ct2.kick_pm(kick)
+            got.append([velocities(ptr, (j * (k - 1) // 8) * m, m) for j in range(9 if k > 1 else 1)])
+        scale = np.sqrt((got[0][0] ** 2).mean())
+        for v in got[1]:
+            assert np.abs(v - got[1][0]).max() < 1e-4 * scale
+            assert np.sqrt(((v - got[0][0]) ** 2).mean()) < 1e-5 * scale
+    finally:
+        ct2.finalize()  # 90 GB
+        ct2.init(0)
+        ct2.pm_init(32, 1.0)
