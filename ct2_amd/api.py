@@ -250,6 +250,14 @@ def near_kernel_table(rs_u: float, rcut_u: float, nt: int = 64):
     return k4, p4
 
 
+def near_potential_table(rs_u: float, rcut_u: float):
+    """The cubic pieces of the filtered potential that the near-field kernel reads
+    (host function): float32 of shape (513, 4)."""
+    p4 = np.zeros((513, 4), np.float32)
+    L.check(L.load().ct2_near_potential_table(rs_u, rcut_u, _p(p4)))
+    return p4
+
+
 def pm_forces():
     """PM force and potential of every particle: (fx, fy, fz, pot)."""
     L.check(L.load().ct2_pm_forces())

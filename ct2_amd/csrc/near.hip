@@ -66,9 +66,12 @@ constexpr int NEAR_MAX_ROWS = 25;  // (2F + 1)^2
 #endif
 constexpr int NEAR_SUB = NEAR_SUB_N;
 // The filtered Newtonian kernel is evaluated from NEAR_NT + 1 cubic pieces of
-// its potential in r^2 over [0, rcut^2]: force and potential within 1e-8
-// (relative to their values at 0) of the closed forms, below FP32 rounding
-// (built on the host in FP64 by near_potential_table).  Fewer, quartic pieces
+// its potential in r^2 over [0, rcut^2] (built on the host in FP64 by
+// near_potential_table).  Force error of the pieces, relative to the force's value,
+// before and after their coefficients are rounded to FP32: 8e-10 and 6e-8 to 4 rs,
+// 6e-9 and 6e-8 to 5.5 rs, 5e-8 and 1e-7 to 8 rs; beyond, where the pieces are long
+// against rs, 6e-7 to 12 rs, 1.3e-5 to 20 rs and 1e-2 to 64 rs, the largest cutoff;
+// the potential's is smaller.  Fewer, quartic pieces
 // (64, 20 bytes to gather) or 64 pieces each of force and potential (32 bytes)
 // cost more LDS and VALU per pair.
 constexpr int NEAR_NT = 512;
@@ -647,6 +650,15 @@ void release_near() {
 }
 
 }  // namespace ct2
+
+static_assert(CT2_NEAR_PIECES == ct2::NEAR_NT + 1, "the pieces of near_force");
+
+extern "C" int ct2_near_potential_table(double rs_u, double rcut_u, float* p4) {
+    if (!(rs_u > 0.0) || !(rcut_u > 0.0) || !p4)
+        return ct2::set_error(CT2_ERR_INVALID, "ct2_near_potential_table: bad argument");
+    ct2::near_potential_table(rs_u, rcut_u, p4);
+    return CT2_OK;
+}
 
 extern "C" int ct2_near_kernel_table(double rs_u, double rcut_u, int nt, float* k4, float* p4) {
     if (!(rs_u > 0.0) || !(rcut_u > 0.0) || nt < 1 || !k4 || !p4)

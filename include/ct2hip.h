@@ -186,11 +186,17 @@ int ct2_pm_near_cells(void);
  *   p_l = erf(u) / (u (2 rs)),   u = r / (2 rs),
  * piece i evaluated at f = r^2 nt / rcut_u^2 - i as c0 + f (c1 + f (c2 + f c3)),
  * coefficients (c0..c3) of piece i at k4[4i..4i+3] and p4[4i..4i+3].  The
- * pair kernel subtracts k_l and p_l from the softened Newtonian kernel (the GPU
- * reads its own pieces of p_l, whose derivative is k_l).  Host only, no device
+ * pair kernel subtracts k_l and p_l from the softened Newtonian kernel; the GPU
+ * reads other pieces, ct2_near_potential_table's.  Host only, no device
  * state.  No counterpart in the reference (its near field is the
  * plain softened kernel with the mesh's far field left out). */
 int ct2_near_kernel_table(double rs_u, double rcut_u, int nt, float* k4, float* p4);
+/* The pieces that the GPU reads: CT2_NEAR_PIECES cubic pieces of p_l alone, in
+ * t = r^2 (CT2_NEAR_PIECES - 1) / rcut_u^2.  Piece i = t rounded to nearest is
+ * evaluated at f = t - i in [-1/2, 1/2] (0 <= f for i = 0), coefficients (c0..c3)
+ * at p4[4i..4i+3]; k_l = -2 (CT2_NEAR_PIECES - 1) / rcut_u^2 dp_l/df.  Host only. */
+#define CT2_NEAR_PIECES 513
+int ct2_near_potential_table(double rs_u, double rcut_u, float* p4);
 /* Mass assignment of the PM force: 1 = cloud in cell (default), 2 =
  * triangular-shaped cloud (27 nodes, quadratic spline; the Green's table
  * deconvolves sinc^6 instead of sinc^4).  TSC lowers the mesh's
