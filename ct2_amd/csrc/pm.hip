@@ -4,10 +4,10 @@
 // and particle_compute_expansions, particle.cpp:180-271, evaluated by L2P at
 // kick.cpp:29) with cloud-in-cell mass assignment, keeping its pipeline:
 //   deposit       fixed-point CIC (default) or TSC weights, uint64 atomics:
-//                 deterministic, bit-identical to the CPU oracle.  Grids of 32
-//                 nodes a side or more: particles binned by 16^3-node tile
+//                 deterministic, bit-identical to the CPU oracle.  Where
+//                 tiles_pay says so: particles binned by 16^3-node tile
 //                 (bin_*), each tile summed in LDS and stored (dep_tile);
-//                 smaller grids: one global atomic per particle and stencil
+//                 elsewhere one global atomic per particle and stencil
 //                 node (mesh_deposit)
 //   rfft_zy_density  z and y passes of the density's FP32 transform to its
 //                 half spectrum (fft.hip; the first reads the uint64 grid
@@ -388,11 +388,13 @@ __global__ __launch_bounds__(TILE_THREADS) void dep_tile(const uint32_t* __restr
 // cell in 205 us; with the half-spectrum z and y passes before it the
 // transforms of one force on 256^3 went from 453 to 327 us, on 64^3 from 36 to
 // 22 us (ten launches to four).
-// On 64^3 grids the columns of the cubes' passes make 66 workgroups; 8 of them
-// (64-byte segments) make 264: 9.1 -> 7.8 us.
+// 16 columns to a workgroup, a 128-byte line's, where there are so many: fewer do not
+// pay for more workgroups nor more columns for fuller ones (us with 32 / 16 / 8 / 4
+// columns: 64^3 7.7 / 7.0 / 7.4 / 7.5; 32^3 - / 5.1 / 5.7 / 5.8; 16^3, 8 at most, 3.7 /
+// 3.9; 128^3 - / 15.3 / 14.7 / 16.3; runs of one differ by 4 %).
 template <int N>
 constexpr int xpass_cols() {
-    return N == 64 ? 8 : Cfg<float, N, N / 2>::COLS;
+    return Cfg<float, N, N / 2>::COLS < 16 ? Cfg<float, N, N / 2>::COLS : 16;
 }
 
 template <int N>
