@@ -63,6 +63,34 @@ def test_fft3d_in_groups_of_planes(ct2, f64, d):
     assert rel_l2(got, cube[1]) < (1e-14 if f64 else 1e-6)
 
 
+def test_fft3d_fp32_of_1024(ct2):
+    """1024^3, the largest: 24 planes to a group, the last one of 16.  A product of three random lines forward,
+    compared with the product of their FP64 transforms on planes of every group, then back to itself."""
+    import ctypes as C
+
+    from ct2_amd import _lib as L
+    n, rng = 1024, np.random.default_rng(10)
+    a = (rng.standard_normal((3, n)) + 1j * rng.standard_normal((3, n))).astype(np.complex64)
+    t = np.fft.fft(a.astype(np.complex128))
+    buf = ct2.DeviceBuffer(n ** 3 * 8)
+    plane, slab = a[1][:, None] * a[2], np.empty((8, n, n), np.complex64)
+    for i in range(0, n, 8):
+        for j in range(8):
+            np.multiply(plane, a[0][i + j], out=slab[j])
+        L.check(L.load().ct2_memcpy_h2d(buf.ptr + i * n * n * 8, slab.ctypes.data_as(C.c_void_p), slab.nbytes))
+    some = sorted(set(range(0, n, 23)) | {1, 512, 1007, 1008, 1022, 1023})
+    for d, lines in ((1, t), (-1, a.astype(np.complex128) * [[n], [n], [n]])):
+        ct2.fft3d_device(buf, n, d)
+        plane, err, ref = lines[1][:, None] * lines[2], 0.0, 0.0
+        for i in some:
+            L.check(L.load().ct2_memcpy_d2h(slab[0].ctypes.data_as(C.c_void_p), buf.ptr + i * n * n * 8, n * n * 8))
+            want = lines[0][i] * plane
+            err += np.linalg.norm(slab[0] - want) ** 2
+            ref += np.linalg.norm(want) ** 2
+        assert (err / ref) ** 0.5 < 1e-6, (d, (err / ref) ** 0.5)
+    buf.close()
+
+
 def test_fft3d_512_round_trip_and_delta(ct2):
     """512^3 (the PM grid of the clustered and stepping configurations):
     delta -> constant, and forward/inverse round trip."""

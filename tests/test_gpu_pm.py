@@ -81,6 +81,40 @@ def test_pm_fields_of_the_density_at_every_grid_size(ct2, ng):
         assert np.linalg.norm(ct2.pm_grid_download(which).ravel() - want) < 2e-6 * np.linalg.norm(want)
 
 
+def test_pm_force_on_1024(ct2):
+    """The largest grid (its own shape of the x pass, real passes of 512 points, planes in ragged groups): particles on
+    nodes, so that deposit and interpolation are exact, against the FP64 sum of the Green's function over all wave
+    vectors, axis by axis.  FP32 transforms stay within 2e-6 of their grid's rms (2-norm); five times that of the
+    fields' largest value at the particles, which are its peaks, is allowed at each."""
+    ng, rs = 1024, 1.0
+    h = ng // 2
+    node = np.array([[3, 5, 7], [4, 5, 7], [1020, 1019, 1022], [500, 511, 512], [3, 517, 1000], [1008, 23, 24]])
+    load(ct2, *(np.ascontiguousarray(node[:, a].astype(np.uint32) << 22) for a in range(3)))
+    gm = f32(1.0 / len(node))
+    ct2.set_force_options(1e-3, gm, 0)
+    try:
+        ct2.pm_init(ng, rs)
+        got = np.stack(ct2.pm_forces()).astype(np.float64)
+    finally:
+        ct2.pm_init(8, 1.25)  # the large grids are released
+    m = np.arange(h + 1)
+    k = 2 * np.pi * m
+    green = -4 * np.pi * gm / np.maximum(k[:, None, None] ** 2 + k[:, None] ** 2 + k ** 2, 1.0)
+    green[0, 0, 0] = 0.0
+    axis = np.exp(-(k * rs / ng) ** 2) / np.sinc(m / ng) ** 4 * np.where((m == 0) | (m == h), 1.0, 2.0)
+    d = ((node[:, None] - node[None]) % ng).reshape(-1, 3)  # particle minus source
+    even = [axis[:, None] * np.cos(2 * np.pi * np.outer(m, v) / ng) for v in d.T]
+    odd = [np.where((m == 0) | (m == h), 0.0, k * axis)[:, None] * np.sin(2 * np.pi * np.outer(m, v) / ng) for v in d.T]
+    want = []
+    for gradient in (0, 1, 2, None):
+        f = [odd[a] if a == gradient else even[a] for a in range(3)]
+        yz = (green.reshape(-1, h + 1) @ f[2]).reshape(h + 1, h + 1, -1)
+        total = np.einsum("xd,yd,xyd->d", f[0], f[1], yz, optimize=True).reshape(len(node), -1).sum(1)
+        want.append(total if gradient is not None else -total)
+    want = np.stack(want)
+    assert (np.abs(got - want).max(1) < 1e-5 * np.abs(want).max(1)).all(), (got, want)
+
+
 def test_pm_matches_periodic_judge_on_a_single_mode(ct2):
     """Linear single-mode lattice: PM long-range force 4 pi psi exp(-k^2 rs^2),
     the periodic FP64 judge the full 4 pi psi."""
