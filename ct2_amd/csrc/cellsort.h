@@ -15,6 +15,7 @@
 #pragma once
 
 #include "internal.h"
+#include "wave.h"
 
 namespace ct2 {
 namespace cellsort {
@@ -31,12 +32,6 @@ struct Records {
     const uint4* r;
     __device__ __forceinline__ uint4 operator()(long e) const { return r[e]; }
 };
-
-__device__ __forceinline__ void wave_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // cnt[tile][digit]
 template <int ITEMS, typename SRC, typename KEY>
@@ -127,9 +122,9 @@ __global__ __launch_bounds__(THREADS) void place(SRC src, KEY key, int n, int sh
         const uint32_t rank =
             __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
         const uint32_t before = hw[d];
-        wave_order();
+        wave_sync();
         if (have && rank == 0) hw[d] = (uint16_t)(before + (uint32_t)__popcll(same));
-        wave_order();
+        wave_sync();
         at[u] = d << 16 | (before + rank);
     }
     __syncthreads();

@@ -22,6 +22,7 @@
 
 #include "epilogue.h"
 #include "internal.h"
+#include "wave.h"
 
 namespace ct2 {
 namespace {
@@ -34,15 +35,6 @@ struct KickConst {
     float hinvu;   //             1/(h 2^32)
     float hinv3u;  //             1/(h 2^32)^3
 };
-
-__device__ __forceinline__ void two_sum(float& s, float& c, float v) {
-#pragma clang fp contract(off)
-    const float t = s + v;
-    const float bp = t - s;
-    const float e = (s - (t - bp)) + (v - bp);
-    s = t;
-    c += e;
-}
 
 template <int KERNEL>
 __device__ __forceinline__ void interact(const uint4 src, uint32_t xi, uint32_t yi, uint32_t zi,
@@ -79,7 +71,7 @@ __device__ __forceinline__ void interact(const uint4 src, uint32_t xi, uint32_t 
 // A workgroup takes 64 sinks; its four waves share every tile of 512 sources, a
 // quarter each, and their sums are added in FP64 in LDS: a quarter of the
 // partial sums that one sink per thread leaves for the same number of waves in
-// flight, and no more than 63 idle lanes in the last workgroup.  (NAIVE: 256
+// flight.  A last workgroup of one sink leaves 63 lanes of each of its waves idle.  (NAIVE: 256
 // sinks and one sum over the chunk each, as its plain FP32 accumulation means.)
 // Bound by VALU issue, 16 instructions a pair.
 template <bool NAIVE>
@@ -820,8 +812,9 @@ int ordered_pass(Context& c, int i0, int i1, int nsrc, bool naive, bool plummer,
     // 16,384 workgroups even out the last ones to finish (8 waves of them are in
     // flight at a time): 15,625 sinks x 1,000,003 sources 4.87 ms, with 8,192
     // 4.94, with 4,096 5.39; 32,768 x 32,768 0.355 / 0.358 / 0.381.  Below 5e8
-    // pairs there is little to even out, and 4,096 workgroups leave at most 8 MiB
-    // of partial sums, what ct2_kick_noalloc has room for.
+    // pairs there is little to even out, and 4,096 workgroups of 64 sinks leave at
+    // most 8 MiB of partial sums, what ct2_kick_noalloc has room for (the naive
+    // kernel's, of 256, four times that: there the split is cut to fit).
     const int want = (double)ns * nsrc > 5e8 ? 16384 : 4096;
     const int max_split = std::max(1, nsrc / (naive ? 4 * tile : tile));
     int nsplit = std::min(max_split, std::max(1, naive ? (4096 + nb - 1) / nb : want / nb));

@@ -19,6 +19,7 @@
 
 #include "epilogue.h"
 #include "internal.h"
+#include "wave.h"
 
 namespace ct2 {
 namespace {
@@ -124,12 +125,6 @@ __device__ __forceinline__ GemmBlock gemm_block(int id, int nrb, int ncb, int S)
         g.z = t / ncb;
     }
     return g;
-}
-
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // A wave's LDS for the GELU / DGELU epilogue of one 32 x 32 tile.

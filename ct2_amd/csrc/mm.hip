@@ -41,6 +41,7 @@
 #include "epilogue.h"
 #include "fft_stages.h"
 #include "internal.h"
+#include "wave.h"
 
 namespace ct2 {
 namespace {
@@ -402,9 +403,7 @@ __global__ __launch_bounds__(256) void mm_p2m(const uint4* __restrict__ P, const
                     pv *= mb;
                 }
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_sync();
             const int cnt = min(MM_P2M_PART, s1 - base);
             for (int j0 = 0; j0 < cnt; j0 += 4) {
 #pragma unroll
@@ -418,9 +417,7 @@ __global__ __launch_bounds__(256) void mm_p2m(const uint4* __restrict__ P, const
                     for (int u = 0; u < 4; ++u) acc[r] += (double)m[u];
                 }
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_sync();
         }
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
@@ -699,12 +696,6 @@ __device__ __forceinline__ void near_pair(float ddx, float ddy, float ddz, float
     ty = fmaf(ddy, k, ty);
     tz = fmaf(ddz, k, tz);
     tp += p;
-}
-
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ __forceinline__ float lane_value(float v, int lane) {

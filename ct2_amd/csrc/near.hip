@@ -40,6 +40,7 @@
 
 #include "cellsort.h"
 #include "internal.h"
+#include "wave.h"
 
 namespace ct2 {
 namespace {
@@ -164,15 +165,6 @@ __global__ __launch_bounds__(SCAN_THREADS) void near_scan(const int* __restrict_
     if (t == 0) out[len] = carry;
 }
 
-__device__ __forceinline__ void two_sum(float& s, float& c, float v) {
-#pragma clang fp contract(off)
-    const float t = s + v;
-    const float bp = t - s;
-    const float e = (s - (t - bp)) + (v - bp);
-    s = t;
-    c += e;
-}
-
 // Softened kernel minus the filtered Newtonian kernel for one pair, in
 // 2^-32 units: returns the force factor k (F += dx k) and potential p.  The
 // filtered potential p_l comes from cubic pieces in LDS and the filtered force
@@ -215,12 +207,6 @@ __global__ __launch_bounds__(256) void near_items(const int* __restrict__ row_ch
     if (r >= nrow) return;
     const int k0 = row_chunk[r], k1 = row_chunk[r + 1];
     for (int k = k0 + lane; k < k1; k += 64) item[k] = make_int2(r, k - k0);
-}
-
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // One wave per work item of S sinks, NEAR_WAVES waves per workgroup (they share

@@ -1,4 +1,4 @@
-// wave.h -- wave64 helpers shared by the binning kernels.
+// wave.h -- device helpers shared by the kernels.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -6,6 +6,24 @@
 #include <cstdint>
 
 namespace ct2 {
+
+// Orders the wave's LDS accesses before and after it: what the lanes wrote is
+// read by the others.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Adds v to the sum s, the rounding error to c.
+__device__ __forceinline__ void two_sum(float& s, float& c, float v) {
+#pragma clang fp contract(off)
+    const float t = s + v;
+    const float bp = t - s;
+    const float e = (s - (t - bp)) + (v - bp);
+    s = t;
+    c += e;
+}
 
 // Counting-sort increment with one atomic per run of equal keys: every lane
 // whose key is >= 0 adds 1 to counter[key] and receives the counter's value
