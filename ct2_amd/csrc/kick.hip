@@ -71,8 +71,9 @@ __device__ __forceinline__ void interact(const uint4 src, uint32_t xi, uint32_t 
 // A workgroup takes 64 sinks; its four waves share every tile of 512 sources, a
 // quarter each, and their sums are added in FP64 in LDS: a quarter of the
 // partial sums that one sink per thread leaves for the same number of waves in
-// flight.  A last workgroup of one sink leaves 63 lanes of each of its waves idle.  (NAIVE: 256
-// sinks and one sum over the chunk each, as its plain FP32 accumulation means.)
+// flight.  A last workgroup of one sink leaves 63 lanes of each of its waves
+// idle.  (NAIVE: 256 sinks and one sum over the chunk each, as its plain FP32
+// accumulation means.)
 // Bound by VALU issue, 16 instructions a pair.
 template <bool NAIVE>
 struct Kick {
