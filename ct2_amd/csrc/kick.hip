@@ -812,7 +812,8 @@ int ordered_pass(Context& c, int i0, int i1, int nsrc, bool naive, bool plummer,
     const int nb = (int)(((long)ns + sinks - 1) / sinks);
     // 16,384 workgroups even out the last ones to finish (8 waves of them are in
     // flight at a time): 15,625 sinks x 1,000,003 sources 4.87 ms, with 8,192
-    // 4.94, with 4,096 5.39; 32,768 x 32,768 0.355 / 0.358 / 0.381.  Below 5e8
+    // 4.94, with 4,096 5.39; 32,768 x 32,768 0.355 / 0.358 / 0.381 (one run; boxes and
+    // clocks differ by 5 %, the kernel traced in 60 passes takes 5.15 and 0.362).  Below 5e8
     // pairs there is little to even out, and 4,096 workgroups of 64 sinks leave at
     // most 8 MiB of partial sums, what ct2_kick_noalloc has room for (the naive
     // kernel's, of 256, four times that: there the split is cut to fit).

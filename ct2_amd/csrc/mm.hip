@@ -285,7 +285,7 @@ struct PutCell {
 // separations of a run are FP32 offsets from the centre of its first cell.  The
 // runs are part of the result, not of the split: the rounding of a close pair's
 // separation grows with its distance from that centre, so other centres move the
-// forces of a set's closest pairs by up to 1e-5 of the whole (2-norm).  An item is
+// forces of a set's closest pairs, and so all of them by up to 2.4e-5 (2-norm).  An item is
 // at most MM_SINKS sinks of one cell and one run, as even as they go:
 // (cell | cells from the run's first to it << 24 | sinks << 27, first sink).
 constexpr int MM_SINKS = 10, MM_RUN = 64;
@@ -588,7 +588,10 @@ __global__ __launch_bounds__(64 * WAVES) void mm_mg2l(const float2* __restrict__
 // ------------------------------------------------------------ L2P
 
 // Where the local expansion's components lie: pairs of z exponents (d, d + 1), d
-// even, column by column, then the highest exponents left over two by two.
+// even, column by column, then the highest exponents left over two by two.  Two
+// components share a complex FP32 transform and its noise, of the size of the larger
+// one: the smallest degree's falls on the z force (with components paired by their
+// number it fell on x), and the whole force's error does not depend on it.
 template <int P>
 struct LocalGrids {
     int pair[P + 1][P + 1] = {};    // grid of a column's first pair
@@ -769,7 +772,7 @@ __device__ __forceinline__ void near_sinks(uint4 own, uint32_t rx, uint32_t ry, 
 // runs in LDS (idle for a fifth of the time, with 135 instructions per column and
 // two per pair on top, but eight waves per SIMD) took 1,109 us for 2^21 particles on
 // 64^3 cells, and two small kernels 39 us to cut the rows into its items; this takes
-// 1,063 and 7.  12 sinks took 1,081 at five waves and 1,237 at four, 9 the same at
+// 1,063 (median of 60 traced passes 1,020) and 18.  12 sinks took 1,081 at five waves and 1,237 at four, 9 the same at
 // six; groups of 2 to 6 sinks interleaved by hand 1,177 to 1,320.  EXACT (8^3 cells,
 // whose offsets are too coarse): separations from the fixed-point positions.
 constexpr int MM_STEPS = 64;  // steps whose run heads are in LDS at a time

@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256) void near_items(const int* __restrict__ row_ch
 // (256^3 grid, rs 1.5, to 5.5 rs), 18.4, 16.7, 18.6 and 21.8 at 2^24 (512^3, rs
 // 2).  With 64 sinks per wave and 64-bit box tests, and 32 bytes gathered per
 // pair for the filtered kernel (LDS busy 72 % of the time), this kernel took
-// 1.57 ms of the first, now 1.15.  Sources as exact pairs of floats, to subtract
+// 1.57 ms of the first, now 1.15 (median of 60 traced passes 1.10).  Sources as exact pairs of floats, to subtract
 // instead of converting each separation from integers: 1.52.
 template <int KERNEL>
 __global__ __launch_bounds__(64 * NEAR_WAVES) void near_force(
