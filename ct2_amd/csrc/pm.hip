@@ -132,10 +132,11 @@ constexpr int TS = 1 << TILE_B;
 constexpr int TROW = TS + 1;                 // padded LDS row
 constexpr int TL = TS + 2;                   // side of the grown tile
 constexpr int TL_NODES = TL * TL * TL;
-// The tiles' kernels: two workgroups per CU.  A set in a corner of the box is a few
-// tiles' work: 2^21 particles in 1/1000 of it on 128^3 (TSC) take 9.8 ms a force,
-// with 512 threads to a tile 16.7; sets that fill the box are the same with either.
-constexpr int TILE_THREADS = 1024;
+// Threads to a tile: 1,024 on grids of at most two tiles per CU, 512 (four workgroups
+// per CU) on larger ones.  us of deposit and interpolation of 2^21 particles on 256^3
+// (TSC) 169 with 512, 176 with 1,024; a force on 128^3 188 / 196 with 1,024 / 512, and
+// where the set lies in a corner, a few tiles' work, 9.8 / 16.7 ms (in 1/1000 of the box).
+constexpr int tile_threads(int tiles) { return tiles <= 2 * 256 ? 1024 : 512; }
 constexpr int TILE_MIN_G = TILE_B + 1;  // grids of at least 2^5 nodes a side
 constexpr int BIN_THREADS = 1024;
 constexpr int BIN_WGS = 128;            // binning workgroups at most
@@ -325,8 +326,8 @@ __global__ __launch_bounds__(BIN_THREADS) void tile_scan(int* __restrict__ in, i
     if (threadIdx.x == 0) out[len] = sum;
 }
 
-template <int ORDER>
-__global__ __launch_bounds__(TILE_THREADS) void dep_tile(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
+template <int ORDER, int THREADS>
+__global__ __launch_bounds__(THREADS) void dep_tile(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
                                                         const uint32_t* __restrict__ Z, const int* __restrict__ order,
                                                         const int* __restrict__ tstart, int g, bool add,
                                                         unsigned long long* __restrict__ W) {
@@ -337,9 +338,9 @@ __global__ __launch_bounds__(TILE_THREADS) void dep_tile(const uint32_t* __restr
     const uint32_t mask = (1u << g) - 1u;
     uint32_t ox, oy, oz;
     tile_origin(tile, g, ox, oy, oz);
-    for (int i = tid; i < TS * TS * TROW; i += TILE_THREADS) acc[i] = 0ull;
+    for (int i = tid; i < TS * TS * TROW; i += THREADS) acc[i] = 0ull;
     __syncthreads();
-    for (int k = b + tid; k < e; k += TILE_THREADS) {
+    for (int k = b + tid; k < e; k += THREADS) {
         const int o = order[k], p = o < 0 ? ~o : o;
         const uint32_t x = X[p], y = Y[p], z = Z[p];
         uint32_t lo;
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(TILE_THREADS) void dep_tile(const uint32_t* __restr
             }
     }
     __syncthreads();
-    for (int i = tid; i < TS * TS * TS; i += TILE_THREADS) {
+    for (int i = tid; i < TS * TS * TS; i += THREADS) {
         const int lz = i % TS, ly = i / TS % TS, lx = i / (TS * TS);
         unsigned long long* const w = W + (((((size_t)(ox + lx) << g) + (oy + ly)) << g) + (oz + lz));
         const unsigned long long v = acc[(lx * TS + ly) * TROW + lz];
@@ -560,8 +561,8 @@ __global__ __launch_bounds__(PM_BLOCK) void mesh_interp(const uint32_t* __restri
 // grown tiles (rows of 144 bytes, 2.1 lines each): 130 us for 2^21 particles on
 // 256^3 with neighbouring tiles on one XCD, 165 with the tiles dealt to the XCDs
 // in turn.
-template <int ORDER>
-__global__ __launch_bounds__(TILE_THREADS) void interp_tile(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
+template <int ORDER, int THREADS>
+__global__ __launch_bounds__(THREADS) void interp_tile(const uint32_t* __restrict__ X, const uint32_t* __restrict__ Y,
                                                            const uint32_t* __restrict__ Z, const int* __restrict__ order,
                                                            const int* __restrict__ tstart, int g,
                                                            const float2* __restrict__ A, float* __restrict__ fx,
@@ -579,22 +580,22 @@ __global__ __launch_bounds__(TILE_THREADS) void interp_tile(const uint32_t* __re
     A += (size_t)blockIdx.y << (3 * g);
     float* out0 = blockIdx.y ? fz : fx;
     float* out1 = blockIdx.y ? pot : fy;
-    constexpr int LOADS = (TL_NODES + TILE_THREADS - 1) / TILE_THREADS;
+    constexpr int LOADS = (TL_NODES + THREADS - 1) / THREADS;
     float2 v[LOADS];  // all in flight before the first is stored
 #pragma unroll
     for (int u = 0; u < LOADS; ++u) {
-        const int i = min(tid + u * TILE_THREADS, TL_NODES - 1);
+        const int i = min(tid + u * THREADS, TL_NODES - 1);
         const int lx = i / (TL * TL), ly = i / TL % TL, lz = i % TL;
         const size_t gx = (ox + lx - 1u) & mask, gy = (oy + ly - 1u) & mask, gz = (oz + lz - 1u) & mask;
         v[u] = A[(((gx << g) + gy) << g) + gz];
     }
 #pragma unroll
     for (int u = 0; u < LOADS; ++u)
-        if (tid + u * TILE_THREADS < TL_NODES) nd[tid + u * TILE_THREADS] = v[u];
+        if (tid + u * THREADS < TL_NODES) nd[tid + u * THREADS] = v[u];
     __syncthreads();
     constexpr uint32_t SHIFT = ORDER == 1 ? 1u : 0u;
     const float q = 0x1p-21f;
-    for (int k = b + tid; k < e; k += TILE_THREADS) {
+    for (int k = b + tid; k < e; k += THREADS) {
         const int p = order[k];
         if (p < 0) continue;  // at home in a neighbour
         const uint32_t x = X[p], y = Y[p], z = Z[p];
@@ -728,7 +729,10 @@ int deposit(const Context& c) {
     for (int k = 0; k < count; ++k) {
         const Slab p = slab(c, k);
         CT2_TRY(bin_particles<ORDER>(p, c.stream));
-        dep_tile<ORDER><<<nt, TILE_THREADS, 0, c.stream>>>(p.x, p.y, p.z, g_pm.order, g_pm.tstart, g, k > 0, g_pm.W);
+        auto dep = [&](auto kernel) {
+            kernel<<<nt, tile_threads(nt), 0, c.stream>>>(p.x, p.y, p.z, g_pm.order, g_pm.tstart, g, k > 0, g_pm.W);
+        };
+        tile_threads(nt) == 1024 ? dep(dep_tile<ORDER, 1024>) : dep(dep_tile<ORDER, 512>);
         CT2_LAUNCH_CHECK();
     }
     return CT2_OK;
@@ -737,13 +741,16 @@ int deposit(const Context& c) {
 // Force and potential by tiles; the lists of the last slab are in place.
 template <int ORDER>
 int interp_by_tiles(const Context& c) {
-    const int count = slab_count(c);
+    const int count = slab_count(c), nt = g_pm.ntile;
     for (int k = count - 1; k >= 0; --k) {
         const Slab p = slab(c, k);
         if (k < count - 1) CT2_TRY(bin_particles<ORDER>(p, c.stream));
-        interp_tile<ORDER><<<dim3(g_pm.ntile, 2), TILE_THREADS, 0, c.stream>>>(
-            p.x, p.y, p.z, g_pm.order, g_pm.tstart, g_pm.g, g_pm.A, c.fx + p.first, c.fy + p.first, c.fz + p.first,
-            c.pot + p.first);
+        auto interp = [&](auto kernel) {
+            kernel<<<dim3(nt, 2), tile_threads(nt), 0, c.stream>>>(p.x, p.y, p.z, g_pm.order, g_pm.tstart, g_pm.g, g_pm.A,
+                                                                   c.fx + p.first, c.fy + p.first, c.fz + p.first,
+                                                                   c.pot + p.first);
+        };
+        tile_threads(nt) == 1024 ? interp(interp_tile<ORDER, 1024>) : interp(interp_tile<ORDER, 512>);
         CT2_LAUNCH_CHECK();
     }
     return CT2_OK;
